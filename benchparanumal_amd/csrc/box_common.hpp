@@ -1,0 +1,13 @@
+// Per-degree launchers of the structured-box kernels (box_*.hip, compiled
+// once per Nq); box_dispatch.cpp maps the run-time degree onto them.
+#pragma once
+#include "box.hpp"
+#include "bpx_internal.hpp"
+
+namespace bpx {
+
+template <typename T, int NQ>
+int launch_box_gather_nq(hipStream_t s, const BoxGrid& g, int F, int K, const T* AqL, long long ldL, T* out,
+                         long long ldo);
+
+}  // namespace bpx

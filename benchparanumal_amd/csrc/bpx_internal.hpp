@@ -8,6 +8,7 @@
 #include <mutex>
 #include <string>
 
+#include "box.hpp"
 #include "bpx.h"
 
 namespace bpx {
@@ -315,6 +316,13 @@ int launch_ogs_gather_dot_fold(hipStream_t s, int Nblocks, const int* blockStart
 template <typename T>
 int launch_ogs_gather_dot(hipStream_t s, int Nblocks, const int* blockStarts, const int* rowStarts,
                           const int* colIds, const T* q, T* gq, const T* p, double* part, int mode = 0);
+
+// The same gather on a structured hex box, no maps (box_gather.hip): F
+// fields in [element][field][node] layout, K vectors of AqL ldL apart and of
+// out ldo apart. A vector of AqL must be smaller than 2^31 - 8 bytes.
+template <typename T>
+int launch_box_gather(hipStream_t s, const BoxGrid& g, int F, int K, const T* AqL, long long ldL, T* out,
+                      long long ldo);
 
 // linAlg. Reductions run on a fixed grid of kRedBlocks workgroups and write
 // kRedBlocks FP64 partials; launch_fold sums partials into a device scalar.

@@ -473,6 +473,13 @@ class bp_t : public solver_t {
   // o_grad (Nnodes) = -sum over local copies of (D lam).G(D u)
   int KappaGradient(const dfloat* o_u, const dfloat* o_lam, dfloat* o_grad);
   hlong LatticeNodes() const;
+  // the hex box's rows in closed form (box.hpp): local values are gathered
+  // without maps while a local vector's byte offsets fit in 31 bits
+  bool haveBox = false;
+  BoxGrid box;
+  // Aq = gather(AqL) on the reference rows, K vectors one after another
+  template <typename T>
+  int GatherLocal(const T* o_AqL, T* o_Aq, int K = 1) const;
   // FP32 CG with FP64 reliable updates every `interval` iterations until
   // ||b - A x|| / ||b|| < tol; stats = {updates, FP32 iterations, rel. residual}
   int SolveMixed(dfloat* o_x, const dfloat* o_b, double tol, int interval, int maxit, double* stats);

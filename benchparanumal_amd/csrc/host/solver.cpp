@@ -347,6 +347,8 @@ int bp_t::Setup(platform_t& p, mesh_t& m, int bp_, dfloat lambda_) {
     if (int st = o_GlobalToLocal.upload(GlobalToLocal, s)) return st;
   }
   if (int st = gHalo.SetupFromGather(ogs)) return st;
+  haveBox = m.elementType == ELEM_HEX && (long long)NLocal * (long long)sizeof(double) < 0x7FFFFFF8LL;
+  if (haveBox) box.set(m.opts.nx, m.opts.ny, m.opts.nz, m.N);
   std::vector<dlong> list(m.Nelements);
   for (dlong e = 0; e < m.Nelements; ++e) list[e] = e;
   if (int st = o_elementList.upload(list, s)) return st;
@@ -529,7 +531,16 @@ int bp_t::Operator(const dfloat* o_q, dfloat* o_Aq) {
   if (int st = gHalo.ExchangeStart(o_q, 1)) return st;
   if (int st = gHalo.ExchangeFinish(o_q, 1)) return st;
   if (int st = AxLocal(o_q, o_AqL.ptr())) return st;
-  return ogs.Gather<double>(*platform, o_Aq, o_AqL.ptr(), 1);
+  return GatherLocal<double>(o_AqL.ptr(), o_Aq);
+}
+
+template <typename T>
+int bp_t::GatherLocal(const T* o_AqL, T* o_Aq, int K) const {
+  if (haveBox && ogs.Ngather > 0)
+    return launch_box_gather<T>(platform->stream, box, Nfields, K, o_AqL, NLocal, o_Aq, ogs.Ngather);
+  for (int r = 0; r < K; ++r)  // one gather per vector, same maps
+    if (int st = ogs.Gather<T>(*platform, o_Aq + (size_t)r * ogs.Ngather, o_AqL + (size_t)r * NLocal, 1)) return st;
+  return BPX_OK;
 }
 
 // The operator with the q.Aq partials on reference-order vectors: through
@@ -562,6 +573,7 @@ int bp_t::FromSolve(const dfloat* o_s, dfloat* o_ref) {
 
 int bp_t::OperatorS(const dfloat* o_q, dfloat* o_Aq) {
   if (int st = AxLocal(o_q, o_AqL.ptr(), SolveG2L())) return st;
+  if (!permuted) return GatherLocal<double>(o_AqL.ptr(), o_Aq);
   const ogs::ogs_t& G = SolveOgs();
   return launch_ogs_gather<double>(platform->stream, G.NrowBlocksT, 1, G.o_blockRowStartsT.ptr(),
                                    G.o_rowStartsT.ptr(), G.o_colIdsT.ptr(), o_AqL.ptr(), o_Aq, ogs.gatherMode);
@@ -803,10 +815,7 @@ int bp_t::OperatorKrhs(int K, const dfloat* o_q, dfloat* o_Aq, int chunk) {
     if (int st = o_AqLk.alloc(need)) return st;
   }
   if (int st = AxLocalKrhs(K, o_q, o_AqLk.ptr(), chunk)) return st;
-  for (int r = 0; r < K; ++r)  // one gather per right-hand side, same maps
-    if (int st = ogs.Gather<double>(*platform, o_Aq + (size_t)r * ogs.Ngather, o_AqLk.ptr() + (size_t)r * NLocal, 1))
-      return st;
-  return BPX_OK;
+  return GatherLocal<double>(o_AqLk.ptr(), o_Aq, K);
 }
 
 int bp_t::OperatorDot32(const float* o_q, float* o_Aq, double* part, int* npart, const CgFold<float>* fold) {
@@ -1116,7 +1125,7 @@ int bp_t::Operator32(const float* o_q, float* o_Aq) {
   if (int st = ax<float>(o_q, o_AqL32.ptr(), o_wJ32.ptr(), o_ggeo32.ptr(), o_gllw32.ptr(), o_D32.ptr(),
                          o_I32.ptr(), o_MM32.ptr(), o_invV32.ptr()))
     return st;
-  return ogs.Gather<float>(*platform, o_Aq, o_AqL32.ptr(), 1);
+  return GatherLocal<float>(o_AqL32.ptr(), o_Aq);
 }
 
 // device copies of the nodal coordinates and GLL weights (forcing, error norms)
