@@ -293,7 +293,7 @@ __global__ __launch_bounds__(BT) void k_bm_init(const BatchChunk* __restrict__ c
     part_true[blockIdx.x] = tt;
     part_rr[blockIdx.x] = tr;
     if (ch.first) {
-      const BatchState z{0, 0, 0, 0, 0, 0, 0, maxit, 0, 0};
+      const BatchState z{0, 0, 0, 0, 0, 0, 0, maxit, 0, 0, 0, 0};
       inner[ch.pid] = z;
       outer[ch.pid] = z;
     }

@@ -39,6 +39,9 @@ struct FastDiv {
   }
 };
 
+// largest vector of the box kernels (bytes): offsets are unsigned 32-bit
+constexpr unsigned kBoxRange = 0xFFF00000u;
+
 struct BoxGrid {
   int nx = 0, ny = 0, nz = 0, N = 0;
   FastDiv dx, dy;

@@ -10,4 +10,12 @@ template <typename T, int NQ>
 int launch_box_gather_nq(hipStream_t s, const BoxGrid& g, int F, int K, const T* AqL, long long ldL, T* out,
                          long long ldo);
 
+template <typename T, int NQ>
+int launch_box_ax_nq(hipStream_t s, const BoxAxArgs<T>& a);
+template <typename T, int NQ>
+int launch_box_update_r_nq(hipStream_t s, const BoxGrid& g, int F, const BoxUpdateR<T>& u, int* nrr);
+
+// elements per workgroup of the Ax: about 256 lanes
+constexpr int box_epb(int Nq) { return Nq * Nq >= 144 ? 1 : 256 / (Nq * Nq); }
+
 }  // namespace bpx

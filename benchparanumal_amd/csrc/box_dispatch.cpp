@@ -20,6 +20,43 @@ int launch_box_gather(hipStream_t s, const BoxGrid& g, int F, int K, const T* Aq
 #undef BPX_CALL
 }
 
+template <typename T>
+int launch_box_ax(hipStream_t s, const BoxAxArgs<T>& a) {
+  const BoxGrid& g = a.g;
+  if (!a.q || !a.AqL) return set_error(BPX_ERR_INVALID_ARGUMENT, "box Ax: null device pointer");
+  if (!a.geo || !a.eo || (a.geoKind == BOX_GEO_TRILINEAR && !a.z) || (a.geoKind != BOX_GEO_TRILINEAR && !a.wJ) ||
+      (a.geoKind != BOX_GEO_STORED && !a.w))
+    return set_error(BPX_ERR_INVALID_ARGUMENT, "box Ax: null geometry/operator pointer");
+  if (a.items) {
+    if (!a.probs || !a.bst || (a.fold && (!a.part || !a.r || !a.p || !a.x || !a.part_rr)))
+      return set_error(BPX_ERR_INVALID_ARGUMENT, "box Ax: incomplete batch arguments");
+  } else if (a.fold && (!a.part || !a.r || !a.p || !a.x || !a.part_rr || !a.hist_rr || !a.hist_alpha || !a.st || a.p == a.q))
+    return set_error(BPX_ERR_INVALID_ARGUMENT, "box Ax: incomplete CG arguments");
+#define BPX_CALL(NQ) case NQ: return launch_box_ax_nq<T, NQ>(s, a);
+  BPX_BOX_SWITCH(BPX_CALL)
+#undef BPX_CALL
+}
+
+int box_ax_elements(int Nq) { return box_epb(Nq); }
+
+int box_ax_partials(const BoxGrid& g, int F) {
+  const int epb = box_epb(g.N + 1);
+  return (g.elements() + epb - 1) / epb * F;
+}
+
+template <typename T>
+int launch_box_update_r(hipStream_t s, const BoxGrid& g, int F, const BoxUpdateR<T>& u, int* nrr) {
+  if (!u.AqL || !u.r || !u.part_pAp || !u.part_rr || !u.st || !u.hist_rr || !u.hist_alpha)
+    return set_error(BPX_ERR_INVALID_ARGUMENT, "box update: null device pointer");
+#define BPX_CALL(NQ) case NQ: return launch_box_update_r_nq<T, NQ>(s, g, F, u, nrr);
+  BPX_BOX_SWITCH(BPX_CALL)
+#undef BPX_CALL
+}
+
+template int launch_box_update_r<double>(hipStream_t, const BoxGrid&, int, const BoxUpdateR<double>&, int*);
+template int launch_box_update_r<float>(hipStream_t, const BoxGrid&, int, const BoxUpdateR<float>&, int*);
+template int launch_box_ax<double>(hipStream_t, const BoxAxArgs<double>&);
+template int launch_box_ax<float>(hipStream_t, const BoxAxArgs<float>&);
 template int launch_box_gather<double>(hipStream_t, const BoxGrid&, int, int, const double*, long long, double*,
                                        long long);
 template int launch_box_gather<float>(hipStream_t, const BoxGrid&, int, int, const float*, long long, float*,

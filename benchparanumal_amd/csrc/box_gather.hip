@@ -20,8 +20,11 @@
 // 288 -> 210 us.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "box_common.hpp"
 #include "buffer_rsrc.hpp"
+#include "fold.hpp"
 
 #ifndef BPX_NQ
 #error "compile with -DBPX_NQ=<Nq>"
@@ -32,6 +35,9 @@ namespace {
 
 constexpr int GT = 256;  // lanes per workgroup
 
+__device__ inline double fmad(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ inline float fmad(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
 template <int NQ>
 constexpr int box_gather_slots() {
   return GT / ((NQ - 1) * (NQ - 1));
@@ -41,9 +47,9 @@ constexpr int box_gather_slots() {
 template <typename T, int NQ>
 struct BoxColumn {
   static constexpr int N = NQ - 1, NQ2 = NQ * NQ, NP = NQ2 * NQ;
-  int row, stride, nk;      // row of k = 1, rows per layer, owned layers (0: idle lane)
-  int own, ox, oy, oxy;     // byte offsets of the copies at k = 0
-  int zown, zx, zy, zxy;    // one layer of elements up, their k = 0 plane
+  int row, stride, nk;         // row of k = 1, rows per layer, owned layers (0: idle lane)
+  unsigned own, ox, oy, oxy;   // byte offsets of the copies at k = 0
+  unsigned zown, zx, zy, zxy;  // one layer of elements up, their k = 0 plane
 
   __device__ inline void set(const BoxGrid& g, int F, int f, int e, int c, bool on) {
     int ex, ey, ez;
@@ -54,19 +60,19 @@ struct BoxColumn {
     stride = Nx * Ny;
     nk = on ? Nz : 0;
     row = g.base<N>(F, ex, ey, ez) + f * stride * Nz + (j - 1) * Nx + i - 1;
-    constexpr int S = (int)sizeof(T);
-    const int ES = F * NP * S;  // bytes of an element
-    const int at = e * ES + f * NP * S;
+    constexpr unsigned S = sizeof(T);
+    const unsigned ES = F * NP * S;  // bytes of an element
+    const unsigned at = e * ES + f * NP * S;
     const bool fx = i == N, fy = j == N, fz = Nz == N;
-    own = on ? at + (j * NQ + i) * S : kBufMasked;
-    ox = on && fx ? at + ES + j * NQ * S : kBufMasked;
-    oy = on && fy ? at + g.nx * ES + i * S : kBufMasked;
-    oxy = on && fx && fy ? at + (g.nx + 1) * ES : kBufMasked;
-    const int up = g.nx * g.ny * ES;
-    zown = on && fz ? own + up : kBufMasked;
-    zx = on && fz && fx ? ox + up : kBufMasked;
-    zy = on && fz && fy ? oy + up : kBufMasked;
-    zxy = on && fz && fx && fy ? oxy + up : kBufMasked;
+    own = on ? at + (j * NQ + i) * S : kBoxMasked;
+    ox = on && fx ? at + ES + j * NQ * S : kBoxMasked;
+    oy = on && fy ? at + g.nx * ES + i * S : kBoxMasked;
+    oxy = on && fx && fy ? at + (g.nx + 1) * ES : kBoxMasked;
+    const unsigned up = g.nx * g.ny * ES;
+    zown = on && fz ? own + up : kBoxMasked;
+    zx = on && fz && fx ? ox + up : kBoxMasked;
+    zy = on && fz && fy ? oy + up : kBoxMasked;
+    zxy = on && fz && fx && fy ? oxy + up : kBoxMasked;
   }
 };
 
@@ -123,12 +129,83 @@ __global__ __launch_bounds__(GT) void k_box_gather(BoxGrid g, int F, int per_xcd
   BoxColumn<T, NQ> b;
   b.set(g, F, blockIdx.y, e, (int)threadIdx.x - es * N2, es < SL && e < g.elements());
   T* o = out + (size_t)blockIdx.z * ldo;
-  box_column_sums<T, NQ>(b, buffer_rsrc(AqL + (size_t)blockIdx.z * ldL), [&](int k, T v) {
+  box_column_sums<T, NQ>(b, box_rsrc(AqL + (size_t)blockIdx.z * ldL), [&](int k, T v) {
     if (k <= b.nk) o[b.row + (k - 1) * b.stride] = v;
   });
 }
 
+// The end of a CG iteration on the box: the gather of Ap with
+// cg::UpdateCG's r -= alpha Ap (libs/core/linearSolverCG.cpp:131-156), Ap
+// itself never stored. alpha = r.r / p.Ap from the Ax kernel's partials;
+// one partial of the new r.r per workgroup. The arithmetic per row and the
+// breakdown test are k_cg_update_r's. A workgroup walks items (element
+// group, field) of its XCD's eighth; its first item's loads are issued
+// before the partials are folded.
+template <typename T, int NQ>
+__global__ __launch_bounds__(GT) void k_box_update_r(BoxGrid g, int F, int items, BoxUpdateR<T> u) {
+  constexpr int N = NQ - 1, N2 = N * N, SL = box_gather_slots<NQ>();
+  __shared__ double s_f[GT + 1];
+  if (u.st->done || u.st->stop_at) return;
+  const int es = (int)threadIdx.x / N2, c = (int)threadIdx.x - es * N2;
+  const int per = (items + 7) / 8, x = blockIdx.x & 7;
+  const int end = min((x + 1) * per, items), step = (int)(gridDim.x >> 3);
+  const __amdgpu_buffer_rsrc_t rs = box_rsrc(u.AqL);
+  T alpha = T(0);
+  double rr = 0;
+  bool folded = false;
+  for (int it = x * per + (int)(blockIdx.x >> 3);; it += step) {
+    const bool have = it < end;
+    if (folded && !have) break;  // (a workgroup without items still folds once: uniform)
+    const int grp = it / F, e = grp * SL + es;
+    BoxColumn<T, NQ> b;
+    b.set(g, F, it - grp * F, e, c, have && es < SL && e < g.elements());
+    T Ap[N], r[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) r[k] = u.r[b.nk > k ? b.row + k * b.stride : 0];
+    box_column_sums<T, NQ>(b, rs, [&](int k, T v) { Ap[k - 1] = v; });
+    if (!folded) {
+      const double pAp = block_fold<GT>(u.part_pAp, u.npAp, s_f);
+      const double al = u.hist_rr[u.k] / pAp;
+      if (!isfinite(al) || !(pAp > 0.0)) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+          u.st->breakdown = 1;
+          u.st->done = 1;
+          u.st->iter = u.k;
+        }
+        return;
+      }
+      if (blockIdx.x == 0 && threadIdx.x == 0) u.hist_alpha[u.k] = al;
+      alpha = (T)al;
+      folded = true;
+    }
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      if (k < b.nk) {
+        const T rn = fmad(-alpha, Ap[k], r[k]);
+        u.r[b.row + k * b.stride] = rn;
+        rr += (double)rn * (double)rn;
+      }
+    }
+  }
+  const double t = block_sum<GT>(rr, s_f);
+  if (threadIdx.x == 0) u.part_rr[blockIdx.x] = t;
+}
+
 }  // namespace
+
+template <typename T, int NQ>
+int launch_box_update_r_nq(hipStream_t s, const BoxGrid& g, int F, const BoxUpdateR<T>& u, int* nrr) {
+  constexpr int SL = box_gather_slots<NQ>();
+  const int items = (g.elements() + SL - 1) / SL * F;
+  const int grid = std::min((items + 7) / 8 * 8, kBoxRrParts);
+  hipLaunchKernelGGL((k_box_update_r<T, NQ>), dim3(grid), dim3(GT), 0, s, g, F, items, u);
+  BPX_HIP(hipGetLastError());
+  *nrr = grid;
+  return BPX_OK;
+}
+
+template int launch_box_update_r_nq<double, BPX_NQ>(hipStream_t, const BoxGrid&, int, const BoxUpdateR<double>&, int*);
+template int launch_box_update_r_nq<float, BPX_NQ>(hipStream_t, const BoxGrid&, int, const BoxUpdateR<float>&, int*);
 
 template <typename T, int NQ>
 int launch_box_gather_nq(hipStream_t s, const BoxGrid& g, int F, int K, const T* AqL, long long ldL, T* out,

@@ -28,7 +28,22 @@ int hip_error(hipError_t e, const char* what);
   } while (0)
 
 // ------------------------------------------------- kernel parameter packs --
-struct CgState;
+// Device-resident CG state (one per solver).
+struct CgState {
+  double tol2;    // stop when r.r <= tol2
+  int iter;       // iterations completed (valid once done, or after finish)
+  int done;       // 1 once r.r <= tol2, the iteration cap is reached, or breakdown
+  int breakdown;  // 1 when p.Ap or r.r stopped being finite/positive
+  int maxit;
+  // k + 1 when the stopping test of k_cg_update_p fired at iteration k, else
+  // 0. That kernel records its stop here, never in `done`: its other
+  // workgroups test `done` and `stop_at <= k` on entry, and a stop written
+  // by its own first workgroup must not make them skip the x update of
+  // iteration k - 1, which every row still needs. The kernels after it
+  // treat stop_at != 0 as done, and k_cg_finish folds it into `done`.
+  int stop_at;
+};
+
 
 // The CG direction update folded into the fused BP5 operator (one field):
 // for the element's interior rows, the only copies of their rows, the Ax
@@ -217,7 +232,11 @@ struct BatchState {
   double tol2;
   double rnorm;    // ||r|| when the problem stopped
   int iter, done, breakdown, maxit;
-  int updates, pad;  // mixed solve: FP64 corrections made
+  int updates;  // mixed solve: FP64 corrections made
+  // FP64 solve: k + 1 when the stopping test fired at iteration k (see
+  // CgState::stop_at), alpha of the last iteration, the tolerance
+  int stop_at;
+  double alpha, tol;
 };
 // BP5 Ax over the elements of one degree group; variant = workgroup shape
 // (bp5_batch_epb: elements per workgroup, 0 if the variant does not exist)
@@ -324,6 +343,88 @@ template <typename T>
 int launch_box_gather(hipStream_t s, const BoxGrid& g, int F, int K, const T* AqL, long long ldL, T* out,
                       long long ldo);
 
+// One problem of a batch on the box kernels and one workgroup's elements of
+// it (workgroups never straddle problems)
+struct BoxBatchProb {
+  BoxGrid g;
+  long long off = 0;   // first row in the concatenated vectors
+  long long loc = 0;   // first local node
+  long long el0 = 0;   // first element in the degree's coefficient array
+  int pAp0 = 0, npAp = 0;  // partials of p.Ap (one per Ax workgroup)
+  int rr0 = 0, ninit = 0, nrr = 0;  // partials of r.r: of the initial residual, of later ones
+};
+struct BoxBatchItem {
+  int pid, e0;
+};
+struct BatchState;
+
+// BP5 / BP6 Ax on a structured hex box (box_ax.hip): F fields, q on the
+// reference rows, AqL in [element][field][node] layout, both smaller than
+// 2^31 - 8 bytes.
+enum { BOX_GEO_TRILINEAR = 0, BOX_GEO_AFFINE = 1, BOX_GEO_STORED = 2 };
+template <typename T>
+struct BoxAxArgs {
+  BoxGrid g;
+  int F = 1;
+  int geoKind = BOX_GEO_TRILINEAR;
+  const T* geo = nullptr;    // 24 map coefficients per element, 6 factors per element, or 6 per node (FP32 only)
+  const T* wJ = nullptr;     // J per element (affine), wJ per node (stored)
+  const T* z = nullptr;      // GLL nodes (trilinear)
+  const T* w = nullptr;      // GLL weights (trilinear, affine)
+  const T* eo = nullptr;     // even-odd table of D (EvenOdd, box_ax.hip)
+  const T* kappa = nullptr;  // coefficient on the node lattice (FP64), or null
+  T lambda = 0;
+  const T* q = nullptr;
+  T* AqL = nullptr;
+  int K = 1;  // right-hand sides, q ldq apart, AqL ldAq apart
+  long long ldq = 0, ldAq = 0;
+  hipEvent_t evStart = nullptr, evStop = nullptr;  // as AxArgs
+  // set: also one FP64 partial of q.Aq per workgroup and field (box_ax_partials of them)
+  double* part = nullptr;
+  // The start of CG iteration k inside the Ax (k_cg_update_p's arithmetic,
+  // stopping test and flags): q is the direction of iteration k-1, the new
+  // direction r + beta q goes to p (another vector: neighbours read q), and
+  // with pending x += alpha_{k-1} q
+  int fold = 0, k = 0, pending = 0, nrr = 0;
+  const T* r = nullptr;
+  T* p = nullptr;
+  T* x = nullptr;
+  const double* part_rr = nullptr;
+  double* hist_rr = nullptr;
+  const double* hist_alpha = nullptr;
+  CgState* st = nullptr;
+  double tol = 0;
+  // a degree's problems of a batch (FP64, trilinear): nitems workgroups; the
+  // vectors, geo and the partials are the concatenated ones, p the other
+  // direction vector and the iteration, its scalars and flags the problem's
+  // state (q and p by the parity of its iteration)
+  int nitems = 0;
+  const BoxBatchItem* items = nullptr;
+  const BoxBatchProb* probs = nullptr;
+  BatchState* bst = nullptr;
+};
+template <typename T>
+int launch_box_ax(hipStream_t s, const BoxAxArgs<T>& a);
+int box_ax_elements(int Nq);  // elements per workgroup
+int box_ax_partials(const BoxGrid& g, int F);
+
+// The end of a CG iteration: r -= alpha gather(AqL) with alpha from the p.Ap
+// partials, and partials of r.r (*nrr of them, at most kBoxRrParts)
+constexpr int kBoxRrParts = 1024;
+template <typename T>
+struct BoxUpdateR {
+  const T* AqL = nullptr;
+  T* r = nullptr;
+  int k = 0, npAp = 0;
+  const double* part_pAp = nullptr;
+  double* part_rr = nullptr;
+  CgState* st = nullptr;
+  const double* hist_rr = nullptr;
+  double* hist_alpha = nullptr;
+};
+template <typename T>
+int launch_box_update_r(hipStream_t s, const BoxGrid& g, int F, const BoxUpdateR<T>& u, int* nrr);
+
 // linAlg. Reductions run on a fixed grid of kRedBlocks workgroups and write
 // kRedBlocks FP64 partials; launch_fold sums partials into a device scalar.
 constexpr int kRedThreads = 1024;
@@ -343,22 +444,6 @@ int launch_dot(hipStream_t s, dlong N, const T* x, const T* y, double* part, dou
 // cg::UpdateCG (r -= alpha Ap, x += alpha p) with r.r into *out (device)
 int launch_update_cg(hipStream_t s, dlong N, double alpha, const double* p, const double* Ap, double* x,
                      double* r, double* part, double* out);
-
-// Device-resident CG state (one per solver).
-struct CgState {
-  double tol2;    // stop when r.r <= tol2
-  int iter;       // iterations completed (valid once done, or after finish)
-  int done;       // 1 once r.r <= tol2, the iteration cap is reached, or breakdown
-  int breakdown;  // 1 when p.Ap or r.r stopped being finite/positive
-  int maxit;
-  // k + 1 when the stopping test of k_cg_update_p fired at iteration k, else
-  // 0. That kernel records its stop here, never in `done`: its other
-  // workgroups test `done` and `stop_at <= k` on entry, and a stop written
-  // by its own first workgroup must not make them skip the x update of
-  // iteration k - 1, which every row still needs. The kernels after it
-  // treat stop_at != 0 as done, and k_cg_finish folds it into `done`.
-  int stop_at;
-};
 
 // Work buffers of the allocation-free CG solve, carved from the file-scope
 // device array of cg_noalloc.hip (sizes: kNoAllocMaxN for p and Ap,

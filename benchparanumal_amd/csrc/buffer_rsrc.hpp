@@ -5,6 +5,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "box.hpp"
+
 namespace bpx {
 namespace {
 
@@ -15,6 +17,16 @@ constexpr int kBufFlags = 0x00020000;         // dword 3: 32-bit data format (gf
 template <typename T>
 __device__ inline __amdgpu_buffer_rsrc_t buffer_rsrc(const T* base) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), (short)0, kBufRange, kBufFlags);
+}
+
+// The structured-box kernels' resources: vectors of up to kBoxRange bytes.
+// Offsets are unsigned 32-bit numbers; kBoxMasked plus any offset within an
+// element stays beyond the range without wrapping.
+constexpr unsigned kBoxMasked = kBoxRange;  // (kBoxRange: box.hpp; the host tests sizes against it)
+
+template <typename T>
+__device__ inline __amdgpu_buffer_rsrc_t box_rsrc(const T* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(base), (short)0, (int)kBoxRange, kBufFlags);
 }
 
 template <typename T>

@@ -743,7 +743,7 @@ int bpx_bp_create(bpx_platform p, bpx_mesh m, int bp, double lambda, bpx_bp* out
     delete b;
     return st;
   }
-  b->solver = new cg(*p->p, b->bp.Ns, 0, b->bp.GatherPartials());
+  b->solver = new cg(*p->p, std::max(b->bp.Ns, b->bp.ogs.Ngather), 0, b->bp.GatherPartials());
   if (int st = b->solver->status()) {
     delete b;
     return st;
@@ -820,7 +820,10 @@ int bpx_bp_set_tuning(bpx_bp b, int gatherMode, int fused, int fused32) {
     return set_error(BPX_ERR_UNSUPPORTED, "bp: no fused operator for this problem (BP5, one field)");
   auto& t = b->bp.tuning;
   if (gatherMode >= 0) t.gatherMode = b->bp.ogs.gatherMode = gatherMode;
-  if (fused >= 0) t.fused64 = fused;
+  if (fused >= 0) {
+    t.fused64 = fused;
+    b->bp.boxFused64 = fused != 0;
+  }
   if (fused32 >= 0) {
     if (int st = b->bp.Prepare32()) return st;  // so a later first use does not re-time
     t.fused32 = fused32;

@@ -121,6 +121,41 @@ int bp_batch_t::Setup(platform_t& p, const std::vector<MeshOpts>& opts, dfloat l
     if (int st = G.D.upload(*D, s)) return st;
   }
 
+  // ---- the box kernels' tables: per degree the elements' map coefficients
+  // and the Ax workgroups, per problem its grid and offsets
+  std::vector<BoxBatchProb> probs(nprob);
+  int npAp = 0;
+  for (auto& G : groups) {
+    const int epb = box_ax_elements(G.Nq);
+    std::vector<double> geo, eo;
+    std::vector<BoxBatchItem> items;
+    const mesh_t* any = nullptr;
+    for (int i = 0; i < nprob; ++i) {
+      const mesh_t& m = meshes[i];
+      if (m.N != G.N) continue;
+      any = &m;
+      BoxBatchProb& pr = probs[i];
+      pr.g.set(m.opts.nx, m.opts.ny, m.opts.nz, m.N);
+      pr.off = off[i];
+      pr.loc = localOff[i];
+      pr.el0 = (long long)geo.size() / 24;
+      pr.pAp0 = npAp;
+      pr.npAp = (m.Nelements + epb - 1) / epb;
+      npAp += pr.npAp;
+      std::vector<double> c;
+      m.TrilinearCoefficients(c);
+      geo.insert(geo.end(), c.begin(), c.end());
+      for (dlong e = 0; e < m.Nelements; e += epb) items.push_back({i, (int)e});
+    }
+    if (int st = box_even_odd_table(*any, eo)) return st;
+    if (int st = G.boxGeo.upload(geo, s)) return st;
+    if (int st = G.boxEo.upload(eo, s)) return st;
+    if (int st = G.boxZ.upload(any->gllz, s)) return st;
+    if (int st = G.boxW.upload(any->gllw, s)) return st;
+    if (int st = G.boxItems.upload(items, s)) return st;
+  }
+  if (int st = o_probs.upload(probs, s)) return st;
+
   // ---- concatenated gather maps, super-blocks and chunks
   std::vector<dlong> rowStarts(1, 0), colIds;
   std::vector<BatchSuper> supers;
@@ -170,6 +205,24 @@ int bp_batch_t::Setup(platform_t& p, const std::vector<MeshOpts>& opts, dfloat l
 int bp_batch_t::AxGroup(const Group& G, int variant, const double* q, double* AqL) const {
   return launch_bp5_batch(stream, G.N, variant, (int)G.Nel, G.elementList.ptr(), G.G2L.ptr(), G.wJ.ptr(),
                           G.ggeo.ptr(), G.D.ptr(), lambda, q, AqL + G.loff, G.elemPid.ptr(), o_state.ptr());
+}
+
+// the box kernels' Ax of one degree's problems that their states do not skip
+BoxAxArgs<double> bp_batch_t::BoxArgs(const Group& G, const double* q) {
+  BoxAxArgs<double> a;
+  a.g.N = G.N;
+  a.geo = G.boxGeo.ptr();
+  a.z = G.boxZ.ptr();
+  a.w = G.boxW.ptr();
+  a.eo = G.boxEo.ptr();
+  a.lambda = lambda;
+  a.q = q;
+  a.AqL = o_AqL.ptr();
+  a.nitems = (int)G.boxItems.length();
+  a.items = G.boxItems.ptr();
+  a.probs = o_probs.ptr();
+  a.bst = o_state.ptr();
+  return a;
 }
 
 // Times every workgroup shape of each degree group's Ax on the group's own
@@ -346,9 +399,7 @@ int bp_batch_t::Segment(double* o_x, const double* o_b, double tol, int interval
   }
   if (int st = launch_bm_flush(stream, nchunks, o_chunks.ptr(), o_c32.ptr(), o_x, out)) return st;
   for (const auto& G : groups)
-    if (int st = launch_bp5_batch(stream, G.N, G.variant, (int)G.Nel, G.elementList.ptr(), G.G2L.ptr(), G.wJ.ptr(),
-                                  G.ggeo.ptr(), G.D.ptr(), lambda, o_x, o_AqL.ptr() + G.loff, G.elemPid.ptr(), out))
-      return st;
+    if (int st = launch_box_ax<double>(stream, BoxArgs(G, o_x))) return st;  // (the outer states are o_state)
   if (int st = launch_batch_gather_only(stream, nsupers, o_supers.ptr(), o_rowStarts.ptr(), o_colIds.ptr(),
                                         o_AqL.ptr(), o_Ax64.ptr(), out))
     return st;

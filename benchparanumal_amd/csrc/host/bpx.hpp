@@ -145,12 +145,9 @@ class mesh_t {
   void MaskedGlobalIds(int Nfields, std::vector<hlong>& ids) const;
   // per element, for x, y and z in turn, the coefficients of r, s, t, rs,
   // rt, st, rst of the trilinear map through its 8 vertices, and one pad
-  // (24 values): the nodal coordinates are this map at the GLL nodes
+  // (24 values): the nodal coordinates are this map at the GLL nodes, by
+  // construction (Setup and SetupDevice)
   void TrilinearCoefficients(std::vector<double>& c) const;
-  // whether every local node lies on its element's trilinear map of the 8
-  // vertices at the GLL point (to 1e-12 of the box size): then the
-  // geometric factors are the map's exact derivatives
-  bool NodesAreTrilinear() const;
   // mesh_t::PlotFields (libs/mesh/meshPlotFields3D.cpp:31-121): VTU file of
   // the local nodes with Nfields values each (QL: host, [e][f][n]); each
   // element is drawn as N^3 sub-cubes of 6 tetrahedra
@@ -163,9 +160,6 @@ class mesh_t {
   // until EnsureHost copies them down.
   int SetupDevice(platform_t& p, const MeshOpts& o);
   int EnsureHost();
-  // whether every node is its element's trilinear map (NodesAreTrilinear),
-  // checked on the device for a device mesh
-  bool NodesTrilinear();
   // masked ids (MaskedGlobalIds) formed on the device from o_globalIds
   int MaskedGlobalIdsDevice(int Nfields, hlong* o_ids) const;
   bool onDevice = false;
@@ -300,6 +294,19 @@ struct CgWork {
   double* hist_alpha = nullptr;
 };
 
+// A CG iteration that an operator queues whole, in its own kernels: iterate(k)
+// does k_cg_update_p's work of iteration k (with pending also the x update of
+// k-1), the operator with p.Ap, and k_cg_update_r's.
+template <typename T>
+class CgSteps {
+ public:
+  virtual ~CgSteps() = default;
+  virtual int iterate(int k, double tol, bool pending) = 0;
+  virtual const T* direction(int k) const = 0;  // p of iteration k
+  int nrr = kRedBlocks;                         // partials of r.r that the last iteration left
+  dlong rows = 0;                               // of the vectors
+};
+
 // cg (libs/core/linearSolverCG.cpp:33-156) with device-resident scalars.
 // T is the vector/operator precision; reductions accumulate in FP64.
 template <typename T>
@@ -318,7 +325,10 @@ class cg_t {
   // npart_max: most partials apply_dot writes (at least kRedBlocks is kept)
   int Setup(platform_t& p, dlong N, int npart_max = 0);
   int Solve(const Apply& apply, const ApplyDot& apply_dot, T* o_x, T* o_r, double tol, int MAXIT,
-            int* iterations, const ApplyFold& apply_fold = ApplyFold(), dlong fold_rows = 0);
+            int* iterations, const ApplyFold& apply_fold = ApplyFold(), dlong fold_rows = 0,
+            CgSteps<T>* steps = nullptr);
+  int Reserve(int MAXIT);  // histories of MAXIT + 1 entries
+  bool padded = true;      // rows of o_p and o_Ap that belong to no node hold zeros
   // squared residual norms r.r of the last Solve (entry 0 = initial)
   int History(std::vector<double>& rr, std::vector<double>& alpha);
 
@@ -336,7 +346,8 @@ class cg_t {
 template <typename T>
 int cg_run(hipStream_t s, dlong N, const CgWork<T>& w, const typename cg_t<T>::Apply& apply,
            const typename cg_t<T>::ApplyDot& apply_dot, T* o_x, T* o_r, double tol, int MAXIT, int* iterations,
-           const typename cg_t<T>::ApplyFold& apply_fold = typename cg_t<T>::ApplyFold(), dlong fold_rows = 0);
+           const typename cg_t<T>::ApplyFold& apply_fold = typename cg_t<T>::ApplyFold(), dlong fold_rows = 0,
+           CgSteps<T>* steps = nullptr);
 
 class cg : public linearSolver_t {
  public:
@@ -344,6 +355,9 @@ class cg : public linearSolver_t {
   int status() const { return status_; }
   int Solve(solver_t& solver, dfloat* o_x, dfloat* o_r, dfloat tol, int MAXIT, int verbose,
             int* iterations) override;
+  // the same with whole iterations queued by `steps` (null: by the solver's calls)
+  int Solve(solver_t& solver, dfloat* o_x, dfloat* o_r, dfloat tol, int MAXIT, int verbose, int* iterations,
+            CgSteps<dfloat>* steps);
   cg_t<double> impl;
 
  private:
@@ -361,7 +375,7 @@ class bp_t : public solver_t {
   int OperatorDot(const dfloat* o_q, dfloat* o_Aq, double* part, int* npart) override;
   int GatherPartials() const {
     return std::max({ogs_gather_partials(ogs.NrowBlocksT), ogs_gather_partials(sharedOgs.NrowBlocksT),
-                     ogs_gather_partials(solveOgs.NrowBlocksT), 1});
+                     ogs_gather_partials(solveOgs.NrowBlocksT), haveBox ? box_ax_partials(box, Nfields) : 1, 1});
   }
 
   // Solve space: the row order the CG solvers run in. For BP5 with one
@@ -388,10 +402,10 @@ class bp_t : public solver_t {
   // partials (FP64 and FP32; fused or not as tuned)
   int OperatorS(const dfloat* o_q, dfloat* o_Aq);
   int OperatorDotS(const dfloat* o_q, dfloat* o_Aq, double* part, int* npart);
-  int OperatorDot32(const float* o_q, float* o_Aq, double* part, int* npart, const CgFold<float>* fold = nullptr);
+  int OperatorDot32(const float* o_q, float* o_Aq, double* part, int* npart);
   // cg::Solve on reference-order x and r, run in the solve space
   int SolveCG(cg& solver, dfloat* o_x, dfloat* o_r, dfloat tol, int maxit, int verbose, int* iterations);
-  deviceBuffer<double> o_sx, o_sr, o_sb;  // solve-space copies (created on first use)
+  deviceBuffer<double> o_sx, o_sr;  // solve-space copies
   // times the launch choices that give identical results (gather
   // workgroup order; fused or unfused CG operator) and keeps the fastest
   int Tune();
@@ -424,29 +438,31 @@ class bp_t : public solver_t {
     size_t used = 0;
   };
   OpTimer* opTimer32 = nullptr;
+  int TimedStep32(const std::function<int()>& step);  // step with those events
   // when set, the next Ax launch (BP1-BP6) stamps its start and end into
   // these (AxArgs::evStart / evStop)
   hipEvent_t axEvStart = nullptr, axEvStop = nullptr;
-  // Fused operator for CG (BP5, one field): single-copy nodes written by
+  // Fused operator for CG: on the box (boxAx) the two kernels above. BP5 at
+  // N = 15 in FP64: single-copy nodes written by
   // the Ax straight into Aq, shared nodes gathered (see launch_bp5_fused).
   // fused = the maps are built; tuning.fused64/fused32 = it is used.
   bool fused = false;
   int PrepareFused();
   int PrepareFusedDevice();  // PrepareFused from the device maps (device mesh)
-  template <typename T>
-  int OperatorDotFused(const T* o_q, T* o_Aq, double* part, int* npart, const CgFold<T>* fold = nullptr);
+  int OperatorDotFused(const double* o_q, double* o_Aq, double* part, int* npart,
+                       const CgFold<double>* fold = nullptr);
   // the rows a folded CG operator leaves to k_cg_update_p (the solve space's
-  // rows before the first interior run), or 0 where no fold applies:
-  // precision 64 or 32, the fused operator in use, and cgFold set
-  dlong FoldRows(int precision) const;
-  // fold the CG direction update into the fused operator (same bits): bit 0
-  // for the FP64 solves, bit 1 for the FP32 iterations of the mixed solve
-  int cgFold = 1;
+  // rows before the first interior run), or 0 where no fold applies
+  dlong FoldRows() const;
+  // fold the CG direction update into the Ax (same bits): bit 0 for the FP64
+  // solves, bit 1 for the FP32 iterations of the mixed solve
+  int cgFold = 3;
   int OperatorDotUnfusedS(const dfloat* o_q, dfloat* o_Aq, double* part, int* npart);
-  int OperatorDotUnfused32(const float* o_q, float* o_Aq, double* part, int* npart);
-  // Ax into the local vector; G2L = the GlobalToLocal map to read q
+  // Ax into the local vector
+  int AxLocal(const dfloat* o_q, dfloat* o_AqL);
+  // the same from the stored factors; G2L = the GlobalToLocal map to read q
   // through (default: the reference rows)
-  int AxLocal(const dfloat* o_q, dfloat* o_AqL, const dlong* G2L = nullptr);
+  int AxStored(const dfloat* o_q, dfloat* o_AqL, const dlong* G2L = nullptr);
   int Operator32(const float* o_q, float* o_Aq);
   int Forcing(dfloat* o_b);
   int NodeCoordinates();  // o_x, o_y, o_z, o_gllwRhs on first use
@@ -477,6 +493,35 @@ class bp_t : public solver_t {
   // without maps while a local vector's byte offsets fit in 31 bits
   bool haveBox = false;
   BoxGrid box;
+  // BP5 and BP6 on the box: the geometry formed in the kernel from the
+  // elements' trilinear maps (or their affine factors), no index maps
+  // (box_ax.hip). BP5 at N = 15 in FP64 keeps the stored factors.
+  bool boxAx = false;
+  deviceBuffer<double> o_boxGeo, o_boxZ, o_boxEo, o_kappa;
+  deviceBuffer<float> o_boxEo32;
+  // the box Ax's arguments in precision T; q and AqL as given
+  template <typename T>
+  BoxAxArgs<T> BoxArgs(const T* o_q, T* o_AqL) const;
+  // whether precision T's operator runs on box_ax.hip
+  template <typename T>
+  bool BoxAx() const {
+    return sizeof(T) == 8 ? boxAx : haveBox && bp == 5;
+  }
+  // The CG operator in two kernels per iteration, the Ax with the direction
+  // update and the gather with the residual update, on the reference rows
+  // unless pinned off: boxFused64 (FP64), tuning.fused32 (FP32 and, for
+  // affine elements, tuning.fused64 are timed).
+  bool boxFused64 = true;
+  bool BoxFused(int precision) const {
+    if (precision == 32) return tuning.fused32;
+    return bp == 5 && mesh->opts.affine ? tuning.fused64 != 0 : boxFused64;
+  }
+  // CG iterations on reference-order x and r with the directions p0 and p1
+  // (p1 is Ap where the two kernels are not used)
+  template <typename T>
+  std::unique_ptr<CgSteps<T>> BoxSteps(T* p0, T* p1, T* x, T* r, T* AqL, const CgWork<T>& w);
+  template <typename T>
+  int TuneBox(int& choice, double& fused_us, double& unfused_us);
   // Aq = gather(AqL) on the reference rows, K vectors one after another
   template <typename T>
   int GatherLocal(const T* o_AqL, T* o_Aq, int K = 1) const;
@@ -488,7 +533,7 @@ class bp_t : public solver_t {
   struct MixedWork {
     dlong N = -1;
     int maxit = 0;
-    deviceBuffer<double> Ax64, part_true, part_rr, part_pAp, hist_rr, hist_alpha, norm, xs, bs;
+    deviceBuffer<double> Ax64, part_true, part_rr, part_pAp, hist_rr, hist_alpha, norm;
     deviceBuffer<float> r32, p32, Ap32, c32;
     deviceBuffer<CgState> state;
   } mixed;
@@ -522,7 +567,6 @@ class bp_t : public solver_t {
   // 0..Nshared-1 of the solve space), the first interior row, the Ax
   // kernel's p.Ap partials
   deviceBuffer<double> o_slots;
-  deviceBuffer<float> o_slots32;
   ogs::ogs_t sharedOgs;
   dlong fusedS0 = 0;
   deviceBuffer<double> o_partAx;
@@ -531,10 +575,9 @@ class bp_t : public solver_t {
   int Prepare32();
   bool have32 = false;
   int tri32 = 0;  // the FP32 BP5 operator forms its geometric factors from the trilinear maps
-  // FP32 BP5 geometry: 0 = from the elements' trilinear maps when every
-  // node is its element's trilinear map of the vertices (checked on the
-  // host), else stored factors rounded to FP32; 1 = stored factors rounded
-  // to FP32 always. Changing it rebuilds the FP32 operator on next use.
+  // FP32 BP5 geometry (non-affine): 0 = from the elements' trilinear maps,
+  // 1 = stored factors rounded to FP32. Changing it rebuilds the FP32
+  // operator on next use.
   int fp32Geometry = 0;
   int SetFp32Geometry(int mode);
   deviceBuffer<float> o_wJ32, o_ggeo32, o_gllw32, o_D32, o_I32, o_MM32, o_invV32, o_AqL32;
@@ -557,12 +600,16 @@ class bp_solve_view_t : public solver_t {
   int OperatorDot(const dfloat* o_q, dfloat* o_Aq, double* part, int* npart) override {
     return bp.OperatorDotS(o_q, o_Aq, part, npart);
   }
-  dlong FoldRows() const override { return bp.FoldRows(64); }
+  dlong FoldRows() const override { return bp.FoldRows(); }
   int OperatorDotFold(const CgFold<dfloat>& fold, dfloat* o_Aq, double* part, int* npart) override {
-    return bp.OperatorDotFused<double>(fold.p, o_Aq, part, npart, &fold);
+    return bp.OperatorDotFused(fold.p, o_Aq, part, npart, &fold);
   }
   bp_t& bp;
 };
+
+// the box kernels' table of D (EvenOdd in box_ax.hip): one row of Nq values
+// per n <= (Nq-1)/2; an error if D is not antisymmetric to rounding
+int box_even_odd_table(const mesh_t& m, std::vector<double>& t);
 
 // Ragged batch of BP5 problems (box meshes of any size and degree), one CG
 // per problem, all problems advanced together from a replayed hipGraph.
@@ -589,6 +636,9 @@ class bp_batch_t {
     deviceBuffer<dlong> elementList, G2L, elemPid;
     deviceBuffer<double> wJ, ggeo, D;
     deviceBuffer<float> wJ32, ggeo32, D32;  // rounded to FP32 for the mixed solve
+    // the FP64 operator on the box kernels: map coefficients, 1D data, workgroups
+    deviceBuffer<double> boxGeo, boxZ, boxW, boxEo;
+    deviceBuffer<BoxBatchItem> boxItems;
     int variant = 0;             // workgroup shape chosen by the tuner
     double us[3] = {-1, -1, -1};  // its timings (us; -1 = shape not available)
   };
@@ -603,6 +653,8 @@ class bp_batch_t {
  private:
   int Tune();
   int AxGroup(const Group& G, int variant, const double* q, double* AqL) const;
+  BoxAxArgs<double> BoxArgs(const Group& G, const double* q);
+  deviceBuffer<BoxBatchProb> o_probs;
   int Iteration(double* o_x, double tol);
   int Capture(double* o_x, double tol);
   int Prepare32();

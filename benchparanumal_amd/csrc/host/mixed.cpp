@@ -28,23 +28,16 @@ int bp_t::SolveMixed(dfloat* o_x, const dfloat* o_b, double tol, int interval, i
   if (!(tol > 0) || interval < 1 || maxit < 1)
     return set_error(BPX_ERR_INVALID_ARGUMENT, "mixed solve: tol > 0, interval >= 1 and maxit >= 1 required");
   if (int st = Prepare32()) return st;
-  const dlong N = Ns;  // the recurrence runs in the solve space
+  const dlong N = ogs.Ngather;
   hipStream_t s = platform->stream;
   MixedWork& w = mixed;
   if (w.N != N || w.maxit < maxit) {
     int st;
     if ((st = w.Ax64.alloc(N)) || (st = w.r32.alloc(N)) || (st = w.p32.alloc(N)) || (st = w.Ap32.alloc(N)) ||
-        (st = w.xs.alloc(N)) || (st = w.bs.alloc(N)) ||
-        (st = w.c32.alloc(N)) || (st = w.part_true.alloc(kRedBlocks)) || (st = w.part_rr.alloc(kRedBlocks)) ||
+        (st = w.c32.alloc(N)) || (st = w.part_true.alloc(kRedBlocks)) || (st = w.part_rr.alloc(std::max(kRedBlocks, kBoxRrParts))) ||
         (st = w.part_pAp.alloc(std::max(GatherPartials(), kRedBlocks))) || (st = w.hist_rr.alloc(maxit + 1)) ||
         (st = w.hist_alpha.alloc(maxit + 1)) || (st = w.state.alloc(1)) || (st = w.norm.alloc(1)))
       return st;
-    // padding rows of the solve space are never written by the fused
-    // operator: they must hold zeros from the start
-    if (N > 0) {
-      BPX_HIP(hipMemsetAsync(w.Ap32.ptr(), 0, (size_t)N * sizeof(float), s));
-      BPX_HIP(hipMemsetAsync(w.p32.ptr(), 0, (size_t)N * sizeof(float), s));
-    }
     w.N = N;
     w.maxit = maxit;
   }
@@ -56,14 +49,10 @@ int bp_t::SolveMixed(dfloat* o_x, const dfloat* o_b, double tol, int interval, i
     if (stats) stats[0] = stats[1] = stats[2] = 0;
     return platform->finish();
   }
-  double* xs = w.xs.ptr();
-  const double* bs = w.bs.ptr();
-  if (int st = ToSolve(o_x, xs)) return st;
-  if (int st = ToSolve(o_b, w.bs.ptr())) return st;
   // true residual of the initial guess
   auto true_residual = [&](double* rn) -> int {
-    if (int st = OperatorS(xs, w.Ax64.ptr())) return st;
-    if (int st = launch_true_residual(s, N, bs, w.Ax64.ptr(), w.r32.ptr(), w.part_true.ptr(), w.part_rr.ptr()))
+    if (int st = Operator(o_x, w.Ax64.ptr())) return st;
+    if (int st = launch_true_residual(s, N, o_b, w.Ax64.ptr(), w.r32.ptr(), w.part_true.ptr(), w.part_rr.ptr()))
       return st;
     if (int st = launch_fold(s, w.part_true.ptr(), kRedBlocks, w.norm.ptr())) return st;
     BPX_HIP(hipMemcpyAsync(platform->h_scalar, w.norm.ptr(), sizeof(double), hipMemcpyDeviceToHost, s));
@@ -77,45 +66,43 @@ int bp_t::SolveMixed(dfloat* o_x, const dfloat* o_b, double tol, int interval, i
   if (!std::isfinite(rn) || !std::isfinite(nb)) return set_error(BPX_ERR_BREAKDOWN, "mixed solve: non-finite residual");
   int k = 0, kseg = 0, updates = 0;  // kseg: iteration within the current recurrence
   CgState* st_d = w.state.ptr();
-  // with the fused FP32 operator the direction update of the interior rows
-  // is done inside it (CgFold); k_cg_update_p covers the rows below
-  const dlong frows = FoldRows(32);
+  CgWork<float> cw;
+  cw.state = st_d;
+  cw.part_rr = w.part_rr.ptr();
+  cw.part_pAp = w.part_pAp.ptr();
+  cw.hist_rr = w.hist_rr.ptr();
+  cw.hist_alpha = w.hist_alpha.ptr();
+  std::unique_ptr<CgSteps<float>> steps;  // the box operator queues whole iterations
+  if (BoxAx<float>())
+    steps = BoxSteps<float>(w.p32.ptr(), w.Ap32.ptr(), w.c32.ptr(), w.r32.ptr(), o_AqL32.ptr(), cw);
   while (rn > tol * nb && k < maxit) {
     const int n = std::min(interval, maxit - k);
     for (int j = 0; j < n; ++j, ++k, ++kseg) {
       // tol = 0: the recurrence never stops itself; the FP64 test decides.
       // c += alpha p of the previous iteration rides along (not across a
       // correction, before which it is flushed)
-      if (int st = launch_cg_update_p<float>(s, frows > 0 ? frows : N, kseg, w.r32.ptr(), w.p32.ptr(), w.c32.ptr(),
-                                             w.part_rr.ptr(), kRedBlocks, st_d, w.hist_rr.ptr(), w.hist_alpha.ptr(),
-                                             0.0, j > 0))
+      if (steps) {
+        if (j == 0) steps->nrr = kRedBlocks;  // r.r of the true residual
+        if (int st = steps->iterate(kseg, 0.0, j > 0)) return st;
+        continue;
+      }
+      if (int st = launch_cg_update_p<float>(s, N, kseg, w.r32.ptr(), w.p32.ptr(), w.c32.ptr(), w.part_rr.ptr(),
+                                             kRedBlocks, st_d, w.hist_rr.ptr(), w.hist_alpha.ptr(), 0.0, j > 0))
         return st;
       int npart = 0;
-      if (frows > 0) {
-        CgFold<float> f;
-        f.on = 1;
-        f.k = kseg;
-        f.pending = j > 0;
-        f.p = w.p32.ptr();
-        f.r = w.r32.ptr();
-        f.x = w.c32.ptr();
-        f.hist_rr = w.hist_rr.ptr();
-        f.hist_alpha = w.hist_alpha.ptr();
-        f.st = st_d;
-        if (int st = OperatorDot32(w.p32.ptr(), w.Ap32.ptr(), w.part_pAp.ptr(), &npart, &f)) return st;
-      } else if (int st = OperatorDot32(w.p32.ptr(), w.Ap32.ptr(), w.part_pAp.ptr(), &npart)) {
+      if (int st = TimedStep32([&] { return OperatorDot32(w.p32.ptr(), w.Ap32.ptr(), w.part_pAp.ptr(), &npart); }))
         return st;
-      }
       if (int st = launch_cg_update_r<float>(s, N, kseg, w.Ap32.ptr(), w.r32.ptr(), w.part_pAp.ptr(), npart,
                                              w.part_rr.ptr(), st_d, w.hist_rr.ptr(), w.hist_alpha.ptr()))
         return st;
     }
     // the last iteration's c update (unless the recurrence stopped, which
     // has applied or dropped it already)
-    if (int st = launch_cg_flush_x<float>(s, N, kseg - 1, w.p32.ptr(), w.c32.ptr(), w.hist_alpha.ptr(), st_d, true))
+    if (int st = launch_cg_flush_x<float>(s, N, kseg - 1, steps ? steps->direction(kseg - 1) : w.p32.ptr(), w.c32.ptr(),
+                                          w.hist_alpha.ptr(), st_d, true))
       return st;
     // reliable update: x += c, r = b - A x in FP64, r32 = float(r)
-    if (int st = launch_accumulate_f32(s, N, w.c32.ptr(), xs)) return st;
+    if (int st = launch_accumulate_f32(s, N, w.c32.ptr(), o_x)) return st;
     if (int st = true_residual(&rn)) return st;
     ++updates;
     if (!std::isfinite(rn)) return set_error(BPX_ERR_BREAKDOWN, "mixed solve: non-finite residual");
@@ -126,7 +113,6 @@ int bp_t::SolveMixed(dfloat* o_x, const dfloat* o_b, double tol, int interval, i
     // residual unless that has converged
     if (hst.done || hst.stop_at || hst.breakdown) kseg = 0;
   }
-  if (int st = FromSolve(xs, o_x)) return st;
   if (int st = platform->finish()) return st;
   if (stats) {
     stats[0] = updates;

@@ -69,6 +69,12 @@ int hip_error(hipError_t e, const char* what) {
   return set_error(code, std::string(what) + ": " + hipGetErrorString(e));
 }
 
+int box_even_odd_table(const mesh_t& m, std::vector<double>& t) {
+  if (!even_odd_rows(m.D.data(), m.Nq, m.Nq, -1, t))
+    return set_error(BPX_ERR_INVALID_ARGUMENT, "bp: the derivative matrix is not antisymmetric");
+  return BPX_OK;
+}
+
 // ----------------------------------------------------------- platform ---
 platform_t::~platform_t() {
   if (device >= 0) (void)hipSetDevice(device);
@@ -149,7 +155,7 @@ int cg_t<T>::Setup(platform_t& p, dlong N_, int npart_max) {
   if (int st = o_p.alloc(N)) return st;
   if (int st = o_Ap.alloc(N)) return st;
   if (int st = o_state.alloc(1)) return st;
-  if (int st = o_part_rr.alloc(kRedBlocks)) return st;
+  if (int st = o_part_rr.alloc(std::max(kRedBlocks, kBoxRrParts))) return st;
   if (int st = o_part_pAp.alloc(std::max(npart_max, kRedBlocks))) return st;
   if (N > 0) {
     BPX_HIP(hipMemsetAsync(o_p.ptr(), 0, N * sizeof(T), p.stream));
@@ -163,13 +169,9 @@ int cg_t<T>::Setup(platform_t& p, dlong N_, int npart_max) {
 // after every chunk of 16 iterations, so a converged solve stops early.
 template <typename T>
 int cg_t<T>::Solve(const Apply& apply, const ApplyDot& apply_dot, T* o_x, T* o_r, double tol, int MAXIT,
-                   int* iterations, const ApplyFold& apply_fold, dlong fold_rows) {
+                   int* iterations, const ApplyFold& apply_fold, dlong fold_rows, CgSteps<T>* steps) {
   if (MAXIT < 0) return set_error(BPX_ERR_INVALID_ARGUMENT, "cg: MAXIT < 0");
-  if (hist_len < MAXIT + 1) {
-    if (int st = o_hist_rr.alloc(MAXIT + 1)) return st;
-    if (int st = o_hist_alpha.alloc(MAXIT + 1)) return st;
-    hist_len = MAXIT + 1;
-  }
+  if (int st = Reserve(MAXIT)) return st;
   CgWork<T> w;
   w.p = o_p.ptr();
   w.Ap = o_Ap.ptr();
@@ -178,14 +180,23 @@ int cg_t<T>::Solve(const Apply& apply, const ApplyDot& apply_dot, T* o_x, T* o_r
   w.part_pAp = o_part_pAp.ptr();
   w.hist_rr = o_hist_rr.ptr();
   w.hist_alpha = o_hist_alpha.ptr();
-  return cg_run<T>(platform->stream, N, w, apply, apply_dot, o_x, o_r, tol, MAXIT, iterations, apply_fold,
-                   fold_rows);
+  return cg_run<T>(platform->stream, steps ? steps->rows : N, w, apply, apply_dot, o_x, o_r, tol, MAXIT, iterations, apply_fold,
+                   fold_rows, steps);
+}
+
+template <typename T>
+int cg_t<T>::Reserve(int MAXIT) {
+  if (hist_len >= MAXIT + 1) return BPX_OK;
+  if (int st = o_hist_rr.alloc(MAXIT + 1)) return st;
+  if (int st = o_hist_alpha.alloc(MAXIT + 1)) return st;
+  hist_len = MAXIT + 1;
+  return BPX_OK;
 }
 
 template <typename T>
 int cg_run(hipStream_t s, dlong N, const CgWork<T>& w, const typename cg_t<T>::Apply& apply,
            const typename cg_t<T>::ApplyDot& apply_dot, T* o_x, T* o_r, double tol, int MAXIT, int* iterations,
-           const typename cg_t<T>::ApplyFold& apply_fold, dlong fold_rows) {
+           const typename cg_t<T>::ApplyFold& apply_fold, dlong fold_rows, CgSteps<T>* steps) {
   if (MAXIT < 0) return set_error(BPX_ERR_INVALID_ARGUMENT, "cg: MAXIT < 0");
   CgState* st_d = w.state;
   double* prr = w.part_rr;
@@ -205,6 +216,10 @@ int cg_run(hipStream_t s, dlong N, const CgWork<T>& w, const typename cg_t<T>::A
     const int n = std::min(chunk, MAXIT - queued);
     for (int k = queued; k < queued + n; ++k) {
       int npart = kRedBlocks;
+      if (steps) {
+        if (int st = steps->iterate(k, tol, k > 0)) return st;
+        continue;
+      }
       if (apply_fold) {
         // the direction update of the rows below fold_rows here, of the
         // others inside the operator
@@ -240,7 +255,7 @@ int cg_run(hipStream_t s, dlong N, const CgWork<T>& w, const typename cg_t<T>::A
         return st;
     }
     queued += n;
-    if (int st = launch_cg_finish(s, queued, MAXIT, prr, kRedBlocks, st_d, w.hist_rr)) return st;
+    if (int st = launch_cg_finish(s, queued, MAXIT, prr, steps ? steps->nrr : kRedBlocks, st_d, w.hist_rr)) return st;
     if (queued < MAXIT) {
       BPX_HIP(hipMemcpyAsync(&hst, st_d, sizeof(CgState), hipMemcpyDeviceToHost, s));
       BPX_HIP(hipStreamSynchronize(s));
@@ -252,7 +267,8 @@ int cg_run(hipStream_t s, dlong N, const CgWork<T>& w, const typename cg_t<T>::A
   // stopped after its last queued iteration (converged there, or MAXIT):
   // that iteration's x update is still to be applied
   if (MAXIT > 0 && hst.done && !hst.breakdown && hst.iter == queued) {
-    if (int st = launch_cg_flush_x<T>(s, N, queued - 1, w.p, o_x, w.hist_alpha, st_d, false)) return st;
+    const T* p = steps ? steps->direction(queued - 1) : w.p;
+    if (int st = launch_cg_flush_x<T>(s, N, queued - 1, p, o_x, w.hist_alpha, st_d, false)) return st;
     BPX_HIP(hipStreamSynchronize(s));
   }
   if (iterations) *iterations = (MAXIT == 0) ? 0 : hst.iter;
@@ -277,14 +293,19 @@ template class cg_t<double>;
 template class cg_t<float>;
 template int cg_run<double>(hipStream_t, dlong, const CgWork<double>&, const cg_t<double>::Apply&,
                             const cg_t<double>::ApplyDot&, double*, double*, double, int, int*,
-                            const cg_t<double>::ApplyFold&, dlong);
+                            const cg_t<double>::ApplyFold&, dlong, CgSteps<double>*);
 template int cg_run<float>(hipStream_t, dlong, const CgWork<float>&, const cg_t<float>::Apply&,
                            const cg_t<float>::ApplyDot&, float*, float*, double, int, int*,
-                           const cg_t<float>::ApplyFold&, dlong);
+                           const cg_t<float>::ApplyFold&, dlong, CgSteps<float>*);
 
 cg::cg(platform_t& p, dlong N, dlong Nhalo, int npart_max) { status_ = impl.Setup(p, N + Nhalo, npart_max); }
 
 int cg::Solve(solver_t& solver, dfloat* o_x, dfloat* o_r, dfloat tol, int MAXIT, int verbose, int* iterations) {
+  return Solve(solver, o_x, o_r, tol, MAXIT, verbose, iterations, nullptr);
+}
+
+int cg::Solve(solver_t& solver, dfloat* o_x, dfloat* o_r, dfloat tol, int MAXIT, int verbose, int* iterations,
+              CgSteps<dfloat>* steps) {
   if (status_) return status_;
   int its = 0;
   cg_t<double>::ApplyDot fused;
@@ -297,7 +318,7 @@ int cg::Solve(solver_t& solver, dfloat* o_x, dfloat* o_r, dfloat tol, int MAXIT,
       return solver.OperatorDotFold(f, Aq, part, n);
     };
   const int st = impl.Solve([&](const double* q, double* Aq) { return solver.Operator(q, Aq); }, fused, o_x, o_r,
-                            tol, MAXIT, &its, fold, foldRows);
+                            tol, MAXIT, &its, fold, foldRows, steps);
   if (iterations) *iterations = its;
   if (verbose) {
     std::vector<double> rr, al;
@@ -347,7 +368,8 @@ int bp_t::Setup(platform_t& p, mesh_t& m, int bp_, dfloat lambda_) {
     if (int st = o_GlobalToLocal.upload(GlobalToLocal, s)) return st;
   }
   if (int st = gHalo.SetupFromGather(ogs)) return st;
-  haveBox = m.elementType == ELEM_HEX && (long long)NLocal * (long long)sizeof(double) < 0x7FFFFFF8LL;
+  // (one field always fits: a mesh has at most 2^31/6 local nodes)
+  haveBox = m.elementType == ELEM_HEX && (unsigned long long)NLocal * sizeof(double) <= kBoxRange;
   if (haveBox) box.set(m.opts.nx, m.opts.ny, m.opts.nz, m.N);
   std::vector<dlong> list(m.Nelements);
   for (dlong e = 0; e < m.Nelements; ++e) list[e] = e;
@@ -415,7 +437,20 @@ int bp_t::Setup(platform_t& p, mesh_t& m, int bp_, dfloat lambda_) {
     if (!eo.empty())
       if (int st = o_eo.upload(eo, s)) return st;
   }
+  boxAx = haveBox && (bp == 6 || (bp == 5 && m.N < 15));
+  if (boxAx) {
+    std::vector<double> eo;
+    if (int st = box_even_odd_table(m, eo)) return st;
+    if (int st = o_boxEo.upload(eo, s)) return st;
+    if (int st = o_boxZ.upload(m.gllz, s)) return st;
+    if (!affine) {
+      std::vector<double> c;
+      m.TrilinearCoefficients(c);
+      if (int st = o_boxGeo.upload(c, s)) return st;
+    }
+  }
   if (int st = m.onDevice ? PrepareFusedDevice() : PrepareFused()) return st;
+  if (boxAx && bp == 5 && affine) fused = true;
   if (int st = Tune()) return st;
   return p.finish();
 }
@@ -448,7 +483,6 @@ int bp_t::ax(const T* q, T* AqL, const T* wJ, const T* ggeo, const T* gllw, cons
     else
       a.eo = o_eo32.length() ? o_eo32.ptr() : nullptr;
   }
-  if constexpr (std::is_same<T, float>::value) a.tri = tri32;
   a.evStart = axEvStart;
   a.evStop = axEvStop;
   if (mesh->elementType != ELEM_HEX) {
@@ -468,7 +502,41 @@ int bp_t::ax(const T* q, T* AqL, const T* wJ, const T* ggeo, const T* gllw, cons
   return launch_bp3_ax<T>(platform->stream, a);
 }
 
-int bp_t::AxLocal(const dfloat* o_q, dfloat* o_AqL, const dlong* G2L) {
+template <typename T>
+BoxAxArgs<T> bp_t::BoxArgs(const T* o_q, T* o_AqL) const {
+  BoxAxArgs<T> a;
+  const int affine = mesh->opts.affine;
+  a.g = box;
+  a.F = Nfields;
+  if constexpr (std::is_same<T, double>::value) {
+    a.geoKind = affine ? BOX_GEO_AFFINE : BOX_GEO_TRILINEAR;
+    a.geo = affine ? o_ggeo.ptr() : o_boxGeo.ptr();
+    a.wJ = o_wJ.ptr();
+    a.z = o_boxZ.ptr();
+    a.w = o_gllw.ptr();
+    a.eo = o_boxEo.ptr();
+    a.kappa = haveKappa ? o_kappa.ptr() : nullptr;
+  } else {
+    a.geoKind = affine ? BOX_GEO_AFFINE : tri32 ? BOX_GEO_TRILINEAR : BOX_GEO_STORED;
+    a.geo = o_ggeo32.ptr();
+    a.wJ = a.z = o_wJ32.ptr();  // the GLL nodes with the trilinear maps
+    a.w = o_gllw32.ptr();
+    a.eo = o_boxEo32.ptr();
+  }
+  a.lambda = (T)lambda;
+  a.q = o_q;
+  a.AqL = o_AqL;
+  a.evStart = axEvStart;
+  a.evStop = axEvStop;
+  return a;
+}
+
+int bp_t::AxLocal(const dfloat* o_q, dfloat* o_AqL) {
+  if (boxAx) return launch_box_ax<double>(platform->stream, BoxArgs<double>(o_q, o_AqL));
+  return AxStored(o_q, o_AqL);
+}
+
+int bp_t::AxStored(const dfloat* o_q, dfloat* o_AqL, const dlong* G2L) {
   if (haveKappa)
     return ax<double>(o_q, o_AqL, mesh->opts.affine ? o_wJK.ptr() : o_wJ.ptr(), o_ggeoK.ptr(), o_gllw.ptr(),
                       o_D.ptr(), nullptr, nullptr, nullptr, G2L);
@@ -500,10 +568,19 @@ int bp_t::SetKappa(const dfloat* o_kappa) {
     if (int st = o_lattice.upload(lat, s)) return st;
     if (int st = latticeOgs.SetupRows(NLocal, (dlong)Nnodes, lat.data())) return st;
     if (int st = latticeOgs.Upload(*platform)) return st;
-    if (int st = o_ggeoK.alloc((size_t)NLocal * 6)) return st;
-    if (m.opts.affine)
-      if (int st = o_wJK.alloc(NLocal)) return st;
+    if (boxAx) {
+      if (int st = this->o_kappa.alloc((size_t)Nnodes)) return st;
+    } else {
+      if (int st = o_ggeoK.alloc((size_t)NLocal * 6)) return st;
+      if (m.opts.affine)
+        if (int st = o_wJK.alloc(NLocal)) return st;
+    }
     if (int st = o_gradL.alloc(NLocal)) return st;
+  }
+  if (boxAx) {  // the kernel scales by the lattice values themselves
+    BPX_HIP(hipMemcpyAsync(this->o_kappa.ptr(), o_kappa, (size_t)Nnodes * sizeof(double), hipMemcpyDeviceToDevice, s));
+    haveKappa = true;
+    return BPX_OK;
   }
   if (int st = launch_kappa_geometry(s, NLocal, m.Nq, m.opts.affine, o_lattice.ptr(), o_kappa, o_ggeo.ptr(),
                                      o_wJ.ptr(), o_gllw.ptr(), o_ggeoK.ptr(), o_wJK.ptr()))
@@ -547,6 +624,13 @@ int bp_t::GatherLocal(const T* o_AqL, T* o_Aq, int K) const {
 // the solve space when the rows are renumbered (the Aq rows are the same
 // sums either way, bit for bit).
 int bp_t::OperatorDot(const dfloat* o_q, dfloat* o_Aq, double* part, int* npart) {
+  if (boxAx) {
+    BoxAxArgs<double> a = BoxArgs<double>(o_q, o_AqL.ptr());
+    a.part = part;
+    *npart = box_ax_partials(box, Nfields);
+    if (int st = launch_box_ax<double>(platform->stream, a)) return st;
+    return GatherLocal<double>(o_AqL.ptr(), o_Aq);
+  }
   if (!permuted) return OperatorDotUnfusedS(o_q, o_Aq, part, npart);
   if (int st = ToSolve(o_q, o_sx.ptr())) return st;
   if (int st = OperatorDotS(o_sx.ptr(), o_sr.ptr(), part, npart)) return st;
@@ -572,7 +656,7 @@ int bp_t::FromSolve(const dfloat* o_s, dfloat* o_ref) {
 }
 
 int bp_t::OperatorS(const dfloat* o_q, dfloat* o_Aq) {
-  if (int st = AxLocal(o_q, o_AqL.ptr(), SolveG2L())) return st;
+  if (int st = AxStored(o_q, o_AqL.ptr(), SolveG2L())) return st;
   if (!permuted) return GatherLocal<double>(o_AqL.ptr(), o_Aq);
   const ogs::ogs_t& G = SolveOgs();
   return launch_ogs_gather<double>(platform->stream, G.NrowBlocksT, 1, G.o_blockRowStartsT.ptr(),
@@ -580,12 +664,12 @@ int bp_t::OperatorS(const dfloat* o_q, dfloat* o_Aq) {
 }
 
 int bp_t::OperatorDotS(const dfloat* o_q, dfloat* o_Aq, double* part, int* npart) {
-  if (fused && tuning.fused64) return OperatorDotFused<double>(o_q, o_Aq, part, npart);
+  if (fused && tuning.fused64) return OperatorDotFused(o_q, o_Aq, part, npart);
   return OperatorDotUnfusedS(o_q, o_Aq, part, npart);
 }
 
 int bp_t::OperatorDotUnfusedS(const dfloat* o_q, dfloat* o_Aq, double* part, int* npart) {
-  if (int st = AxLocal(o_q, o_AqL.ptr(), SolveG2L())) return st;
+  if (int st = AxStored(o_q, o_AqL.ptr(), SolveG2L())) return st;
   const ogs::ogs_t& G = SolveOgs();
   *npart = ogs_gather_partials(G.NrowBlocksT);
   return launch_ogs_gather_dot<double>(platform->stream, G.NrowBlocksT, G.o_blockRowStartsT.ptr(),
@@ -593,8 +677,116 @@ int bp_t::OperatorDotUnfusedS(const dfloat* o_q, dfloat* o_Aq, double* part, int
                                        ogs.gatherMode);
 }
 
+// CG iterations of a box operator (BoxAx) on the reference rows. fused: the
+// Ax (with the direction update, or with fold off after k_cg_update_p) and
+// k_box_update_r; else k_cg_update_p, Ax, gather into p1 and k_cg_update_r.
+// Both take p.Ap from the Ax's partials and give the same bits but for the
+// order of the r.r sums.
+template <typename T>
+class BoxCgSteps : public CgSteps<T> {
+ public:
+  BoxCgSteps(bp_t& b_, T* p0, T* p1, T* x_, T* r_, T* AqL_, const CgWork<T>& w_)
+      : b(b_), p{p0, p1}, x(x_), r(r_), AqL(AqL_), w(w_) {
+    const int precision = 8 * (int)sizeof(T);
+    this->rows = b.ogs.Ngather;
+    fused = b.BoxFused(precision);
+    fold = fused && (b.cgFold & (precision == 64 ? 1 : 2));
+  }
+  int iterate(int k, double tol, bool pending) override {
+    hipStream_t s = b.platform->stream;
+    const dlong N = b.ogs.Ngather;
+    if (!fold)
+      if (int st = launch_cg_update_p<T>(s, N, k, r, p[0], x, w.part_rr, this->nrr, w.state, w.hist_rr, w.hist_alpha,
+                                         tol, pending))
+        return st;
+    const int npAp = box_ax_partials(b.box, b.Nfields);
+    auto apply = [&]() -> int {
+      BoxAxArgs<T> a = b.BoxArgs<T>(fold ? p[(k + 1) & 1] : p[0], AqL);
+      a.part = w.part_pAp;
+      if (fold) {
+        a.fold = 1;
+        a.k = k;
+        a.pending = pending;
+        a.nrr = this->nrr;
+        a.r = r;
+        a.p = p[k & 1];
+        a.x = x;
+        a.part_rr = w.part_rr;
+        a.hist_rr = w.hist_rr;
+        a.hist_alpha = w.hist_alpha;
+        a.st = w.state;
+        a.tol = tol;
+      }
+      if (int st = launch_box_ax<T>(s, a)) return st;
+      if (!fused) return b.GatherLocal<T>(AqL, p[1]);
+      BoxUpdateR<T> u;
+      u.AqL = AqL;
+      u.r = r;
+      u.k = k;
+      u.npAp = npAp;
+      u.part_pAp = w.part_pAp;
+      u.part_rr = w.part_rr;
+      u.st = w.state;
+      u.hist_rr = w.hist_rr;
+      u.hist_alpha = w.hist_alpha;
+      return launch_box_update_r<T>(s, b.box, b.Nfields, u, &this->nrr);
+    };
+    if (int st = sizeof(T) == 4 ? b.TimedStep32(apply) : apply()) return st;
+    if (fused) return BPX_OK;
+    this->nrr = kRedBlocks;
+    return launch_cg_update_r<T>(s, N, k, p[1], r, w.part_pAp, npAp, w.part_rr, w.state, w.hist_rr, w.hist_alpha);
+  }
+  const T* direction(int k) const override { return fold ? p[k & 1] : p[0]; }
+
+ private:
+  bp_t& b;
+  T* p[2];
+  T *x, *r, *AqL;
+  CgWork<T> w;
+  bool fused, fold;
+};
+
+template <typename T>
+std::unique_ptr<CgSteps<T>> bp_t::BoxSteps(T* p0, T* p1, T* x, T* r, T* AqL, const CgWork<T>& w) {
+  return std::unique_ptr<CgSteps<T>>(new BoxCgSteps<T>(*this, p0, p1, x, r, AqL, w));
+}
+template std::unique_ptr<CgSteps<float>> bp_t::BoxSteps<float>(float*, float*, float*, float*, float*,
+                                                               const CgWork<float>&);
+
+// Solves to a tolerance, with a variable coefficient or on affine elements
+// run on the box operator. A fixed number of iterations (tol = 0) on the
+// perturbed box keeps the reference's stored factors and the summation order
+// that its history is compared in: once CG has resolved the isolated top of
+// the spectrum, a difference of 1e-16 in the operator grows 1000-fold every
+// 30 iterations (24^3, p = 7, 100 iterations: residuals of two equally exact
+// operators 2e-12 to 1e-7 apart over 12 meshes), so a faster operator would
+// give another history, where a converged solution is the same.
 int bp_t::SolveCG(cg& solver, dfloat* o_x, dfloat* o_r, dfloat tol, int maxit, int verbose, int* iterations) {
-  if (!permuted) return solver.Solve(*this, o_x, o_r, tol, maxit, verbose, iterations);
+  if (boxAx && ogs.Ngather > 0 && (tol > 0 || haveKappa || mesh->opts.affine)) {
+    if (solver.status()) return solver.status();
+    if (maxit < 0) return set_error(BPX_ERR_INVALID_ARGUMENT, "cg: MAXIT < 0");
+    cg_t<double>& c = solver.impl;
+    if (int st = c.Reserve(maxit)) return st;
+    CgWork<double> w;
+    w.state = c.o_state.ptr();
+    w.part_rr = c.o_part_rr.ptr();
+    w.part_pAp = c.o_part_pAp.ptr();
+    w.hist_rr = c.o_hist_rr.ptr();
+    w.hist_alpha = c.o_hist_alpha.ptr();
+    c.padded = false;  // both directions' buffers hold reference rows now
+    const auto steps = BoxSteps<double>(c.o_p.ptr(), c.o_Ap.ptr(), o_x, o_r, o_AqL.ptr(), w);
+    return solver.Solve(*this, o_x, o_r, tol, maxit, verbose, iterations, steps.get());
+  }
+  if (!permuted) {
+    if (!boxAx) return solver.Solve(*this, o_x, o_r, tol, maxit, verbose, iterations);
+    bp_solve_view_t view(*this);
+    return solver.Solve(view, o_x, o_r, tol, maxit, verbose, iterations);
+  }
+  if (!solver.impl.padded) {  // padding rows must hold zeros
+    if (int st = launch_set<double>(platform->stream, Ns, 0.0, solver.impl.o_p.ptr())) return st;
+    if (int st = launch_set<double>(platform->stream, Ns, 0.0, solver.impl.o_Ap.ptr())) return st;
+    solver.impl.padded = true;
+  }
   if (int st = ToSolve(o_x, o_sx.ptr())) return st;
   if (int st = ToSolve(o_r, o_sr.ptr())) return st;
   bp_solve_view_t view(*this);
@@ -615,7 +807,8 @@ int bp_t::PrepareFused() {
   fused = false;
   permuted = false;
   Ns = ogs.Ngather;
-  if (bp != 5 || Nfields != 1 || mesh->elementType != ELEM_HEX) return BPX_OK;
+  // affine elements: the box iteration on the reference rows instead
+  if (bp != 5 || mesh->elementType != ELEM_HEX || (boxAx && mesh->opts.affine)) return BPX_OK;
   const dlong Ng = ogs.Ngather, Nel = mesh->Nelements;
   const int Nq = mesh->Nq, Np = mesh->Np;
   const long long NIP = fused_interior_pad(Nq), NSP = fused_surface_pad(Nq);
@@ -672,69 +865,58 @@ int bp_t::PrepareFused() {
   return BPX_OK;
 }
 
-dlong bp_t::FoldRows(int precision) const {
-  if (!(cgFold & (precision == 64 ? 1 : 2)) || !fused || !permuted) return 0;
-  if (precision == 64 ? !tuning.fused64 : !tuning.fused32) return 0;
+dlong bp_t::FoldRows() const {
+  if (!(cgFold & 1) || !fused || !permuted || !tuning.fused64) return 0;
   // the FP64 operator at N = 15 runs on the matrix-core kernel, which keeps
   // the separate update kernel
-  if (precision == 64 && mesh->N == 15 && axEngine != AX_ENGINE_VECTOR) return 0;
+  if (mesh->N == 15 && axEngine != AX_ENGINE_VECTOR) return 0;
   return fusedS0;
 }
 
-template <typename T>
-int bp_t::OperatorDotFused(const T* o_q, T* o_Aq, double* part, int* npart, const CgFold<T>* fold) {
+int bp_t::OperatorDotFused(const double* o_q, double* o_Aq, double* part, int* npart, const CgFold<double>* fold) {
   hipStream_t s = platform->stream;
-  AxArgs<T> a;
+  AxArgs<double> a;
   if (fold) a.fold = *fold;
   a.N = mesh->N;
   a.Nelements = mesh->Nelements;
   a.Nfields = 1;
   a.elementList = o_elementList.ptr();
   a.GlobalToLocal = o_G2Ls.ptr();
-  a.lambda = (T)lambda;
+  a.lambda = lambda;
   a.q = o_q;
   a.ldq = fusedS0;  // the first interior row
-  T* AqL;
-  if constexpr (std::is_same<T, double>::value) {
-    a.affine = haveKappa ? 0 : mesh->opts.affine;
-    a.wJ = (haveKappa && mesh->opts.affine) ? o_wJK.ptr() : o_wJ.ptr();
-    a.ggeo = haveKappa ? o_ggeoK.ptr() : o_ggeo.ptr();
-    a.gllw = o_gllw.ptr();
-    a.D = o_D.ptr();
-    a.engine = axEngine;
-    AqL = o_slots.ptr();
-  } else {
-    if (haveKappa) return set_error(BPX_ERR_UNSUPPORTED, "bp: the FP32 operator has no variable coefficient");
-    if (int st = Prepare32()) return st;
-    a.affine = mesh->opts.affine;
-    a.tri = tri32;
-    a.wJ = o_wJ32.ptr();
-    a.ggeo = o_ggeo32.ptr();
-    a.gllw = o_gllw32.ptr();
-    a.D = o_D32.ptr();
-    AqL = o_slots32.ptr();
-  }
-  a.Aq = AqL;
+  a.affine = haveKappa ? 0 : mesh->opts.affine;
+  a.wJ = (haveKappa && mesh->opts.affine) ? o_wJK.ptr() : o_wJ.ptr();
+  a.ggeo = haveKappa ? o_ggeoK.ptr() : o_ggeo.ptr();
+  a.gllw = o_gllw.ptr();
+  a.D = o_D.ptr();
+  a.engine = axEngine;
+  a.Aq = o_slots.ptr();
   a.evStart = axEvStart;
   a.evStop = axEvStop;
-  if (int st = launch_bp5_fused<T>(s, a, o_Aq, o_partAx.ptr())) return st;
+  if (int st = launch_bp5_fused<double>(s, a, o_Aq, o_partAx.ptr())) return st;
   if (sharedOgs.NrowBlocksT > 0) {
     *npart = ogs_gather_partials(sharedOgs.NrowBlocksT);
-    return launch_ogs_gather_dot_fold<T>(s, sharedOgs.NrowBlocksT, sharedOgs.o_blockRowStartsT.ptr(),
-                                         sharedOgs.o_rowStartsT.ptr(), sharedOgs.o_colIdsT.ptr(), AqL, o_Aq, o_q,
-                                         part, o_partAx.ptr(), naxParts, ogs.gatherMode);
+    return launch_ogs_gather_dot_fold<double>(s, sharedOgs.NrowBlocksT, sharedOgs.o_blockRowStartsT.ptr(),
+                                              sharedOgs.o_rowStartsT.ptr(), sharedOgs.o_colIdsT.ptr(), a.Aq, o_Aq,
+                                              o_q, part, o_partAx.ptr(), naxParts, ogs.gatherMode);
   }
   *npart = 1;  // no shared rows (a single element): the Ax partials are the whole dot
   return launch_fold(s, o_partAx.ptr(), naxParts, part);
 }
 
-template int bp_t::OperatorDotFused<double>(const double*, double*, double*, int*, const CgFold<double>*);
-template int bp_t::OperatorDotFused<float>(const float*, float*, double*, int*, const CgFold<float>*);
-
 int bp_t::AxLocalKrhs(int K, const dfloat* o_q, dfloat* o_AqL, int chunk) {
   if (bp != 5 || mesh->elementType != ELEM_HEX)
     return set_error(BPX_ERR_UNSUPPORTED, "bp: k right-hand sides are implemented for BP5 on hexahedra");
   if (haveKappa) return set_error(BPX_ERR_UNSUPPORTED, "bp: k right-hand sides use the constant coefficient");
+  if (chunk == 0 && boxAx) {
+    if (K < 1 || K > 65535) return set_error(BPX_ERR_INVALID_ARGUMENT, "bp: K outside 1..65535");
+    BoxAxArgs<double> b = BoxArgs<double>(o_q, o_AqL);
+    b.K = K;
+    b.ldq = ogs.Ngather;
+    b.ldAq = NLocal;
+    return launch_box_ax<double>(platform->stream, b);
+  }
   AxArgs<double> a;
   a.N = mesh->N;
   a.Nelements = mesh->Nelements;
@@ -818,17 +1000,28 @@ int bp_t::OperatorKrhs(int K, const dfloat* o_q, dfloat* o_Aq, int chunk) {
   return GatherLocal<double>(o_AqLk.ptr(), o_Aq, K);
 }
 
-int bp_t::OperatorDot32(const float* o_q, float* o_Aq, double* part, int* npart, const CgFold<float>* fold) {
+int bp_t::OperatorDot32(const float* o_q, float* o_Aq, double* part, int* npart) {
   if (Nfields != 1) return set_error(BPX_ERR_UNSUPPORTED, "bp: the FP32 operator covers one field (BP1/3/5)");
   if (haveKappa) return set_error(BPX_ERR_UNSUPPORTED, "bp: the FP32 operator has no variable coefficient");
   if (int st = Prepare32()) return st;
-  if (fold && !(fused && tuning.fused32))
-    return set_error(BPX_ERR_INVALID_ARGUMENT, "bp: the folded CG update needs the fused FP32 operator");
-  auto apply = [&]() {
-    return (fused && tuning.fused32) ? OperatorDotFused<float>(o_q, o_Aq, part, npart, fold)
-                                     : OperatorDotUnfused32(o_q, o_Aq, part, npart);
-  };
-  if (!opTimer32 || opTimer32->used + 3 > opTimer32->ev.size()) return apply();
+  if (BoxAx<float>()) {
+    BoxAxArgs<float> a = BoxArgs<float>(o_q, o_AqL32.ptr());
+    a.part = part;
+    *npart = box_ax_partials(box, Nfields);
+    if (int st = launch_box_ax<float>(platform->stream, a)) return st;
+    return GatherLocal<float>(o_AqL32.ptr(), o_Aq);
+  }
+  if (int st = ax<float>(o_q, o_AqL32.ptr(), o_wJ32.ptr(), o_ggeo32.ptr(), o_gllw32.ptr(), o_D32.ptr(),
+                         o_I32.ptr(), o_MM32.ptr(), o_invV32.ptr()))
+    return st;
+  *npart = ogs_gather_partials(ogs.NrowBlocksT);
+  return launch_ogs_gather_dot<float>(platform->stream, ogs.NrowBlocksT, ogs.o_blockRowStartsT.ptr(),
+                                      ogs.o_rowStartsT.ptr(), ogs.o_colIdsT.ptr(), o_AqL32.ptr(), o_Aq, o_q, part,
+                                      ogs.gatherMode);
+}
+
+int bp_t::TimedStep32(const std::function<int()>& step) {
+  if (!opTimer32 || opTimer32->used + 3 > opTimer32->ev.size()) return step();
   hipEvent_t* e = &opTimer32->ev[opTimer32->used];
   opTimer32->used += 3;
   int st;
@@ -839,7 +1032,7 @@ int bp_t::OperatorDot32(const float* o_q, float* o_Aq, double* part, int* npart,
     } clear{axEvStart, axEvStop};
     axEvStart = e[0];  // stamped by the Ax dispatch itself
     axEvStop = e[1];
-    st = apply();
+    st = step();
   }
   if (st) return st;
   BPX_HIP(hipEventRecord(e[2], platform->stream));
@@ -890,17 +1083,6 @@ int bp_t::TimeOperatorInSolve(dfloat* o_x, const dfloat* o_b, double tol, int in
   return BPX_OK;
 }
 
-int bp_t::OperatorDotUnfused32(const float* o_q, float* o_Aq, double* part, int* npart) {
-  if (int st = ax<float>(o_q, o_AqL32.ptr(), o_wJ32.ptr(), o_ggeo32.ptr(), o_gllw32.ptr(), o_D32.ptr(),
-                         o_I32.ptr(), o_MM32.ptr(), o_invV32.ptr(), SolveG2L()))
-    return st;
-  const ogs::ogs_t& G = SolveOgs();
-  *npart = ogs_gather_partials(G.NrowBlocksT);
-  return launch_ogs_gather_dot<float>(platform->stream, G.NrowBlocksT, G.o_blockRowStartsT.ptr(),
-                                      G.o_rowStartsT.ptr(), G.o_colIdsT.ptr(), o_AqL32.ptr(), o_Aq, o_q, part,
-                                      ogs.gatherMode);
-}
-
 namespace {
 // best of three event-timed runs after one untimed run, in microseconds
 template <typename F>
@@ -934,10 +1116,57 @@ int time_best(hipStream_t s, F&& fn, double& us) {
 }
 }  // namespace
 
+// One CG iteration of a box operator in two kernels (choice 1) against four
+// (0), on vectors of ones with the scalars of a running solve.
+template <typename T>
+int bp_t::TuneBox(int& choice, double& fused_us, double& unfused_us) {
+  if (ogs.Ngather == 0) return BPX_OK;
+  hipStream_t s = platform->stream;
+  const size_t n = (size_t)ogs.Ngather;
+  constexpr int kIt = 1;  // the iteration queued: x and r are updated, nothing stops
+  const int nrr = std::max(kRedBlocks, kBoxRrParts);
+  deviceBuffer<T> v;
+  deviceBuffer<double> d;
+  deviceBuffer<CgState> state;
+  if (int st = v.alloc(4 * n)) return st;
+  if (int st = d.alloc((size_t)nrr + GatherPartials() + 4)) return st;
+  if (int st = state.alloc(1)) return st;
+  if (int st = launch_set<T>(s, (dlong)(4 * n), T(1), v.ptr())) return st;
+  if (int st = launch_set<double>(s, (dlong)d.length(), 1.0, d.ptr())) return st;
+  const CgState running = {0.0, 0, 0, 0, 0, 0};
+  BPX_HIP(hipMemcpyAsync(state.ptr(), &running, sizeof(running), hipMemcpyHostToDevice, s));
+  CgWork<T> w;
+  w.state = state.ptr();
+  w.part_rr = d.ptr();
+  w.part_pAp = d.ptr() + nrr;
+  w.hist_rr = w.part_pAp + GatherPartials();
+  w.hist_alpha = w.hist_rr + 2;
+  const int chosen = choice, folds = cgFold;
+  cgFold = 3;
+  T* AqL;
+  if constexpr (sizeof(T) == 8)
+    AqL = o_AqL.ptr();
+  else
+    AqL = o_AqL32.ptr();
+  int st = BPX_OK;
+  for (int form = 1; form >= 0 && st == BPX_OK; --form) {
+    choice = form;
+    const auto steps = BoxSteps<T>(v.ptr(), v.ptr() + n, v.ptr() + 2 * n, v.ptr() + 3 * n, AqL, w);
+    st = time_best(s, [&] { return steps->iterate(kIt, 0.0, true); }, form ? fused_us : unfused_us);
+  }
+  cgFold = folds;
+  choice = st == BPX_OK ? (fused_us < unfused_us ? 1 : 0) : chosen;
+  if (st) return st;
+  BPX_HIP(hipStreamSynchronize(s));
+  return BPX_OK;
+}
+
 int bp_t::Tune() {
   hipStream_t s = platform->stream;
   const dlong Ng = ogs.Ngather;
   if (Ng == 0 || ogs.NrowBlocksT == 0) return BPX_OK;
+  if (boxAx && mesh->opts.affine)
+    return bp == 5 ? TuneBox<double>(tuning.fused64, tuning.fused_us, tuning.unfused_us) : BPX_OK;
   deviceBuffer<double> v, part;
   if (int st = v.alloc(2 * (size_t)Ng)) return st;
   if (int st = part.alloc(GatherPartials())) return st;
@@ -961,8 +1190,7 @@ int bp_t::Tune() {
   if (int st = w.alloc(2 * (size_t)Ns)) return st;
   BPX_HIP(hipMemsetAsync(w.ptr(), 0, 2 * (size_t)Ns * sizeof(double), s));
   int np = 0;
-  if (int st = time_best(s, [&] { return OperatorDotFused<double>(w.ptr(), w.ptr() + Ns, part.ptr(), &np); },
-                         tuning.fused_us))
+  if (int st = time_best(s, [&] { return OperatorDotFused(w.ptr(), w.ptr() + Ns, part.ptr(), &np); }, tuning.fused_us))
     return st;
   if (int st = time_best(s, [&] { return OperatorDotUnfusedS(w.ptr(), w.ptr() + Ns, part.ptr(), &np); },
                          tuning.unfused_us))
@@ -973,23 +1201,8 @@ int bp_t::Tune() {
 
 // The same choice for the FP32 operator, timed when it is first built
 int bp_t::Tune32() {
-  if (!fused) return BPX_OK;
-  hipStream_t s = platform->stream;
-  if (Ns == 0) return BPX_OK;
-  deviceBuffer<float> v;
-  deviceBuffer<double> part;
-  if (int st = v.alloc(2 * (size_t)Ns)) return st;
-  if (int st = part.alloc(GatherPartials())) return st;
-  BPX_HIP(hipMemsetAsync(v.ptr(), 0, 2 * (size_t)Ns * sizeof(float), s));
-  int np = 0;
-  if (int st = time_best(s, [&] { return OperatorDotFused<float>(v.ptr(), v.ptr() + Ns, part.ptr(), &np); },
-                         tuning.fused32_us))
-    return st;
-  if (int st = time_best(s, [&] { return OperatorDotUnfused32(v.ptr(), v.ptr() + Ns, part.ptr(), &np); },
-                         tuning.unfused32_us))
-    return st;
-  tuning.fused32 = tuning.fused32_us < tuning.unfused32_us ? 1 : 0;
-  return BPX_OK;
+  if (!BoxAx<float>()) return BPX_OK;
+  return TuneBox<float>(tuning.fused32, tuning.fused32_us, tuning.unfused32_us);
 }
 
 // The CG operator as the solvers apply it (solve space, tuned form), timed
@@ -1001,7 +1214,7 @@ int bp_t::TimeOperator(int precision, int launches, double* out) {
   if (precision == 32)
     if (int st = Prepare32()) return st;
   hipStream_t s = platform->stream;
-  const size_t n = (size_t)std::max<dlong>(Ns, 1);
+  const size_t n = (size_t)std::max<dlong>(std::max(Ns, ogs.Ngather), 1);
   deviceBuffer<double> v64, part;
   deviceBuffer<float> v32;
   if (int st = part.alloc(std::max(GatherPartials(), 1))) return st;
@@ -1014,8 +1227,10 @@ int bp_t::TimeOperator(int precision, int launches, double* out) {
   }
   auto run = [&]() -> int {
     int np = 0;
-    return precision == 64 ? OperatorDotS(v64.ptr(), v64.ptr() + n, part.ptr(), &np)
-                           : OperatorDot32(v32.ptr(), v32.ptr() + n, part.ptr(), &np);
+    if (precision == 64)
+      return boxAx ? OperatorDot(v64.ptr(), v64.ptr() + n, part.ptr(), &np)
+                   : OperatorDotS(v64.ptr(), v64.ptr() + n, part.ptr(), &np);
+    return OperatorDot32(v32.ptr(), v32.ptr() + n, part.ptr(), &np);
   };
   for (int w = 0; w < 3; ++w)
     if (int st = run()) return st;
@@ -1072,21 +1287,21 @@ int bp_t::Prepare32() {
   const int affine = m.opts.affine;
   int st = BPX_OK;
   tri32 = 0;
-  if (bp == 5 && !affine && fp32Geometry == 0 && mesh->NodesTrilinear()) {
+  if (bp == 5) {
+    std::vector<double> eo;
+    if ((st = box_even_odd_table(m, eo)) || (st = cvt(o_boxEo32, eo))) return st;
+  }
+  if (bp == 5 && !affine && fp32Geometry == 0) {
     // the FP32 operator forms its geometric factors from the elements'
     // trilinear maps: 96 B per element instead of 28 B per node
     std::vector<double> tri;
     m.TrilinearCoefficients(tri);
-    if ((st = cvt(o_wJ32, m.gllz)) || (st = cvt(o_ggeo32, tri)) || (st = cvt(o_gllw32, m.gllw)) ||
-        (st = cvt(o_D32, m.D)))
-      return st;
+    if ((st = cvt(o_wJ32, m.gllz)) || (st = cvt(o_ggeo32, tri)) || (st = cvt(o_gllw32, m.gllw))) return st;
     tri32 = 1;
   } else if ((st = mesh->EnsureHost())) {
     return st;
-  } else if (bp == 5 || bp == 6) {
-    if ((st = cvt(o_wJ32, m.wJ)) || (st = cvt(o_ggeo32, m.ggeo)) || (st = cvt(o_gllw32, m.gllw)) ||
-        (st = cvt(o_D32, m.D)))
-      return st;
+  } else if (bp == 5) {
+    if ((st = cvt(o_wJ32, m.wJ)) || (st = cvt(o_ggeo32, m.ggeo)) || (st = cvt(o_gllw32, m.gllw))) return st;
   } else if (bp == 1 || bp == 2) {
     if ((st = cvt(o_wJ32, affine ? m.wJ : m.cubwJ)) || (st = cvt(o_I32, m.cubInterp)) || (st = cvt(o_MM32, m.MM)))
       return st;
@@ -1101,7 +1316,6 @@ int bp_t::Prepare32() {
     if (!eo.empty() && (st = cvt(o_eo32, eo))) return st;
   }
   if ((st = o_AqL32.alloc(NLocal))) return st;
-  if (fused && (st = o_slots32.alloc(o_slots.length()))) return st;
   if ((st = platform->finish())) return st;
   have32 = true;
   if ((st = Tune32())) return st;
@@ -1122,9 +1336,11 @@ int bp_t::Operator32(const float* o_q, float* o_Aq) {
   if (Nfields != 1) return set_error(BPX_ERR_UNSUPPORTED, "bp: the FP32 operator covers one field (BP1/3/5)");
   if (haveKappa) return set_error(BPX_ERR_UNSUPPORTED, "bp: the FP32 operator has no variable coefficient");
   if (int st = Prepare32()) return st;
-  if (int st = ax<float>(o_q, o_AqL32.ptr(), o_wJ32.ptr(), o_ggeo32.ptr(), o_gllw32.ptr(), o_D32.ptr(),
-                         o_I32.ptr(), o_MM32.ptr(), o_invV32.ptr()))
-    return st;
+  const int st = BoxAx<float>()
+                     ? launch_box_ax<float>(platform->stream, BoxArgs<float>(o_q, o_AqL32.ptr()))
+                     : ax<float>(o_q, o_AqL32.ptr(), o_wJ32.ptr(), o_ggeo32.ptr(), o_gllw32.ptr(), o_D32.ptr(),
+                                 o_I32.ptr(), o_MM32.ptr(), o_invV32.ptr());
+  if (st) return st;
   return GatherLocal<float>(o_AqL32.ptr(), o_Aq);
 }
 

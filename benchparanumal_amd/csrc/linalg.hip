@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "bpx_internal.hpp"
+#include "fold.hpp"
 
 namespace bpx {
 namespace {
@@ -54,29 +55,6 @@ __device__ inline double block_allsum(double v, double* s_w) {
   }
   __syncthreads();
   return s_w[32];
-}
-
-// Sum of partials[0..n) in a fixed order, by one wavefront: lane l folds
-// l, l+64, ... into four accumulators (so its loads are in flight
-// together), then an xor butterfly (each step adds the same two operands on
-// both lanes of a pair, so every lane ends with the same bits). Every
-// wavefront that folds the same partials gets the same value, whatever
-// kernel or workgroup size it runs in.
-__device__ inline double wave_fold(const double* __restrict__ part, int n) {
-  const int lane = threadIdx.x & 63;
-  double a0 = 0, a1 = 0, a2 = 0, a3 = 0;
-  int i = lane;
-  for (; i + 192 < n; i += 256) {
-    a0 += part[i];
-    a1 += part[i + 64];
-    a2 += part[i + 128];
-    a3 += part[i + 192];
-  }
-  for (; i < n; i += 64) a0 += part[i];
-  double v = (a0 + a1) + (a2 + a3);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
 }
 
 // wave_fold by wavefront 0, broadcast to the workgroup through LDS

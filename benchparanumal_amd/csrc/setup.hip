@@ -255,31 +255,6 @@ __global__ void k_masked_ids(dlong Nel, int Nq, int Nfields, long long LX, long 
     ids[(size_t)e * Np * Nfields + (size_t)f * Np + n] = boundary ? 0 : (g + 1) * Nfields + f;
 }
 
-// bad = 1 where a node is off its element's trilinear map by more than tol
-// (c: 24 coefficients per element, as mesh_t::TrilinearCoefficients)
-__global__ void k_check_trilinear(dlong Nel, int Nq, double tol, const double* __restrict__ gllz,
-                                  const double* __restrict__ c, const double* __restrict__ EX,
-                                  const double* __restrict__ EY, const double* __restrict__ EZ,
-                                  const double* __restrict__ x, const double* __restrict__ y,
-                                  const double* __restrict__ z, int* __restrict__ bad) {
-  const int Np = Nq * Nq * Nq;
-  const size_t id = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (id >= (size_t)Nel * Np) return;
-  const dlong e = (dlong)(id / Np);
-  const int n = (int)(id - (size_t)e * Np);
-  const double r = gllz[n % Nq], s = gllz[(n / Nq) % Nq], t = gllz[n / (Nq * Nq)];
-  const double* V[3] = {EX + (size_t)e * 8, EY + (size_t)e * 8, EZ + (size_t)e * 8};
-  const double* X[3] = {x, y, z};
-  for (int d = 0; d < 3; ++d) {
-    const double* cd = c + (size_t)e * 24 + 8 * d;
-    double c0 = 0;
-    for (int v = 0; v < 8; ++v) c0 += 0.125 * V[d][v];
-    const double m = c0 + cd[0] * r + cd[1] * s + cd[2] * t + cd[3] * r * s + cd[4] * r * t + cd[5] * s * t +
-                     cd[6] * r * s * t;
-    if (fabs(m - X[d][id]) > tol) *bad = 1;
-  }
-}
-
 // -------------------------------------------------------------- ogs -----
 
 __global__ void k_ogs_keys(dlong N, const hlong* __restrict__ ids, unsigned long long* __restrict__ key,
@@ -506,28 +481,6 @@ int mesh_t::EnsureHost() {
   if (int st = o_cubwJ.download(cubwJ, s)) return st;
   if (int st = o_cubggeo.download(cubggeo, s)) return st;
   return o_globalIds.download(globalIds, s);
-}
-
-bool mesh_t::NodesTrilinear() {
-  if (!onDevice) return NodesAreTrilinear();
-  if (hipSetDevice(devPlatform->device) != hipSuccess) return false;
-  hipStream_t s = devPlatform->stream;
-  std::vector<double> c;
-  TrilinearCoefficients(c);
-  deviceBuffer<double> dc, dEX, dEY, dEZ, dz;
-  deviceBuffer<int> bad;
-  if (dc.upload(c, s) || dEX.upload(EX, s) || dEY.upload(EY, s) || dEZ.upload(EZ, s) || dz.upload(gllz, s) ||
-      bad.alloc(1) || fill(s, 1, 0, bad.ptr()))
-    return false;
-  const double scale = std::max(opts.dim[0], std::max(opts.dim[1], opts.dim[2]));
-  const size_t NL = (size_t)Nelements * Np;
-  if (NL > 0)
-    hipLaunchKernelGGL(k_check_trilinear, dim3(blocks_for(NL)), dim3(kT), 0, s, Nelements, Nq, 1e-12 * scale,
-                       dz.ptr(), dc.ptr(), dEX.ptr(), dEY.ptr(), dEZ.ptr(), o_x.ptr(), o_y.ptr(), o_z.ptr(),
-                       bad.ptr());
-  int hbad = 1;
-  if (hipGetLastError() != hipSuccess || read_value(s, bad.ptr(), hbad)) return false;
-  return hbad == 0;
 }
 
 int mesh_t::MaskedGlobalIdsDevice(int Nfields, hlong* o_ids) const {
@@ -839,7 +792,8 @@ int bp_t::PrepareFusedDevice() {
   fused = false;
   permuted = false;
   Ns = ogs.Ngather;
-  if (bp != 5 || Nfields != 1) return BPX_OK;
+  // affine elements: the box iteration on the reference rows instead
+  if (bp != 5 || (boxAx && mesh->opts.affine)) return BPX_OK;
   hipStream_t s = platform->stream;
   const dlong Ng = ogs.Ngather, Nel = mesh->Nelements;
   const int Nq = mesh->Nq;

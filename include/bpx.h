@@ -358,10 +358,11 @@ int bpx_bp_info(bpx_bp b, int64_t* out, int capacity);
  * order 0, of order 1; out[3..5]: FP64 CG operator fused (1: the Ax writes
  * single-copy rows, the gather sums the shared rows) or unfused (0: Ax,
  * then the full gather; -1 = no fused form for this problem), time fused,
- * time unfused; out[6..8]: the same for the FP32 operator (timed when it is
- * first used); out[9]: 1 if the FP32 operator forms its geometric factors
- * from the elements' trilinear maps, 0 if it reads stored factors rounded
- * to FP32, -1 if it has not been built yet. Returns the number of values. */
+ * time unfused (affine elements: a CG iteration in two kernels or in four);
+ * out[6..8]: the same for the FP32 operator (timed when it is first used);
+ * out[9]: 1 if the FP32 operator forms its geometric factors from the
+ * elements' trilinear maps, 0 if it reads stored factors rounded to FP32,
+ * -1 if it has not been built yet. Returns the number of values. */
 int bpx_bp_tuning(bpx_bp b, double* out, int capacity);
 /* No reference counterpart: copy one of the problem's device arrays to host
  * memory dst (NULL: query *count). Names: rowStartsT colIdsT blockRowStartsT
@@ -378,12 +379,10 @@ int bpx_bp_array(bpx_bp b, const char* name, void* dst, int64_t* count, int* dty
 int bpx_bp_set_tuning(bpx_bp b, int gatherMode, int fused, int fused32);
 /* No reference counterpart: the geometry of the FP32 BP5 operator (the
  * inner operator of bpx_bp_solve_mixed). mode 0 (default): formed in the
- * kernel from each element's trilinear map when every node of the mesh is
- * its element's trilinear map of the 8 vertices (checked on the host; the
- * box meshes of bpx_mesh_create are), else stored factors; mode 1: the FP64
- * geometric factors rounded to FP32 and streamed (the operator of the
- * reference's kernels with dfloat = float). Other operators always use
- * stored factors. The FP32 operator is rebuilt on its next use. */
+ * kernel from each element's trilinear map of its 8 vertices (what the box
+ * meshes of bpx_mesh_create are); mode 1: the FP64 geometric factors
+ * rounded to FP32 and streamed (the operator of the reference's kernels
+ * with dfloat = float). The FP32 operator is rebuilt on its next use. */
 int bpx_bp_set_fp32_geometry(bpx_bp b, int mode);
 /* No reference counterpart: where the BP5 Ax at N = 15 in FP64 (one field)
  * runs its r and s contractions: 0 = auto (the matrix cores; default), 1 =
@@ -400,13 +399,11 @@ int bpx_bp_set_ax_engine(bpx_bp b, int engine);
  * agree to rounding, not bit for bit. Other problems have one kernel. */
 int bpx_bp_set_cub_form(bpx_bp b, int form);
 /* No reference counterpart (launch choice, same results): mask = 1 (FP64
- * solves), 2 (the FP32 iterations of the mixed solve) or 3 (both): those CG
- * solves that use the fused BP5 operator do the direction update of the
- * elements' interior rows (x += alpha p, p = r + beta p) inside that
- * operator's Ax, and the separate update kernel covers the shared rows
- * only; elsewhere (mask 0: everywhere) one update kernel covers all rows.
- * Default 1: at 24^3, p = 7 the fold saves 2% of an FP64 iteration and
- * costs 2% of an FP32 one, whose Ax is bound by instruction issue. */
+ * solves), 2 (the FP32 iterations of the mixed solve) or 3 (both, the
+ * default): those CG solves do the direction update (x += alpha p, p = r +
+ * beta p) inside the operator's Ax (with the stored factors: the elements'
+ * interior rows; the separate update kernel then covers the shared rows
+ * only); elsewhere (mask 0: everywhere) one update kernel covers all rows. */
 int bpx_bp_set_cg_fold(bpx_bp b, int mask);
 /* No reference counterpart (measurement): the CG operator as the solvers
  * apply it (their row order, the tuned fused or unfused form) in FP64
@@ -426,12 +423,13 @@ int bpx_bp_time_operator(bpx_bp b, int precision, int launches, double* out);
  * us. Synchronises. */
 int bpx_bp_time_krhs(bpx_bp b, int K, int chunk, int launches, const double* o_q, double* out);
 /* bpN_t::Operator(o_q, o_Aq) (BP/BP5/src/bp5Operator.cpp:29-85): Ax over the
- * local elements, then the T gather. Device vectors of length Ngather. */
+ * local elements, then the T gather. Device vectors of length Ngather. BP5
+ * (N <= 14) and BP6 on hexahedra form the geometric factors in the kernel
+ * from the elements' trilinear maps (the stored factors' values to their
+ * rounding, and closer to the exact ones). */
 int bpx_bp_operator(bpx_bp b, const double* o_q, double* o_Aq);
 /* The operator as CG applies it: cg::Solve's Operator followed by
- * innerProd(p, Ap) (libs/core/linearSolverCG.cpp:99-106) in one pass. For
- * BP5 the Ax kernel writes nodes that are the only copy of their global row
- * straight into o_Aq and the gather sums only the shared rows; o_Aq equals
+ * innerProd(p, Ap) (libs/core/linearSolverCG.cpp:99-106); o_Aq equals
  * bpx_bp_operator's bit for bit. *qAq (host) = q.Aq. Synchronises. */
 int bpx_bp_operator_dot(bpx_bp b, const double* o_q, double* o_Aq, double* qAq);
 /* Ax alone into the local vector (BK/BK5/src/bk5Run.cpp:59-71). */
@@ -481,7 +479,10 @@ int bpx_bp_rhs_forcing(bpx_bp b, double* o_b);
  * scalars: no host wait inside an iteration. o_r holds b on entry and the
  * residual on exit; o_x the initial guess / solution. rnorm_hist (host,
  * may be NULL) gets maxit+1 residual norms (entry 0 = initial). Returns
- * BPX_OK and *iterations. */
+ * BPX_OK and *iterations. BP5 and BP6 on hexahedra: solves to a tolerance
+ * apply the operator of bpx_bp_operator; a fixed number of iterations (tol =
+ * 0, constant coefficient, not affine) applies the reference's stored
+ * factors, whose residual history it reproduces. */
 int bpx_bp_solve(bpx_bp b, double* o_x, double* o_r, double tol, int maxit, int verbose,
                  int* iterations, double* rnorm_hist);
 /* No reference counterpart: CG in FP32 (FP32 operator and vectors, FP64

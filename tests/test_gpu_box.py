@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 import torch
 
+import oracle_lib
 from benchparanumal_amd import capi
 
 pytestmark = pytest.mark.gpu
@@ -58,3 +59,104 @@ def test_box_gather_of_several_vectors(plat, N, K):
     for r in range(K):
         b.operator_krhs(q[r * b.Ngather:].contiguous(), one, 1)
         np.testing.assert_array_equal(host(Aq[r * b.Ngather:(r + 1) * b.Ngather]), host(one))
+
+
+# ---------------------------------------------------------- box_ax.hip ----
+def pair(bp, N, nx, ny, nz, affine=False, lam=1.3):
+    kw = dict(N=N, nx=nx, ny=ny, nz=nz, affine=affine, perturb=0.0 if affine else 0.1, seed=7)
+    return capi.Mesh(**kw), oracle_lib.Problem(bp=bp, lam=lam, **kw)
+
+
+def rel_err(got, ref):
+    return float(np.abs(got - ref).max() / max(np.abs(ref).max(), 1e-300))
+
+
+@pytest.mark.parametrize("affine", [False, True])
+@pytest.mark.parametrize("bp,N", [(bp, N) for bp in (5, 6) for N in range(1, 16)])
+def test_box_operator_matches_oracle(plat, bp, N, affine):
+    """BP5 and BP6 at every degree on a box whose element count leaves the
+    last workgroup partly empty, against the oracle: the FP64 bar (the
+    oracle's factors come from its own D, the kernel's from the exact map),
+    and q.Aq of the CG form."""
+    m, P = pair(bp, N, 3, 2, 3 if N < 10 else 1, affine=affine)
+    b = capi.BP(plat, m, bp, lam=1.3)
+    q = np.random.default_rng(N).standard_normal(b.Ngather)
+    A, A2 = torch.full((2, b.Ngather), float("nan"), dtype=torch.float64, device="cuda")
+    b.operator(torch.from_numpy(q).cuda(), A)
+    ref = P.operator(q)
+    assert rel_err(host(A), ref) <= 1e-12
+    qAq = b.operator_dot(torch.from_numpy(q).cuda(), A2)
+    np.testing.assert_array_equal(host(A2), host(A))
+    assert abs(qAq - float(np.dot(q, host(A)))) <= 1e-13 * np.abs(q * host(A)).sum()
+
+
+@pytest.mark.parametrize("geometry", [0, 1])
+@pytest.mark.parametrize("N,affine", [(N, False) for N in range(1, 16)] + [(2, True), (7, True), (11, True)])
+def test_box_operator_f32(plat, N, affine, geometry):
+    """FP32: trilinear, stored and affine factors against the FP64 oracle."""
+    m, P = pair(5, N, 3, 2, 2, affine=affine)
+    b = capi.BP(plat, m, 5, lam=1.3)
+    b.set_fp32_geometry(geometry)
+    q = np.random.default_rng(N).standard_normal(b.Ngather)
+    A = torch.full((b.Ngather,), float("nan"), dtype=torch.float32, device="cuda")
+    b.operator_f32(torch.from_numpy(q).cuda().float(), A)
+    assert rel_err(host(A).astype(np.float64), P.operator(q)) <= 2e-5
+
+
+@pytest.mark.parametrize("bp,N,nx,ny,nz,affine", [(5, 1, 4, 4, 3, False), (5, 4, 5, 3, 2, False), (5, 7, 3, 3, 2, False),
+                                                  (5, 7, 3, 2, 2, True), (5, 9, 2, 3, 2, False), (5, 12, 2, 2, 2, False),
+                                                  (6, 3, 3, 3, 2, False), (6, 7, 2, 2, 3, True), (5, 2, 1, 1, 1, False)])
+def test_box_cg_forms(plat, bp, N, nx, ny, nz, affine):
+    """CG to a tolerance on the box: the direction update inside the Ax or in
+    its own kernel (the same bits), and four kernels per iteration (the r.r
+    sums in another order); the true residual reaches the tolerance, and the
+    solution agrees with the oracle's to the tolerance times the condition
+    number's reach (100)."""
+    m, P = pair(bp, N, nx, ny, nz, affine=affine, lam=1.0)
+    b = capi.BP(plat, m, bp, lam=1.0)
+    rhs = capi.random_normal(5, b.Ngather)
+    x_ref, it_ref, _, _ = P.cg(rhs, 5000, tol=1e-12)
+    sols = []
+    for fold, fused in ((3, 1), (0, 1), (0, 0)):
+        b.set_cg_fold(fold)
+        if bp == 5:
+            b.set_tuning(fused=fused)
+        x = torch.zeros(b.Ngather, dtype=torch.float64, device="cuda")
+        its, hist = b.solve(x, torch.from_numpy(rhs).cuda(), tol=1e-10, maxit=5000)
+        Ax = torch.zeros_like(x)
+        b.operator(x, Ax)
+        assert np.linalg.norm(rhs - host(Ax)) <= 2e-10 * max(np.linalg.norm(rhs), 1.0)
+        assert np.linalg.norm(host(x) - x_ref) <= 1e-8 * np.linalg.norm(x_ref)
+        sols.append((its, hist, host(x)))
+    assert sols[0][0] == sols[1][0] and abs(sols[2][0] - sols[0][0]) <= 1
+    np.testing.assert_array_equal(sols[0][1], sols[1][1])
+    np.testing.assert_array_equal(sols[0][2], sols[1][2])
+
+
+def test_fixed_count_after_tolerance_solve(plat):
+    """A fixed number of iterations (stored factors, the solve space's padded
+    rows) gives the same bits before and after a solve to a tolerance, which
+    uses the same work vectors for reference rows."""
+    b = capi.BP(plat, capi.Mesh(N=5, nx=4, ny=3, nz=3, perturb=0.1, seed=7), 5, lam=1.0)
+    rhs = capi.random_normal(5, b.Ngather)
+    out = []
+    for tol, maxit in ((0.0, 30), (1e-10, 3000), (0.0, 30)):
+        x = torch.zeros(b.Ngather, dtype=torch.float64, device="cuda")
+        _, hist = b.solve(x, torch.from_numpy(rhs).cuda(), tol=tol, maxit=maxit)
+        out.append((hist, host(x)))
+    np.testing.assert_array_equal(out[0][0], out[2][0])
+    np.testing.assert_array_equal(out[0][1], out[2][1])
+
+
+@pytest.mark.parametrize("N,affine", [(1, False), (2, True), (4, False), (8, False), (12, True), (14, False)])
+def test_box_kappa_operator(plat, N, affine):
+    """The variable coefficient read from the lattice, against the oracle."""
+    m, P = pair(5, N, 3, 2, 2, affine=affine, lam=0.4)
+    b = capi.BP(plat, m, 5, lam=0.4)
+    kap = np.exp(0.3 * np.random.default_rng(N).standard_normal(b.Nnodes))
+    b.set_kappa(torch.from_numpy(kap).cuda())
+    P.set_kappa(kap)
+    q = np.random.default_rng(N + 1).standard_normal(b.Ngather)
+    A = torch.full((b.Ngather,), float("nan"), dtype=torch.float64, device="cuda")
+    b.operator(torch.from_numpy(q).cuda(), A)
+    assert rel_err(host(A), P.operator(q)) <= 1e-12
