@@ -71,13 +71,6 @@ constexpr int bp5_waves_v() {
   return bp5_waves<NQ, NF, VAR == 1>();
 }
 
-// occupancy target of the FP32 kernels with the trilinear geometry (the
-// plain one at Nq = 8 spills at 7 and at 5 waves; 4 hold it)
-template <int NQ, int VAR>
-constexpr int bp5_waves_tri() {
-  return (VAR == 0 && NQ == 8) ? 4 : bp5_waves_v<float, NQ, 1, VAR>();
-}
-
 // D rows/columns in registers (saves 4*Nq LDS reads per node) for one
 // field per sweep in FP64 up to Nq = 8; with several fields the registers
 // hold the extra pencils. Measured at 24^3, p=7: the FP64 plain Ax is
@@ -152,16 +145,6 @@ __device__ inline T geo_load(const T* p) {
   return *p;
 }
 
-// TRI (FP32, one field, non-affine; plain or fused): the geometric factors
-// are computed in the kernel from the element's trilinear map instead of
-// read from memory. ggeo then holds 24 values per element, for x, y and z
-// in turn the coefficients of r, s, t, rs, rt, st, rst of
-// x(r,s,t) = sum_v (1+r_v r)(1+s_v s)(1+t_v t) X_v / 8 and one pad, and wJ
-// holds the Nq GLL nodes. Lane (i,j) keeps the derivatives' pencil
-// constants (x_r and x_s are linear in t along the pencil, x_t is
-// constant); each node then forms the adjugate of the Jacobian, J and
-// G = adj adj^T w / J (the formula of the stored factors), ~55 VALU
-// operations in place of 28 B of HBM traffic per node.
 // FOLD (FUSED only): the CG direction update of the element's interior rows
 // (rows >= S0 = ldq, each the only copy of its row) is done here, as
 // k_cg_update_p does it for the rows below S0: x <- alpha_{k-1} p + x and
@@ -169,7 +152,7 @@ __device__ inline T geo_load(const T* p) {
 // solve gives the bits it gives with the update in its own kernel. q is
 // then the direction p itself (fold.p, updated in place: no other lane
 // reads an interior row).
-template <typename T, int NQ, int NF, int EPB, bool AFFINE, int WAVES, int VAR, bool TRI = false, bool FOLD = false,
+template <typename T, int NQ, int NF, int EPB, bool AFFINE, int WAVES, int VAR, bool FOLD = false,
           int FS = 1>
 __global__ __launch_bounds__(NQ* NQ* EPB) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_bp5_ax(
     int Nelements, int K, const int* __restrict__ elementList, const int* __restrict__ G2L,
@@ -182,28 +165,12 @@ __global__ __launch_bounds__(NQ* NQ* EPB) __attribute__((amdgpu_waves_per_eu(WAV
   constexpr bool FUSED = VAR == VAR_FUSED;
   static_assert(!FUSED || NF == 1, "the fused operator covers one field");
   static_assert(!FOLD || FUSED, "the folded direction update is a form of the fused operator");
-  static_assert(!TRI || (sizeof(T) == 4 && NF == 1 && !AFFINE && (VAR == VAR_PLAIN || FUSED)),
-                "TRI: FP32, one field, non-affine");
-  static_assert(FS == 1 || (NF == 1 && EPB == 1 && VAR == VAR_PLAIN && !TRI),
+  static_assert(FS == 1 || (NF == 1 && EPB == 1 && VAR == VAR_PLAIN),
                 "field split: the plain one-field sweep, one element per workgroup");
   constexpr int NQ2 = NQ * NQ;
   constexpr int NP = NQ2 * NQ;
   constexpr int LD = NQ + 1;  // padded LDS row
-  // TRI moves ~77 MB per launch at 24^3, p = 7 instead of ~274 MB, and
-  // the LDS reads become the bound: D rows/columns in registers and the
-  // broadcast D[k][m] from scalar (constant address space) loads
-  // (measured Ax 44.1 -> 38.2 -> 36.5 us, the mixed solve 111.1 -> 101.6 ms).
-  // Both only at Nq = 8 and 16. With D in registers and D[k][m] from LDS
-  // the FP32 operator came out 20-42% off at Nq = 5..15 except 8 (right at
-  // 2, 3, 4): the compiler's IR load/store vectorizer merges the load of
-  // s_D[i][1] with the lane's column load s_D[0][i] as if the two were
-  // adjacent (they are only for i = 0), so lanes i > 0 use a wrong D entry;
-  // the same code built with that pass off is right at every Nq. Those Nq
-  // keep D in LDS, which the pass leaves intact.
-  constexpr bool DREG = (TRI && NQ % 8 == 0) || bp5_dreg<T, NQ, NF, VAR>();
-  constexpr bool SDK = TRI && NQ % 8 == 0;
-  typedef const __attribute__((address_space(4))) T* cptr;
-  const cptr Dc = (cptr)D;
+  constexpr bool DREG = bp5_dreg<T, NQ, NF, VAR>();
 
   __shared__ T s_D[NQ][LD];
   __shared__ T s_q[NF][EPB][NQ][LD];
@@ -335,47 +302,7 @@ __global__ __launch_bounds__(NQ* NQ* EPB) __attribute__((amdgpu_waves_per_eu(WAV
   // geometry of the current slab (non-affine: prefetched one slab ahead)
   T g0 = 0, g1 = 0, g2 = 0, g3 = 0, g4 = 0, g5 = 0, gw = 0;
   T wij = 0;
-  // TRI: along the pencil, x_r = Ar + Br t, x_s = As + Bs t, x_t = Ct, so
-  // the adjugate rows J grad r = x_s x x_t = Pr + Qr t and J grad s =
-  // x_t x x_r = Ps + Qs t are linear in t, J grad t = x_r x x_s = T0 + T1 t
-  // + T2 t^2 is quadratic, and so is J = x_t . (J grad t) = j0 + j1 t + j2 t^2
-  // (14 operations per node instead of 27 for the derivatives, adjugate and J)
-  T Pr[TRI ? 3 : 1], Qr[TRI ? 3 : 1], Ps[TRI ? 3 : 1], Qs[TRI ? 3 : 1];
-  T T0[TRI ? 3 : 1], T1[TRI ? 3 : 1], T2[TRI ? 3 : 1], jt[TRI ? 3 : 1];
-  if (TRI) {
-    const T r = wJ[i], sn = wJ[j];
-    const T* ce = ggeo + (size_t)24 * e;
-    T Ar[3], Br[3], As[3], Bs[3], Ct[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      const T c_r = ce[8 * d + 0], c_s = ce[8 * d + 1], c_t = ce[8 * d + 2], c_rs = ce[8 * d + 3];
-      const T c_rt = ce[8 * d + 4], c_st = ce[8 * d + 5], c_rst = ce[8 * d + 6];
-      Ar[d] = fmad(c_rs, sn, c_r);
-      Br[d] = fmad(c_rst, sn, c_rt);
-      As[d] = fmad(c_rs, r, c_s);
-      Bs[d] = fmad(c_rst, r, c_st);
-      Ct[d] = fmad(Br[d], r, fmad(c_st, sn, c_t));
-    }
-    // (a x b)_d = a_{d+1} b_{d+2} - a_{d+2} b_{d+1}
-    auto cross = [](const T* a, const T* b, int d) {
-      const int d1 = (d + 1) % 3, d2 = (d + 2) % 3;
-      return fmad(a[d1], b[d2], -(a[d2] * b[d1]));
-    };
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      Pr[d] = cross(As, Ct, d);
-      Qr[d] = cross(Bs, Ct, d);
-      Ps[d] = cross(Ct, Ar, d);
-      Qs[d] = cross(Ct, Br, d);
-      T0[d] = cross(Ar, As, d);
-      T1[d] = cross(Ar, Bs, d) + cross(Br, As, d);
-      T2[d] = cross(Br, Bs, d);
-    }
-    jt[0] = fmad(Ct[0], T0[0], fmad(Ct[1], T0[1], Ct[2] * T0[2]));
-    jt[1] = fmad(Ct[0], T1[0], fmad(Ct[1], T1[1], Ct[2] * T1[2]));
-    jt[2] = fmad(Ct[0], T2[0], fmad(Ct[1], T2[1], Ct[2] * T2[2]));
-    wij = gllw[i] * gllw[j];
-  } else if (AFFINE) {
+  if (AFFINE) {
     const T* ge = ggeo + (size_t)6 * e;
     g0 = ge[0]; g1 = ge[1]; g2 = ge[2]; g3 = ge[3]; g4 = ge[4]; g5 = ge[5];
     gw = wJ[e];
@@ -409,24 +336,7 @@ __global__ __launch_bounds__(NQ* NQ* EPB) __attribute__((amdgpu_waves_per_eu(WAV
       for (int m = 0; m < NQ; ++m) asm volatile("" : "+v"(rA[f][m]));
 
     T G00 = 0, G01 = 0, G02 = 0, G11 = 0, G12 = 0, G22 = 0, W;
-    // TRI: rows of the adjugate (J grad r, J grad s, J grad t) and w/J; G is
-    // applied as adj (w/J) adj^T without forming it (21 operations per node
-    // instead of 24 to form G and 9 to apply it)
-    T arx = 0, ary = 0, arz = 0, asx = 0, asy = 0, asz = 0, atx = 0, aty = 0, atz = 0, sc = 0;
-    if (TRI) {
-      const T tk = wJ[k];
-      arx = fmad(Qr[0], tk, Pr[0]); ary = fmad(Qr[1], tk, Pr[1]); arz = fmad(Qr[2], tk, Pr[2]);
-      asx = fmad(Qs[0], tk, Ps[0]); asy = fmad(Qs[1], tk, Ps[1]); asz = fmad(Qs[2], tk, Ps[2]);
-      atx = fmad(fmad(T2[0], tk, T1[0]), tk, T0[0]);
-      aty = fmad(fmad(T2[1], tk, T1[1]), tk, T0[1]);
-      atz = fmad(fmad(T2[2], tk, T1[2]), tk, T0[2]);
-      const T J = fmad(fmad(jt[2], tk, jt[1]), tk, jt[0]);
-      const T w = wij * gllw[k];
-      // hardware reciprocal (1 ulp) in place of the correctly rounded
-      // division, which takes ~10 instructions (Ax 44.8 -> 44.1 us)
-      sc = w * __builtin_amdgcn_rcpf(J);
-      W = J * w;
-    } else if (AFFINE) {
+    if (AFFINE) {
       const T w = wij * gllw[k];
       G00 = g0 * w; G01 = g1 * w; G02 = g2 * w; G11 = g3 * w; G12 = g4 * w; G22 = g5 * w;
       W = gw * w;
@@ -452,26 +362,16 @@ __global__ __launch_bounds__(NQ* NQ* EPB) __attribute__((amdgpu_waves_per_eu(WAV
       for (int m = 0; m < NQ; ++m) {
         qr = fmad((DREG ? Di[m] : s_D[i][m]), s_q[f][es][j][m], qr);
         qs = fmad((DREG ? Dj[m] : s_D[j][m]), s_q[f][es][m][i], qs);
-        qt = fmad((SDK ? Dc[k * NQ + m] : s_D[k][m]), rq[f][m], qt);
+        qt = fmad(s_D[k][m], rq[f][m], qt);
       }
-      T Gr, Gs, Gt;
-      if (TRI) {
-        const T gx = sc * fmad(atx, qt, fmad(asx, qs, arx * qr));
-        const T gy = sc * fmad(aty, qt, fmad(asy, qs, ary * qr));
-        const T gz = sc * fmad(atz, qt, fmad(asz, qs, arz * qr));
-        Gr = fmad(arz, gz, fmad(ary, gy, arx * gx));
-        Gs = fmad(asz, gz, fmad(asy, gy, asx * gx));
-        Gt = fmad(atz, gz, fmad(aty, gy, atx * gx));
-      } else {
-        Gr = fmad(G02, qt, fmad(G01, qs, G00 * qr));
-        Gs = fmad(G12, qt, fmad(G11, qs, G01 * qr));
-        Gt = fmad(G22, qt, fmad(G12, qs, G02 * qr));
-      }
+      const T Gr = fmad(G02, qt, fmad(G01, qs, G00 * qr));
+      const T Gs = fmad(G12, qt, fmad(G11, qs, G01 * qr));
+      const T Gt = fmad(G22, qt, fmad(G12, qs, G02 * qr));
       s_r[f][es][j][i] = Gr;
       s_s[f][es][j][i] = Gs;
       rA[f][k] = fmad(lambda * W, rq[f][k], rA[f][k]);
 #pragma unroll
-      for (int m = 0; m < NQ; ++m) rA[f][m] = fmad((SDK ? Dc[k * NQ + m] : s_D[k][m]), Gt, rA[f][m]);
+      for (int m = 0; m < NQ; ++m) rA[f][m] = fmad(s_D[k][m], Gt, rA[f][m]);
     }
     __syncthreads();
     asm volatile("" ::: "memory");
@@ -1089,16 +989,6 @@ int launch_bp5_v(hipStream_t s, const AxArgs<T>& a, T* Ap, double* part) {
   if (blocks == 0) return BPX_OK;
   const int* noPid = nullptr;
   const BatchState* noState = nullptr;
-  if constexpr (std::is_same<T, float>::value && NF == 1 && (VAR == VAR_PLAIN || VAR == VAR_FUSED)) {
-    if (a.tri && !a.affine) {
-      constexpr int WT = bp5_waves_tri<NQ, VAR>();
-      launch_stamped(k_bp5_ax<T, NQ, 1, EPB, false, WT, VAR, true, FOLD>, dim3(blocks), dim3(NQ * NQ * EPB), s,
-                     a.evStart, a.evStop, a.Nelements, a.K, a.elementList, a.GlobalToLocal, a.wJ, a.ggeo, a.gllw,
-                     a.D, a.lambda, a.q, a.Aq, a.ldq, a.ldAq, noPid, noState, Ap, part, a.fold);
-      BPX_HIP(hipGetLastError());
-      return BPX_OK;
-    }
-  }
   if constexpr (NF == 3 && VAR == VAR_PLAIN && EPB == 1) {
     // three fields, non-affine: one workgroup per field running the
     // one-field sweep (3 waves per SIMD in FP64 at Nq = 8, where the
@@ -1106,7 +996,7 @@ int launch_bp5_v(hipStream_t s, const AxArgs<T>& a, T* Ap, double* part) {
     if (!a.affine) {
       constexpr int W1 = bp5_waves_v<T, NQ, 1, VAR>();
       const unsigned fblocks = 8u * 3u * (unsigned)((a.Nelements + 7) / 8);
-      launch_stamped(k_bp5_ax<T, NQ, 1, 1, false, W1, VAR, false, false, 3>, dim3(fblocks), dim3(NQ * NQ), s,
+      launch_stamped(k_bp5_ax<T, NQ, 1, 1, false, W1, VAR, false, 3>, dim3(fblocks), dim3(NQ * NQ), s,
                      a.evStart, a.evStop, a.Nelements, a.K, a.elementList, a.GlobalToLocal, a.wJ, a.ggeo, a.gllw,
                      a.D, a.lambda, a.q, a.Aq, a.ldq, a.ldAq, noPid, noState, Ap, part, a.fold);
       BPX_HIP(hipGetLastError());
@@ -1114,11 +1004,11 @@ int launch_bp5_v(hipStream_t s, const AxArgs<T>& a, T* Ap, double* part) {
     }
   }
   if (a.affine)
-    launch_stamped(k_bp5_ax<T, NQ, NF, EPB, true, WV, VAR, false, FOLD>, dim3(blocks), dim3(NQ * NQ * EPB), s,
+    launch_stamped(k_bp5_ax<T, NQ, NF, EPB, true, WV, VAR, FOLD>, dim3(blocks), dim3(NQ * NQ * EPB), s,
                    a.evStart, a.evStop, a.Nelements, a.K, a.elementList, a.GlobalToLocal, a.wJ, a.ggeo, a.gllw,
                    a.D, a.lambda, a.q, a.Aq, a.ldq, a.ldAq, noPid, noState, Ap, part, a.fold);
   else
-    launch_stamped(k_bp5_ax<T, NQ, NF, EPB, false, WV, VAR, false, FOLD>, dim3(blocks), dim3(NQ * NQ * EPB), s,
+    launch_stamped(k_bp5_ax<T, NQ, NF, EPB, false, WV, VAR, FOLD>, dim3(blocks), dim3(NQ * NQ * EPB), s,
                    a.evStart, a.evStop, a.Nelements, a.K, a.elementList, a.GlobalToLocal, a.wJ, a.ggeo, a.gllw,
                    a.D, a.lambda, a.q, a.Aq, a.ldq, a.ldAq, noPid, noState, Ap, part, a.fold);
   BPX_HIP(hipGetLastError());
@@ -1310,47 +1200,6 @@ int launch_bp5_kappa_grad_nq(hipStream_t s, int Nelements, int affine, const int
   return BPX_OK;
 }
 
-// Batch variants for the setup-time tuner: workgroup shapes that round
-// identically (the default elements per workgroup, twice that, half of
-// it), so the tuner's choice never changes a result bit.
-template <int NQ, int V>
-constexpr int batch_epb() {
-  return V == 0 ? bp5_epb<NQ>() : V == 1 ? 2 * bp5_epb<NQ>() : bp5_epb<NQ>() / 2;
-}
-
-template <int NQ, int V>
-int launch_batch_v(hipStream_t s, int Nelements, const int* elementList, const int* G2L, const double* wJ,
-                   const double* ggeo, const double* D, double lambda, const double* q, double* Aq,
-                   const int* elemPid, const BatchState* done) {
-  constexpr int EPB = batch_epb<NQ, V>();
-  static_assert(EPB >= 1 && NQ * NQ * EPB <= 1024, "workgroup shape");
-  constexpr int WV = bp5_waves<NQ, 1, false>();
-  const int blocks = (Nelements + EPB - 1) / EPB;
-  if (blocks == 0) return BPX_OK;
-  hipLaunchKernelGGL((k_bp5_ax<double, NQ, 1, EPB, false, WV, VAR_BATCH>), dim3(blocks), dim3(NQ * NQ * EPB), 0,
-                     s, Nelements, 1, elementList, G2L, wJ, ggeo, (const double*)nullptr, D, lambda, q, Aq, 0LL,
-                     0LL, elemPid, done, (double*)nullptr, (double*)nullptr, CgFold<double>());
-  BPX_HIP(hipGetLastError());
-  return BPX_OK;
-}
-
-template <int NQ>
-int launch_bp5_batch_nq(hipStream_t s, int variant, int Nelements, const int* elementList, const int* G2L,
-                        const double* wJ, const double* ggeo, const double* D, double lambda, const double* q,
-                        double* Aq, const int* elemPid, const BatchState* done) {
-  if (variant == 0)
-    return launch_batch_v<NQ, 0>(s, Nelements, elementList, G2L, wJ, ggeo, D, lambda, q, Aq, elemPid, done);
-  if constexpr (NQ * NQ * 2 * bp5_epb<NQ>() <= 1024) {
-    if (variant == 1)
-      return launch_batch_v<NQ, 1>(s, Nelements, elementList, G2L, wJ, ggeo, D, lambda, q, Aq, elemPid, done);
-  }
-  if constexpr (bp5_epb<NQ>() >= 2) {
-    if (variant == 2)
-      return launch_batch_v<NQ, 2>(s, Nelements, elementList, G2L, wJ, ggeo, D, lambda, q, Aq, elemPid, done);
-  }
-  return set_error(BPX_ERR_INVALID_ARGUMENT, "batch Ax: variant not available for this degree");
-}
-
 // FP32 batch Ax (the mixed batch's inner operator): the default shape only
 template <int NQ>
 int launch_bp5_batch_f32_nq(hipStream_t s, int Nelements, const int* elementList, const int* G2L, const float* wJ,
@@ -1370,9 +1219,6 @@ int launch_bp5_batch_f32_nq(hipStream_t s, int Nelements, const int* elementList
 template int launch_bp5_batch_f32_nq<BPX_NQ>(hipStream_t, int, const int*, const int*, const float*, const float*,
                                              const float*, float, const float*, float*, const int*,
                                              const BatchState*);
-template int launch_bp5_batch_nq<BPX_NQ>(hipStream_t, int, int, const int*, const int*, const double*,
-                                         const double*, const double*, double, const double*, double*, const int*,
-                                         const BatchState*);
 template int launch_bp5_kappa_grad_nq<BPX_NQ>(hipStream_t, int, int, const int*, const double*, const double*,
                                               const double*, const double*, const double*, double*);
 template <typename T, int NQ>
@@ -1381,7 +1227,6 @@ int launch_bp5_fused_nq(hipStream_t s, const AxArgs<T>& a, T* Ap, double* part) 
 }
 
 template int launch_bp5_fused_nq<double, BPX_NQ>(hipStream_t, const AxArgs<double>&, double*, double*);
-template int launch_bp5_fused_nq<float, BPX_NQ>(hipStream_t, const AxArgs<float>&, float*, double*);
 template int launch_bp5_nq<double, BPX_NQ, 1>(hipStream_t, const AxArgs<double>&);
 template int launch_bp5_nq<double, BPX_NQ, 3>(hipStream_t, const AxArgs<double>&);
 template int launch_bp5_nq<float, BPX_NQ, 1>(hipStream_t, const AxArgs<float>&);

@@ -11,10 +11,6 @@ template <typename T, int NQ>
 int launch_bp5_fused_nq(hipStream_t s, const AxArgs<T>& a, T* Ap, double* part);
 template <typename T, int NQ> int launch_bp5_krhs_nq(hipStream_t s, const AxArgs<T>& a, int chunk);
 template <int NQ>
-int launch_bp5_batch_nq(hipStream_t s, int variant, int Nelements, const int* elementList, const int* G2L,
-                        const double* wJ, const double* ggeo, const double* D, double lambda, const double* q,
-                        double* Aq, const int* elemPid, const BatchState* done);
-template <int NQ>
 int launch_bp5_batch_f32_nq(hipStream_t s, int Nelements, const int* elementList, const int* G2L, const float* wJ,
                             const float* ggeo, const float* D, float lambda, const float* q, float* Aq,
                             const int* elemPid, const BatchState* done);

@@ -127,29 +127,11 @@ int launch_bp5_fused(hipStream_t s, const AxArgs<T>& a, T* Ap, double* part) {
 }
 
 template int launch_bp5_fused<double>(hipStream_t, const AxArgs<double>&, double*, double*);
-template int launch_bp5_fused<float>(hipStream_t, const AxArgs<float>&, float*, double*);
 
 int bp5_workgroups(int N, int Nelements) {
   const int Nq = N + 1;
   const int epb = Nq >= 8 ? 1 : 256 / (Nq * Nq);
   return (Nelements + epb - 1) / epb;
-}
-
-#define BPX_BATCH_CASE(NQ) \
-  case NQ:                  \
-    return launch_bp5_batch_nq<NQ>(s, variant, Nelements, elementList, G2L, wJ, ggeo, D, lambda, q, Aq, elemPid, done);
-
-int launch_bp5_batch(hipStream_t s, int N, int variant, int Nelements, const int* elementList, const int* G2L,
-                     const double* wJ, const double* ggeo, const double* D, double lambda, const double* q,
-                     double* Aq, const int* elemPid, const BatchState* done) {
-  if (Nelements <= 0) return BPX_OK;
-  switch (N + 1) {
-    BPX_BATCH_CASE(2) BPX_BATCH_CASE(3) BPX_BATCH_CASE(4) BPX_BATCH_CASE(5) BPX_BATCH_CASE(6)
-    BPX_BATCH_CASE(7) BPX_BATCH_CASE(8) BPX_BATCH_CASE(9) BPX_BATCH_CASE(10) BPX_BATCH_CASE(11)
-    BPX_BATCH_CASE(12) BPX_BATCH_CASE(13) BPX_BATCH_CASE(14) BPX_BATCH_CASE(15) BPX_BATCH_CASE(16)
-    default:
-      return set_error(BPX_ERR_UNSUPPORTED, "batch Ax: degree N must be in 1..15");
-  }
 }
 
 #define BPX_BATCH32_CASE(NQ) \
@@ -167,14 +149,6 @@ int launch_bp5_batch_f32(hipStream_t s, int N, int Nelements, const int* element
     default:
       return set_error(BPX_ERR_UNSUPPORTED, "batch Ax: degree N must be in 1..15");
   }
-}
-
-int bp5_batch_epb(int Nq, int variant) {
-  const int epb = Nq >= 8 ? 1 : 256 / (Nq * Nq);
-  if (variant == 0) return epb;
-  if (variant == 1) return Nq * Nq * 2 * epb <= 1024 ? 2 * epb : 0;
-  if (variant == 2) return epb >= 2 ? epb / 2 : 0;
-  return 0;
 }
 
 #define BPX_KGRAD_CASE(NQ) \

@@ -11,15 +11,17 @@
 //
 // Per-problem state lives on the device, so iterations never wait on the
 // host and a whole block of iterations can be captured in one hipGraph and
-// replayed. Writers and readers of each state field are split across
-// kernels so no kernel reads a field it also writes:
-//   update_p  (iteration k): reads rr_prev, iter; first chunk writes rr_k,
-//             tol2 (k = 0), and done/rnorm when the problem stops;
-//   update_xr (iteration k): reads rr_k; first chunk writes rr_prev = rr_k,
-//             iter = k + 1, and done/breakdown on a non-positive p.Ap;
-// every chunk recomputes the scalars it acts on, so all chunks of a
-// problem take the same branch. A converged problem's elements, rows and
-// chunks return at once in every kernel.
+// replayed. The FP64 iteration is the box kernels' pair, the Ax with the
+// direction update and the gather with the residual update (box_ax.hip,
+// box_gather.hip). Writers and readers of each state field are split across
+// them so no kernel reads a field it also writes:
+//   Ax (iteration k): reads rr_prev, alpha, iter; the first workgroup writes
+//             rr_k, tol2 (k = 0), and stop_at/rnorm when the problem stops;
+//   update (iteration k): reads rr_k, stop_at; the first workgroup writes
+//             alpha, rr_prev = rr_k, iter = k + 1, or done after a stop (and
+//             breakdown on a non-positive p.Ap);
+// every workgroup recomputes the scalars it acts on, so all of a problem
+// take the same branch. A finished problem's workgroups return at once.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -65,10 +67,12 @@ __device__ inline double block_sum(double v, double* s_w) {
   return t;
 }
 
-// r = b, x = 0, partial r.r per chunk; state reset
+// r = b, x = 0, partial r.r per chunk (from the problem's rr0 on); state reset
 __global__ __launch_bounds__(BT) void k_batch_init(const BatchChunk* __restrict__ chunks, const double* __restrict__ b,
                                                    double* __restrict__ x, double* __restrict__ r,
-                                                   double* __restrict__ part_rr, BatchState* st, int maxit) {
+                                                   const BoxBatchProb* __restrict__ probs,
+                                                   double* __restrict__ part_rr, BatchState* st, double tol,
+                                                   int maxit) {
   __shared__ double s_w[16];
   const BatchChunk c = chunks[blockIdx.x];
   double v = 0;
@@ -80,90 +84,10 @@ __global__ __launch_bounds__(BT) void k_batch_init(const BatchChunk* __restrict_
   }
   const double t = block_sum(v, s_w);
   if (threadIdx.x == 0) {
-    part_rr[blockIdx.x] = t;
-    if (c.first) {
-      BatchState& s = st[c.pid];
-      s.rr_k = 0;
-      s.rr_prev = 0;
-      s.tol2 = 0;
-      s.rnorm = 0;
-      s.iter = 0;
-      s.done = 0;
-      s.breakdown = 0;
-      s.maxit = maxit;
-    }
-  }
-}
-
-__global__ __launch_bounds__(BT) void k_batch_update_p(const BatchChunk* __restrict__ chunks,
-                                                       const int2* __restrict__ rrRange, const double* __restrict__ r,
-                                                       double* __restrict__ p, const double* __restrict__ part_rr,
-                                                       BatchState* st, double tol) {
-  __shared__ double s_w[16];
-  const BatchChunk c = chunks[blockIdx.x];
-  BatchState* s = st + c.pid;
-  if (s->done) return;
-  const int2 range = rrRange[c.pid];
-  double rr = fold_range(part_rr, range.x, range.y, s_w);
-  const int k = s->iter;
-  double tol2;
-  if (k == 0) {
-    const double nrm = sqrt(rr);  // rdotr = norm2(r)^2 (linearSolverCG.cpp:84-85)
-    rr = nrm * nrm;
-    tol2 = fmax(tol * tol * rr, tol * tol);
-  } else {
-    tol2 = s->tol2;
-  }
-  const bool stop = !(rr > tol2) || !isfinite(rr) || k >= s->maxit;
-  if (c.first && threadIdx.x == 0) {
-    s->rr_k = rr;
-    if (k == 0) s->tol2 = tol2;
-    if (stop) {
-      s->rnorm = sqrt(rr);
-      s->done = 1;
-      if (!isfinite(rr)) s->breakdown = 1;
-    }
-  }
-  if (stop) return;
-  const double beta = k == 0 ? 0.0 : rr / s->rr_prev;
-  for (int n = c.n0 + threadIdx.x; n < c.n1; n += BT) p[n] = k == 0 ? r[n] : 1.0 * r[n] + beta * p[n];
-}
-
-__global__ __launch_bounds__(BT) void k_batch_update_xr(const BatchChunk* __restrict__ chunks,
-                                                        const int2* __restrict__ pApRange,
-                                                        const double* __restrict__ p, const double* __restrict__ Ap,
-                                                        double* __restrict__ x, double* __restrict__ r,
-                                                        const double* __restrict__ part_pAp,
-                                                        double* __restrict__ part_rr, BatchState* st) {
-  __shared__ double s_w[16];
-  const BatchChunk c = chunks[blockIdx.x];
-  BatchState* s = st + c.pid;
-  if (s->done) return;
-  const int2 range = pApRange[c.pid];
-  const double pAp = fold_range(part_pAp, range.x, range.y, s_w);
-  const double rr = s->rr_k;
-  const double alpha = rr / pAp;
-  if (!isfinite(alpha) || !(pAp > 0.0)) {
-    if (c.first && threadIdx.x == 0) {
-      s->breakdown = 1;
-      s->done = 1;
-      s->rnorm = sqrt(rr);
-    }
-    return;
-  }
-  double v = 0;
-  for (int n = c.n0 + threadIdx.x; n < c.n1; n += BT) {
-    const double rn = r[n] - alpha * Ap[n];
-    r[n] = rn;
-    x[n] = alpha * p[n] + 1.0 * x[n];
-    v += rn * rn;
-  }
-  const double t = block_sum(v, s_w);
-  if (threadIdx.x == 0) {
-    part_rr[blockIdx.x] = t;
-    if (c.first) {
-      s->rr_prev = rr;
-      s->iter = s->iter + 1;
+    part_rr[probs[c.pid].rr0 + c.index] = t;
+    if (c.index == 0) {
+      const BatchState z{0, 0, 0, 0, 0, 0, 0, maxit, 0, 0, 0, tol};
+      st[c.pid] = z;
     }
   }
 }
@@ -292,7 +216,7 @@ __global__ __launch_bounds__(BT) void k_bm_init(const BatchChunk* __restrict__ c
   if (threadIdx.x == 0) {
     part_true[blockIdx.x] = tt;
     part_rr[blockIdx.x] = tr;
-    if (ch.first) {
+    if ((ch.index == 0)) {
       const BatchState z{0, 0, 0, 0, 0, 0, 0, maxit, 0, 0, 0, 0};
       inner[ch.pid] = z;
       outer[ch.pid] = z;
@@ -353,7 +277,7 @@ __global__ __launch_bounds__(BT) void k_bm_update_p(const BatchChunk* __restrict
   const double rr = fold_range(part_rr, range.x, range.y, s_w);
   const int k = s->iter;
   const bool stop = !(rr > 0) || !isfinite(rr) || outer[ch.pid].iter >= outer[ch.pid].maxit;
-  if (ch.first && threadIdx.x == 0) {
+  if ((ch.index == 0) && threadIdx.x == 0) {
     s->rr_k = rr;
     if (stop) s->done = 1;
   }
@@ -378,7 +302,7 @@ __global__ __launch_bounds__(BT) void k_bm_update_xr(const BatchChunk* __restric
   const double rr = s->rr_k;
   const double alpha = rr / pAp;
   if (!isfinite(alpha) || !(pAp > 0.0)) {  // the recurrence stops; the next correction restarts it
-    if (ch.first && threadIdx.x == 0) s->done = 1;
+    if ((ch.index == 0) && threadIdx.x == 0) s->done = 1;
     return;
   }
   const float a = (float)alpha;
@@ -392,7 +316,7 @@ __global__ __launch_bounds__(BT) void k_bm_update_xr(const BatchChunk* __restric
   const double t = block_sum(v, s_w);
   if (threadIdx.x == 0) {
     part_rr[blockIdx.x] = t;
-    if (ch.first) {
+    if ((ch.index == 0)) {
       s->rr_prev = rr;
       s->iter = s->iter + 1;
       outer[ch.pid].iter = outer[ch.pid].iter + 1;
@@ -498,37 +422,9 @@ int launch_bm_true_residual(hipStream_t s, int nchunks, const BatchChunk* chunks
 }
 
 int launch_batch_init(hipStream_t s, int nchunks, const BatchChunk* chunks, const double* b, double* x, double* r,
-                      double* part_rr, BatchState* st, int maxit) {
+                      const BoxBatchProb* probs, double* part_rr, BatchState* st, double tol, int maxit) {
   if (nchunks <= 0) return BPX_OK;
-  hipLaunchKernelGGL(k_batch_init, dim3(nchunks), dim3(BT), 0, s, chunks, b, x, r, part_rr, st, maxit);
-  BPX_HIP(hipGetLastError());
-  return BPX_OK;
-}
-
-int launch_batch_update_p(hipStream_t s, int nchunks, const BatchChunk* chunks, const int2* rrRange, const double* r,
-                          double* p, const double* part_rr, BatchState* st, double tol) {
-  if (nchunks <= 0) return BPX_OK;
-  hipLaunchKernelGGL(k_batch_update_p, dim3(nchunks), dim3(BT), 0, s, chunks, rrRange, r, p, part_rr, st, tol);
-  BPX_HIP(hipGetLastError());
-  return BPX_OK;
-}
-
-int launch_batch_update_xr(hipStream_t s, int nchunks, const BatchChunk* chunks, const int2* pApRange,
-                           const double* p, const double* Ap, double* x, double* r, const double* part_pAp,
-                           double* part_rr, BatchState* st) {
-  if (nchunks <= 0) return BPX_OK;
-  hipLaunchKernelGGL(k_batch_update_xr, dim3(nchunks), dim3(BT), 0, s, chunks, pApRange, p, Ap, x, r, part_pAp,
-                     part_rr, st);
-  BPX_HIP(hipGetLastError());
-  return BPX_OK;
-}
-
-int launch_batch_gather(hipStream_t s, int nsupers, const BatchSuper* supers, const int* rowStarts,
-                        const int* colIds, const double* q, double* gq, const double* p, double* part,
-                        const BatchState* st) {
-  if (nsupers <= 0) return BPX_OK;
-  hipLaunchKernelGGL((k_batch_gather<double, true>), dim3(nsupers), dim3(GT), 0, s, supers, rowStarts, colIds, q, gq,
-                     p, part, st);
+  hipLaunchKernelGGL(k_batch_init, dim3(nchunks), dim3(BT), 0, s, chunks, b, x, r, probs, part_rr, st, tol, maxit);
   BPX_HIP(hipGetLastError());
   return BPX_OK;
 }

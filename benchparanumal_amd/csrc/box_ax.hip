@@ -1,34 +1,5 @@
-// BP5 / BP6 Ax on the structured hex box, FP64 and FP32: the operator of
-// okl/bp5AxHex3D.okl:415-569 (and bp6AxHex3D.okl) with the geometry formed
-// in the kernel and the rows of box.hpp in place of GlobalToLocal.
-//
-// What it leaves out of memory. The box's elements are trilinear maps of
-// their 8 vertices, so the 7 factors of a node (56 bytes in FP64, 340 of the
-// 518 MB that the stored-factor kernel moves at 24^3, p = 7) follow from 24
-// numbers per element, and the row of a node from its place in the box. A
-// node then costs its q (read), its result (written) and nothing else:
-// 94 MB. The factors are the exact derivatives of the map; the stored ones
-// are derivatives by D, whose rounding the operator magnifies (relative
-// error against exact arithmetic at 24^3, p = 7: 8e-14 stored, 2e-15 here).
-// Measured there, FP64: Ax 97 -> 30 us, operator 127 -> 57 us; BP6 (three
-// fields, the geometry formed for each) 255 -> 172 us.
-//
-// Layout (the pencil form of ax_bp5.hip): a lane owns the nodes (k, b, a),
-// k = 0..Nq-1, of its element; one-dimensional contractions run along a
-// pencil that one lane holds, with the matrix uniform over the wavefront,
-// and values move between directions through two LDS buffers, 16 accesses
-// per node (the sheet form reads 4 Nq). D is antisymmetric about the middle
-// of the GLL points in both indices, so each contraction works on the even
-// and odd parts of its pencil: Nq^2/2 + 2 Nq operations in place of Nq^2,
-// and D and its transpose share one table of Nq^2/2 values.
-//
-// At Nq = 8 an element is one wavefront, whose LDS traffic needs no
-// workgroup barrier (a wavefront's LDS operations execute in order).
-#include <hip/hip_runtime.h>
-
-#include "box_common.hpp"
-#include "buffer_rsrc.hpp"
-#include "fold.hpp"
+// The Ax of box_ax_body.hpp, one problem per launch. Compiled once per Nq.
+#include "box_ax_body.hpp"
 
 #ifndef BPX_NQ
 #error "compile with -DBPX_NQ=<Nq>"
@@ -37,487 +8,11 @@
 namespace bpx {
 namespace {
 
-__device__ inline double fmad(double a, double b, double c) { return __builtin_fma(a, b, c); }
-__device__ inline float fmad(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-
-// 1/x: FP32 by the hardware (1 ulp), FP64 by two Newton steps on it
-__device__ inline float reciprocal(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ inline double reciprocal(double x) {
-  double y = __builtin_amdgcn_rcp(x);
-  y = fmad(fmad(-x, y, 1.0), y, y);
-  return fmad(fmad(-x, y, 1.0), y, y);
-}
-
-// y = D x (or D^T x) from the even-odd table: row n <= (NQ-1)/2 holds
-// S[n][m] = (D[n][m] + D[n][NQ-1-m])/2 for m < NQ/2, D[n][NQ/2] for odd NQ,
-// A[n][m] = (D[n][m] - D[n][NQ-1-m])/2 for m < NQ/2. Rows come through
-// scalar loads. Up to Nq = 8 the table (64 scalar registers in FP64) may
-// stay in registers; beyond, each row is requested where it is used.
-template <typename T, int NQ>
-struct EvenOdd {
-  static constexpr int H = NQ / 2, ODD = NQ & 1, ROWS = H + ODD;
-  typedef const __attribute__((address_space(4))) T* cptr;
-  static constexpr bool HOLD = NQ <= 8;
-
-  template <typename F>
-  __device__ static inline void rows(cptr tab, F&& body) {
-#pragma unroll
-    for (int n = 0; n < ROWS; ++n) {
-      if constexpr (!HOLD) asm volatile("" : "+s"(tab));
-      T r[NQ];
-#pragma unroll
-      for (int m = 0; m < NQ; ++m) r[m] = tab[n * NQ + m];
-      body(n, r);
-    }
-  }
-
-  __device__ static inline void apply(cptr tab, const T (&x)[NQ], T (&y)[NQ]) {
-    T xe[H], xo[H];
-#pragma unroll
-    for (int m = 0; m < H; ++m) {
-      xe[m] = x[m] + x[NQ - 1 - m];
-      xo[m] = x[m] - x[NQ - 1 - m];
-    }
-    const T xm = x[H];  // the middle value (odd NQ)
-    rows(tab, [&](int n, const T* r) {
-      T ye = 0, yo = 0;
-#pragma unroll
-      for (int m = 0; m < H; ++m) {
-        ye = fmad(r[H + ODD + m], xo[m], ye);
-        if (n < H) yo = fmad(r[m], xe[m], yo);
-      }
-      if (n == H) {
-        y[n] = ye;
-      } else {
-        if constexpr (ODD) yo = fmad(r[H], xm, yo);
-        y[n] = ye + yo;
-        y[NQ - 1 - n] = ye - yo;
-      }
-    });
-  }
-
-  __device__ static inline void apply_transposed(cptr tab, const T (&x)[NQ], T (&y)[NQ]) {
-    T ye[H], yo[H], ym = 0;
-#pragma unroll
-    for (int n = 0; n < H; ++n) ye[n] = yo[n] = T(0);
-    rows(tab, [&](int m, const T* r) {
-      if (m < H) {
-        const T xe = x[m] + x[NQ - 1 - m], xo = x[m] - x[NQ - 1 - m];
-#pragma unroll
-        for (int n = 0; n < H; ++n) {
-          ye[n] = fmad(r[n], xo, ye[n]);
-          yo[n] = fmad(r[H + ODD + n], xe, yo[n]);
-        }
-        if constexpr (ODD) ym = fmad(r[H], xo, ym);
-      } else {  // the middle row: D[mid][n], antisymmetric in n
-#pragma unroll
-        for (int n = 0; n < H; ++n) yo[n] = fmad(r[H + ODD + n], x[H], yo[n]);
-      }
-    });
-#pragma unroll
-    for (int n = 0; n < H; ++n) {
-      y[n] = ye[n] + yo[n];
-      y[NQ - 1 - n] = ye[n] - yo[n];
-    }
-    if constexpr (ODD) y[H] = ym;
-  }
-};
-
-// occupancy handed to the register allocator: what the pencils, the map's
-// 25 constants and the temporaries fit without spilling
-template <typename T, int NQ>
-constexpr int box_waves() {
-  return sizeof(T) == 4 ? (NQ <= 8 ? 7 : NQ <= 12 ? 5 : 4) : (NQ <= 8 ? 4 : NQ <= 12 ? 3 : 2);
-}
-
-template <int NQ>
-__device__ inline void element_sync() {
-  if constexpr (NQ == 8) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    asm volatile("" ::: "memory");
-  } else {
-    __syncthreads();
-  }
-  __builtin_amdgcn_sched_barrier(0);
-}
-
-// MODE_FOLD: the direction update of a CG iteration and the x update of the
-// one before inside the Ax. Every element forms the new direction of all its
-// nodes from r and the old one (neighbours form the same bits), the owner
-// writes it, to another vector. An iteration is then this kernel and
-// k_box_update_r: at 24^3, p = 7 FP32 76 -> 54 us against four kernels with
-// k_bp5_ax, at 10^3, p = 4 affine FP64 23 -> 13 us.
-enum { MODE_PLAIN = 0, MODE_DOT = 1, MODE_FOLD = 2 };
-
-// GEO: where the factors come from
-enum { GEO_TRILINEAR = 0, GEO_AFFINE = 1, GEO_STORED = 2 };
-
-template <typename T, int NQ, int GEO, bool KAPPA, int MODE, bool BATCH = false>
+template <typename T, int NQ, int GEO, bool KAPPA, int MODE>
 __global__ __launch_bounds__(NQ* NQ* box_epb(NQ)) __attribute__((amdgpu_waves_per_eu(box_waves<T, NQ>()))) void k_box_ax(
     BoxAxArgs<T> a, int per_xcd) {
-  constexpr int N = NQ - 1, NQ2 = NQ * NQ, NP = NQ2 * NQ, EPB = box_epb(NQ);
-  constexpr int LK = NQ2 + 8, LE = NQ * LK, S = (int)sizeof(T);
-  using EO = EvenOdd<T, NQ>;
-  typedef typename EO::cptr cptr;
-  __shared__ T s_b[EPB * LE];  // pencils along i
-  __shared__ T s_c[EPB * LE];  // pencils along j
-
-  __shared__ double s_f[MODE == MODE_PLAIN ? 1 : NQ2 * EPB];  // sums; s_f[32] hands the folded r.r out
-
-  const int t = threadIdx.x;
-  BoxGrid g;
-  int grp = 0, it = a.k;  // element group, iteration
-  long long row0v = 0;    // first row of the problem in the vectors
-  BatchState* bs = nullptr;
-  if constexpr (BATCH) {
-    const BoxBatchItem item = a.items[blockIdx.x];
-    const BoxBatchProb* pr = a.probs + item.pid;
-    bs = a.bst + item.pid;
-    if (bs->done) return;
-    g = pr->g;
-    grp = item.e0 / EPB;
-    row0v = pr->off;
-    a.geo += 24 * pr->el0;
-    a.AqL += pr->loc;
-    if constexpr (MODE == MODE_FOLD) {
-      it = bs->iter;
-      if (bs->stop_at != 0 && bs->stop_at <= it) return;
-      if ((it & 1) == 0) {  // the direction of iteration k is in p for odd k
-        const T* q = a.p;
-        a.p = const_cast<T*>(a.q);
-        a.q = q;
-      }
-      a.r += row0v;
-      a.p += row0v;
-      a.x += row0v;
-      a.part_rr += pr->rr0;
-      a.nrr = it == 0 ? pr->ninit : pr->nrr;
-      a.part += pr->pAp0;
-    }
-    a.q += row0v;
-  } else {
-    g = a.g;
-    grp = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-    if constexpr (MODE == MODE_FOLD) {
-      if (a.k > 0 && (a.st->done || (a.st->stop_at != 0 && a.st->stop_at <= a.k))) return;
-    }
-  }
-  const int nel = g.elements();
-  if (grp * EPB >= nel) return;  // uniform
-  int es = t / NQ2;
-  if constexpr (NQ == 8) es = __builtin_amdgcn_readfirstlane(es);
-  const int tl = t - es * NQ2;
-  const int ai = tl % NQ, bj = tl / NQ;
-  const bool active = grp * EPB + es < nel;
-  const int e = active ? grp * EPB + es : 0;
-  const int f = blockIdx.y;
-
-  // rows of the lane's pencil: row0 at k = 0 (owned one layer down), then
-  // row1 + (k-1)*stride; masked ones read 0
-  int ex, ey, ez;
-  g.element(e, ex, ey, ez);
-  const int ox = ex - (ai == 0), oy = ey - (bj == 0);
-  const bool on = active && ox >= 0 && oy >= 0 && !(ai == N && ex == g.nx - 1) && !(bj == N && ey == g.ny - 1);
-  const int Nx = BoxGrid::owned<N>(ox, g.nx), Ny = BoxGrid::owned<N>(oy, g.ny);
-  const int stride = Nx * Ny;
-  const int at = ((bj == 0 ? N : bj) - 1) * Nx + (ai == 0 ? N : ai) - 1;
-  const int Nz = BoxGrid::owned<N>(ez, g.nz);
-  unsigned off[NQ];
-  {
-    const unsigned row1 = (unsigned)(g.template base<N>(a.F, ox, oy, ez) + f * stride * Nz + at);
-    const unsigned row0 = (unsigned)(g.template base<N>(a.F, ox, oy, ez - 1) + (f * N + N - 1) * stride + at);
-    off[0] = on && ez > 0 ? row0 * S : kBoxMasked;
-#pragma unroll
-    for (int k = 1; k < NQ; ++k) off[k] = on && k <= Nz ? (row1 + (k - 1) * stride) * S : kBoxMasked;
-  }
-  T rq[NQ];
-  if constexpr (MODE == MODE_FOLD) {
-    const __amdgpu_buffer_rsrc_t rr_ = box_rsrc(a.r), rp = box_rsrc(a.q), rx = box_rsrc(a.x), ro = box_rsrc(a.p);
-    const bool own = ai > 0 && bj > 0;
-    T pv[NQ], xv[NQ];
-    const bool first = it == 0, apply = (BATCH || a.pending) && !first;
-#pragma unroll
-    for (int k = 0; k < NQ; ++k) rq[k] = buffer_load<T>(rr_, off[k]);
-    if (!first) {
-#pragma unroll
-      for (int k = 0; k < NQ; ++k) pv[k] = buffer_load<T>(rp, off[k]);
-    }
-    if (apply) {
-#pragma unroll
-      for (int k = 1; k < NQ; ++k) xv[k] = buffer_load<T>(rx, own ? off[k] : kBoxMasked);
-    }
-    if (t < 64) {
-      const double v = wave_fold(a.part_rr, a.nrr);
-      if (t == 0) s_f[32] = v;
-    }
-    __syncthreads();
-    double rr = s_f[32], tol2;
-    const double tol = BATCH ? bs->tol : a.tol;
-    if (first) {
-      const double nrm = sqrt(rr);  // rdotr = norm2(r)^2 (linearSolverCG.cpp:84-85)
-      rr = nrm * nrm;
-      tol2 = fmax(tol * tol * rr, tol * tol);
-    } else {
-      tol2 = BATCH ? bs->tol2 : a.st->tol2;
-    }
-    bool stop = !(rr > tol2) || !isfinite(rr);
-    if constexpr (BATCH) {
-      stop = stop || it >= bs->maxit;
-      if (grp == 0 && t == 0) {
-        bs->rr_k = rr;
-        if (first) bs->tol2 = tol2;
-        if (stop) {
-          bs->rnorm = sqrt(rr);
-          if (!isfinite(rr)) bs->breakdown = 1;
-          bs->stop_at = it + 1;
-        }
-      }
-    } else if (blockIdx.x == 0 && blockIdx.y == 0 && t == 0) {
-      a.hist_rr[a.k] = rr;
-      if (first) {
-        a.st->tol2 = tol2;
-        a.st->breakdown = 0;
-        a.st->done = 0;
-        a.st->stop_at = 0;
-      }
-      if (stop) {
-        a.st->iter = a.k;
-        if (!isfinite(rr)) a.st->breakdown = 1;
-        a.st->stop_at = a.k + 1;
-      }
-    }
-    if (apply) {
-      const T al = (T)(BATCH ? bs->alpha : a.hist_alpha[it - 1]);
-#pragma unroll
-      for (int k = 1; k < NQ; ++k) buffer_store<T>(fmad(al, pv[k], xv[k]), rx, own ? off[k] : kBoxMasked);
-    }
-    if (stop) return;  // uniform over the problem
-    if (!first) {
-      const T beta = (T)(rr / (BATCH ? bs->rr_prev : a.hist_rr[it - 1]));
-#pragma unroll
-      for (int k = 0; k < NQ; ++k) rq[k] = fmad(beta, pv[k], rq[k]);
-    }
-#pragma unroll
-    for (int k = 1; k < NQ; ++k) buffer_store<T>(rq[k], ro, own ? off[k] : kBoxMasked);
-  } else {
-    const __amdgpu_buffer_rsrc_t rs = box_rsrc(a.q + (size_t)blockIdx.z * a.ldq);
-#pragma unroll
-    for (int k = 0; k < NQ; ++k) rq[k] = buffer_load<T>(rs, off[k]);
-  }
-
-  // LDS slots. Along k (node (k, b, a)): kb + k*LK in s_b, kc + k*LK in s_c;
-  // along i (node (b, a, m)): oi[m] in s_b; along j (node (b, m, a)):
-  // jc + m*NQ in s_c. (oi[m] = ib + (m + a) mod NQ.) The rotation in s_b keeps its three access patterns
-  // free of bank conflicts.
-  const int kb = es * LE + bj * NQ + (ai + bj) % NQ;
-  const int kc = es * LE + bj * NQ + ai;
-  const int jc = es * LE + bj * LK + ai;
-  const int ib = es * LE + bj * LK + ai * NQ;
-  // formed where they are used (an opaque copy of the lane's a each time),
-  // not held in NQ registers across the node loop
-  auto slots_i = [&](int (&oi)[NQ]) {
-    int r = ai;
-    asm volatile("" : "+v"(r));
-#pragma unroll
-    for (int m = 0; m < NQ; ++m) oi[m] = ib + (m + r < NQ ? m + r : m + r - NQ);
-  };
-  cptr tab = (cptr)a.eo;
-
-#pragma unroll
-  for (int k = 0; k < NQ; ++k) {
-    s_b[k * LK + kb] = rq[k];
-    s_c[k * LK + kc] = rq[k];
-  }
-  element_sync<NQ>();
-  // r derivative at (j, k) = (a, b), s derivative at (i, k) = (a, b); each
-  // lane overwrites only its own pencil
-  {
-    int oi[NQ];
-    slots_i(oi);
-    T v[NQ], y[NQ];
-#pragma unroll
-    for (int m = 0; m < NQ; ++m) v[m] = s_b[oi[m]];
-    EO::apply(tab, v, y);
-#pragma unroll
-    for (int m = 0; m < NQ; ++m) s_b[oi[m]] = y[m];
-#pragma unroll
-    for (int m = 0; m < NQ; ++m) v[m] = s_c[jc + m * NQ];
-    EO::apply(tab, v, y);
-#pragma unroll
-    for (int m = 0; m < NQ; ++m) s_c[jc + m * NQ] = y[m];
-  }
-  element_sync<NQ>();
-
-  // along k: t derivative, the factors, the mass term; Gr and Gs out, Gt kept
-  T gt[NQ], rA[NQ];
-  double dot = 0;
-  EO::apply(tab, rq, gt);
-  __builtin_amdgcn_sched_barrier(0);
-  {
-    // TRILINEAR: along the pencil x_r = Ar + Br t, x_s = As + Bs t and x_t = Ct,
-    // so the adjugate's rows J grad r = x_s x x_t = Pr + Qr t and J grad s =
-    // x_t x x_r = Ps + Qs t are linear in t, and J grad t = x_r x x_s =
-    // T0 + T1 t + T2 t^2 and J = x_t . (J grad t) are quadratic
-    T Pr[3], Qr[3], Ps[3], Qs[3], T0[3], T1[3], T2[3], jt[3], ga[6], gw = 0;
-    if constexpr (GEO == GEO_TRILINEAR) {
-      const T r = a.z[ai], sn = a.z[bj];
-      const cptr ce = (cptr)a.geo + (size_t)24 * e;
-      T Ar[3], Br[3], As[3], Bs[3], Ct[3];
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const T c_r = ce[8 * d + 0], c_s = ce[8 * d + 1], c_t = ce[8 * d + 2], c_rs = ce[8 * d + 3];
-        const T c_rt = ce[8 * d + 4], c_st = ce[8 * d + 5], c_rst = ce[8 * d + 6];
-        Ar[d] = fmad(c_rs, sn, c_r);
-        Br[d] = fmad(c_rst, sn, c_rt);
-        As[d] = fmad(c_rs, r, c_s);
-        Bs[d] = fmad(c_rst, r, c_st);
-        Ct[d] = fmad(Br[d], r, fmad(c_st, sn, c_t));
-      }
-      auto cross = [](const T* u, const T* v, int d) {
-        const int d1 = (d + 1) % 3, d2 = (d + 2) % 3;
-        return fmad(u[d1], v[d2], -(u[d2] * v[d1]));
-      };
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        Pr[d] = cross(As, Ct, d);
-        Qr[d] = cross(Bs, Ct, d);
-        Ps[d] = cross(Ct, Ar, d);
-        Qs[d] = cross(Ct, Br, d);
-        T0[d] = cross(Ar, As, d);
-        T1[d] = cross(Ar, Bs, d) + cross(Br, As, d);
-        T2[d] = cross(Br, Bs, d);
-      }
-      jt[0] = fmad(Ct[0], T0[0], fmad(Ct[1], T0[1], Ct[2] * T0[2]));
-      jt[1] = fmad(Ct[0], T1[0], fmad(Ct[1], T1[1], Ct[2] * T1[2]));
-      jt[2] = fmad(Ct[0], T2[0], fmad(Ct[1], T2[1], Ct[2] * T2[2]));
-    } else if constexpr (GEO == GEO_AFFINE) {
-#pragma unroll
-      for (int c = 0; c < 6; ++c) ga[c] = a.geo[6 * (size_t)e + c];
-      gw = a.wJ[e];
-    }
-    const T wij = GEO == GEO_STORED ? T(0) : a.w[ai] * a.w[bj];
-    T zk[NQ], wk[NQ];  // uniform: scalar loads
-    if constexpr (GEO != GEO_STORED) {
-#pragma unroll
-      for (int k = 0; k < NQ; ++k) {
-        if constexpr (GEO == GEO_TRILINEAR) zk[k] = ((cptr)a.z)[k];
-        wk[k] = ((cptr)a.w)[k];
-      }
-    }
-    const T* kap = nullptr;
-    int kstep = 0;
-    if constexpr (KAPPA) {
-      const int LX = g.nx * N + 1, LY = g.ny * N + 1;
-      kap = a.kappa + (size_t)(ez * N) * ((size_t)LX * LY) + (size_t)(ey * N + bj) * LX + (ex * N + ai);
-      kstep = LX * LY;
-    }
-#pragma unroll
-    for (int k = 0; k < NQ; ++k) {
-      // one node at a time: without these the compiler forms every node's
-      // map values before the first is used and spills
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (GEO == GEO_TRILINEAR) {
-#pragma unroll
-        for (int d = 0; d < 3; ++d) asm volatile("" : "+v"(Pr[d]), "+v"(Ps[d]), "+v"(T0[d]), "+v"(jt[d]));
-      }
-      const T qr = s_b[k * LK + kb], qs = s_c[k * LK + kc], qt = gt[k];
-      T Gr, Gs, Gt, W;
-      if constexpr (GEO == GEO_TRILINEAR) {
-        const T tk = zk[k];
-        T ar[3], as[3], av[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          ar[d] = fmad(Qr[d], tk, Pr[d]);
-          as[d] = fmad(Qs[d], tk, Ps[d]);
-          av[d] = fmad(fmad(T2[d], tk, T1[d]), tk, T0[d]);
-        }
-        const T J = fmad(fmad(jt[2], tk, jt[1]), tk, jt[0]);
-        const T w = wij * wk[k];
-        T sc = w * reciprocal(J);
-        W = J * w;
-        if constexpr (KAPPA) sc *= kap[(size_t)k * kstep];
-        // G (grad q) as adj (w/J) adj^T, G itself not formed
-        T gx[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) gx[d] = sc * fmad(av[d], qt, fmad(as[d], qs, ar[d] * qr));
-        Gr = fmad(ar[2], gx[2], fmad(ar[1], gx[1], ar[0] * gx[0]));
-        Gs = fmad(as[2], gx[2], fmad(as[1], gx[1], as[0] * gx[0]));
-        Gt = fmad(av[2], gx[2], fmad(av[1], gx[1], av[0] * gx[0]));
-      } else {
-        T g[6];
-        if constexpr (GEO == GEO_AFFINE) {
-          const T w = wij * wk[k];
-          T wg = w;
-          if constexpr (KAPPA) wg *= kap[(size_t)k * kstep];
-#pragma unroll
-          for (int c = 0; c < 6; ++c) g[c] = ga[c] * wg;
-          W = gw * w;
-        } else {
-          const size_t n = (size_t)e * NP + k * NQ2 + tl;
-#pragma unroll
-          for (int c = 0; c < 6; ++c) g[c] = a.geo[6 * n + c];
-          W = a.wJ[n];
-        }
-        Gr = fmad(g[2], qt, fmad(g[1], qs, g[0] * qr));
-        Gs = fmad(g[4], qt, fmad(g[3], qs, g[1] * qr));
-        Gt = fmad(g[5], qt, fmad(g[4], qs, g[2] * qr));
-      }
-      s_b[k * LK + kb] = Gr;
-      s_c[k * LK + kc] = Gs;
-      gt[k] = Gt;
-      rA[k] = (a.lambda * W) * rq[k];
-      if constexpr (MODE != MODE_PLAIN && sizeof(T) == 8) {
-        // q.Aq node by node: grad q . G grad q + lambda W q^2
-        dot = fmad(rA[k], rq[k], fmad(Gt, qt, fmad(Gs, qs, fmad(Gr, qr, dot))));
-        asm volatile("" : "+v"(dot));
-      }
-      asm volatile("" : "+v"(gt[k]), "+v"(rA[k]));
-    }
-  }
-  // (the table is requested again: held across the nodes it would take the
-  // scalar registers of their coordinates and weights)
-  asm volatile("" : "+s"(tab));
-  {
-    T y[NQ];
-    EO::apply_transposed(tab, gt, y);
-#pragma unroll
-    for (int k = 0; k < NQ; ++k) rA[k] += y[k];
-  }
-  element_sync<NQ>();
-  // the divergence's r part along i, its s part along j
-  {
-    int oi[NQ];
-    slots_i(oi);
-    T v[NQ], y[NQ];
-#pragma unroll
-    for (int m = 0; m < NQ; ++m) v[m] = s_b[oi[m]];
-    EO::apply_transposed(tab, v, y);
-#pragma unroll
-    for (int m = 0; m < NQ; ++m) s_b[oi[m]] = y[m];
-#pragma unroll
-    for (int m = 0; m < NQ; ++m) v[m] = s_c[jc + m * NQ];
-    EO::apply_transposed(tab, v, y);
-#pragma unroll
-    for (int m = 0; m < NQ; ++m) s_c[jc + m * NQ] = y[m];
-  }
-  element_sync<NQ>();
-#pragma unroll
-  for (int k = 0; k < NQ; ++k) rA[k] += s_b[k * LK + kb] + s_c[k * LK + kc];
-  if constexpr (MODE != MODE_PLAIN) {
-    if constexpr (sizeof(T) == 4) {  // q.Aq from the rounded results, as the rows see them
-#pragma unroll
-      for (int k = 0; k < NQ; ++k) dot = fmad((double)rq[k], (double)rA[k], dot);
-    }
-    const double v = block_sum<NQ2 * EPB>(dot, s_f);
-    if (t == 0) a.part[(size_t)blockIdx.y * ((nel + EPB - 1) / EPB) + grp] = v;
-  }
-  if (active) {
-    T* out = a.AqL + (size_t)blockIdx.z * a.ldAq + ((size_t)e * a.F + f) * NP + tl;
-#pragma unroll
-    for (int k = 0; k < NQ; ++k) out[k * NQ2] = rA[k];
-  }
+  __shared__ BoxAxLds<T, NQ, MODE> lds;
+  box_ax_body<T, NQ, GEO, KAPPA, MODE, false>(a, per_xcd, lds);
 }
 
 template <typename T, int NQ, int GEO, bool KAPPA, int MODE>
@@ -537,25 +32,11 @@ int launch_geo(hipStream_t s, const BoxAxArgs<T>& a) {
   return launch_mode<T, NQ, GEO, KAPPA, MODE_PLAIN>(s, a);
 }
 
-// the batch forms: FP64, trilinear
-template <int NQ>
-int launch_batch(hipStream_t s, const BoxAxArgs<double>& a) {
-  if (a.nitems == 0) return BPX_OK;
-  const dim3 grid((unsigned)a.nitems), block(NQ * NQ * box_epb(NQ));
-  if (a.fold)
-    hipLaunchKernelGGL((k_box_ax<double, NQ, GEO_TRILINEAR, false, MODE_FOLD, true>), grid, block, 0, s, a, 0);
-  else
-    hipLaunchKernelGGL((k_box_ax<double, NQ, GEO_TRILINEAR, false, MODE_PLAIN, true>), grid, block, 0, s, a, 0);
-  BPX_HIP(hipGetLastError());
-  return BPX_OK;
-}
-
 }  // namespace
 
 template <typename T, int NQ>
 int launch_box_ax_nq(hipStream_t s, const BoxAxArgs<T>& a) {
-  if constexpr (sizeof(T) == 8) {  // batches and the variable coefficient are FP64
-    if (a.items) return launch_batch<NQ>(s, a);
+  if constexpr (sizeof(T) == 8) {  // the variable coefficient is an FP64 operator
     if (a.kappa)
       return a.geoKind == BOX_GEO_AFFINE ? launch_geo<T, NQ, GEO_AFFINE, true>(s, a)
                                          : launch_geo<T, NQ, GEO_TRILINEAR, true>(s, a);

@@ -27,15 +27,14 @@ int launch_box_ax(hipStream_t s, const BoxAxArgs<T>& a) {
   if (!a.geo || !a.eo || (a.geoKind == BOX_GEO_TRILINEAR && !a.z) || (a.geoKind != BOX_GEO_TRILINEAR && !a.wJ) ||
       (a.geoKind != BOX_GEO_STORED && !a.w))
     return set_error(BPX_ERR_INVALID_ARGUMENT, "box Ax: null geometry/operator pointer");
-  if (a.items) {
-    if (!a.probs || !a.bst || (a.fold && (!a.part || !a.r || !a.p || !a.x || !a.part_rr)))
-      return set_error(BPX_ERR_INVALID_ARGUMENT, "box Ax: incomplete batch arguments");
-  } else if (a.fold && (!a.part || !a.r || !a.p || !a.x || !a.part_rr || !a.hist_rr || !a.hist_alpha || !a.st || a.p == a.q))
+  if (a.fold && (!a.part || !a.r || !a.p || !a.x || !a.part_rr || !a.hist_rr || !a.hist_alpha || !a.st || a.p == a.q))
     return set_error(BPX_ERR_INVALID_ARGUMENT, "box Ax: incomplete CG arguments");
 #define BPX_CALL(NQ) case NQ: return launch_box_ax_nq<T, NQ>(s, a);
   BPX_BOX_SWITCH(BPX_CALL)
 #undef BPX_CALL
 }
+
+int box_gather_elements(int Nq) { return box_gather_epb(Nq); }
 
 int box_ax_elements(int Nq) { return box_epb(Nq); }
 

@@ -99,10 +99,6 @@ struct AxArgs {
   // rounding, not bit for bit. AX_ENGINE_AUTO = matrix cores where they
   // apply (the faster: 814 against 1084 us at 24^3, p = 15).
   int engine = 0;
-  // FP32 BP5, non-affine: ggeo holds the coefficients of each element's
-  // trilinear map (24 per element) and wJ the GLL nodes; the kernel forms
-  // the geometric factors itself
-  int tri = 0;
   // BP1-BP4 non-affine at Nq <= 8: the pencil kernel (CUB_FORM_AUTO or
   // CUB_FORM_PENCIL) or the wavefront-per-element kernels (CUB_FORM_WAVE);
   // the two agree to rounding, not bit for bit
@@ -219,7 +215,7 @@ int launch_bp5_kappa_grad(hipStream_t s, int N, int Nelements, int affine, const
 // A chunk of one problem's slice of the concatenated vectors; first marks
 // the chunk that writes the problem's state.
 struct BatchChunk {
-  int pid, n0, n1, first;
+  int pid, n0, n1, index;  // index within the problem
 };
 // Rows [r0, r1) of the concatenated gather maps, all of problem pid.
 struct BatchSuper {
@@ -238,22 +234,9 @@ struct BatchState {
   int stop_at;
   double alpha, tol;
 };
-// BP5 Ax over the elements of one degree group; variant = workgroup shape
-// (bp5_batch_epb: elements per workgroup, 0 if the variant does not exist)
-int launch_bp5_batch(hipStream_t s, int N, int variant, int Nelements, const int* elementList, const int* G2L,
-                     const double* wJ, const double* ggeo, const double* D, double lambda, const double* q,
-                     double* Aq, const int* elemPid, const BatchState* done);
-int bp5_batch_epb(int Nq, int variant);
+struct BoxBatchProb;
 int launch_batch_init(hipStream_t s, int nchunks, const BatchChunk* chunks, const double* b, double* x, double* r,
-                      double* part_rr, BatchState* st, int maxit);
-int launch_batch_update_p(hipStream_t s, int nchunks, const BatchChunk* chunks, const int2* rrRange, const double* r,
-                          double* p, const double* part_rr, BatchState* st, double tol);
-int launch_batch_update_xr(hipStream_t s, int nchunks, const BatchChunk* chunks, const int2* pApRange,
-                           const double* p, const double* Ap, double* x, double* r, const double* part_pAp,
-                           double* part_rr, BatchState* st);
-int launch_batch_gather(hipStream_t s, int nsupers, const BatchSuper* supers, const int* rowStarts,
-                        const int* colIds, const double* q, double* gq, const double* p, double* part,
-                        const BatchState* st);
+                      const BoxBatchProb* probs, double* part_rr, BatchState* st, double tol, int maxit);
 int launch_batch_count_done(hipStream_t s, int nprob, const BatchState* st, int* count);
 // quads, triangles and tetrahedra (ax_other.hip, FP64): bp 1..6 on the
 // [element][field][node] local vectors. Quads: W = wJ (BP5/6, per node) or
@@ -349,7 +332,8 @@ struct BoxBatchProb {
   BoxGrid g;
   long long off = 0;   // first row in the concatenated vectors
   long long loc = 0;   // first local node
-  long long el0 = 0;   // first element in the degree's coefficient array
+  long long el0 = 0;   // first element in the coefficient array
+  int tab = 0;             // its degree's GLL nodes, weights and even-odd table
   int pAp0 = 0, npAp = 0;  // partials of p.Ap (one per Ax workgroup)
   int rr0 = 0, ninit = 0, nrr = 0;  // partials of r.r: of the initial residual, of later ones
 };
@@ -394,11 +378,12 @@ struct BoxAxArgs {
   const double* hist_alpha = nullptr;
   CgState* st = nullptr;
   double tol = 0;
-  // a degree's problems of a batch (FP64, trilinear): nitems workgroups; the
-  // vectors, geo and the partials are the concatenated ones, p the other
-  // direction vector and the iteration, its scalars and flags the problem's
-  // state (q and p by the parity of its iteration)
+  // launch_box_batch_ax: nitems workgroups; the vectors, geo and the partials
+  // are the concatenated ones, tab the degrees' 1D data (BoxBatchProb::tab), p
+  // the other direction vector, and the iteration, its scalars and flags the
+  // problem's state (q and p by the parity of its iteration)
   int nitems = 0;
+  const T* tab = nullptr;
   const BoxBatchItem* items = nullptr;
   const BoxBatchProb* probs = nullptr;
   BatchState* bst = nullptr;
@@ -424,6 +409,24 @@ struct BoxUpdateR {
 };
 template <typename T>
 int launch_box_update_r(hipStream_t s, const BoxGrid& g, int F, const BoxUpdateR<T>& u, int* nrr);
+
+// both kernels for the problems of a batch (FP64, trilinear; box_batch.hip):
+// cls = box_batch_class of their degrees, whose items are launched together;
+// items hold box_ax_elements and box_gather_elements elements
+int box_batch_class(int N);
+int launch_box_batch_ax(hipStream_t s, int cls, const BoxAxArgs<double>& a);
+struct BoxBatchUpdate {
+  int nitems = 0;
+  const BoxBatchItem* items = nullptr;
+  const BoxBatchProb* probs = nullptr;
+  BatchState* st = nullptr;
+  const double* AqL = nullptr;
+  double* r = nullptr;
+  const double* part_pAp = nullptr;
+  double* part_rr = nullptr;
+};
+int box_gather_elements(int Nq);
+int launch_box_batch_update_r(hipStream_t s, int cls, const BoxBatchUpdate& u);
 
 // linAlg. Reductions run on a fixed grid of kRedBlocks workgroups and write
 // kRedBlocks FP64 partials; launch_fold sums partials into a device scalar.

@@ -1049,8 +1049,7 @@ int bpx_batch_tuning(bpx_batch b, double* out, int capacity) {
   const int n = 6 * (int)b->b.groups.size();
   for (size_t g = 0; g < b->b.groups.size(); ++g) {
     const auto& G = b->b.groups[g];
-    const double v[6] = {(double)G.N, (double)G.variant, (double)bp5_batch_epb(G.Nq, G.variant), G.us[0], G.us[1],
-                         G.us[2]};
+    const double v[6] = {(double)G.N, 0.0, (double)box_ax_elements(G.Nq), G.us, -1.0, -1.0};
     for (int k = 0; k < 6; ++k)
       if ((int)(6 * g + k) < capacity) out[6 * g + k] = v[k];
   }

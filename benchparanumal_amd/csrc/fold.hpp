@@ -1,9 +1,12 @@
-// Fixed-order sums of reduction partials (device code).
+// Fused multiply-adds and fixed-order sums of reduction partials (device code).
 #pragma once
 #include <hip/hip_runtime.h>
 
 namespace bpx {
 namespace {
+
+__device__ inline double fmad(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ inline float fmad(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
 // Sum of partials[0..n) in a fixed order, by one wavefront: lane l folds
 // l, l+64, ... into four accumulators (so its loads are in flight

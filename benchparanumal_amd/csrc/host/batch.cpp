@@ -27,6 +27,8 @@ bp_batch_t::~bp_batch_t() {
   if (graphExec) (void)hipGraphExecDestroy(graphExec);
   if (graphMixed) (void)hipGraphExecDestroy(graphMixed);
   if (h_count) (void)hipHostFree(h_count);
+  for (auto& e : evCount)
+    if (e) (void)hipEventDestroy(e);
   if (ev0) (void)hipEventDestroy(ev0);
   if (ev1) (void)hipEventDestroy(ev1);
   if (stream) (void)hipStreamDestroy(stream);
@@ -40,7 +42,8 @@ int bp_batch_t::Setup(platform_t& p, const std::vector<MeshOpts>& opts, dfloat l
   BPX_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
   BPX_HIP(hipEventCreateWithFlags(&ev0, hipEventDisableTiming));
   BPX_HIP(hipEventCreateWithFlags(&ev1, hipEventDisableTiming));
-  BPX_HIP(hipHostMalloc((void**)&h_count, sizeof(int), hipHostMallocDefault));
+  for (auto& e : evCount) BPX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  BPX_HIP(hipHostMalloc((void**)&h_count, 2 * sizeof(int), hipHostMallocDefault));
 
   // ---- per-problem host setup (bp5_t: mesh, masked ogs, GlobalToLocal)
   std::vector<mesh_t> meshes(nprob);
@@ -121,40 +124,53 @@ int bp_batch_t::Setup(platform_t& p, const std::vector<MeshOpts>& opts, dfloat l
     if (int st = G.D.upload(*D, s)) return st;
   }
 
-  // ---- the box kernels' tables: per degree the elements' map coefficients
-  // and the Ax workgroups, per problem its grid and offsets
+  // ---- the box kernels' tables: the elements' map coefficients and the
+  // degrees' 1D data, per problem its grid and offsets, per class of degrees
+  // the workgroups (high degrees first: theirs run longest)
   std::vector<BoxBatchProb> probs(nprob);
+  std::vector<double> geo, tab;
+  std::vector<BoxBatchItem> items[2], gitems[2];
+  std::vector<Group*> byDegree;
+  for (auto& G : groups) byDegree.push_back(&G);
+  std::sort(byDegree.begin(), byDegree.end(), [](const Group* a, const Group* b) { return a->N > b->N; });
   int npAp = 0;
-  for (auto& G : groups) {
-    const int epb = box_ax_elements(G.Nq);
-    std::vector<double> geo, eo;
-    std::vector<BoxBatchItem> items;
+  for (Group* G : byDegree) {
+    const int epb = box_ax_elements(G->Nq), gepb = box_gather_elements(G->Nq), cls = box_batch_class(G->N);
+    const int tab0 = (int)tab.size();
     const mesh_t* any = nullptr;
+    G->item0 = (int)items[cls].size();
     for (int i = 0; i < nprob; ++i) {
       const mesh_t& m = meshes[i];
-      if (m.N != G.N) continue;
+      if (m.N != G->N) continue;
       any = &m;
       BoxBatchProb& pr = probs[i];
       pr.g.set(m.opts.nx, m.opts.ny, m.opts.nz, m.N);
       pr.off = off[i];
       pr.loc = localOff[i];
       pr.el0 = (long long)geo.size() / 24;
+      pr.tab = tab0;
       pr.pAp0 = npAp;
       pr.npAp = (m.Nelements + epb - 1) / epb;
       npAp += pr.npAp;
       std::vector<double> c;
       m.TrilinearCoefficients(c);
       geo.insert(geo.end(), c.begin(), c.end());
-      for (dlong e = 0; e < m.Nelements; e += epb) items.push_back({i, (int)e});
+      for (dlong e = 0; e < m.Nelements; e += epb) items[cls].push_back({i, (int)e});
+      for (dlong e = 0; e < m.Nelements; e += gepb) gitems[cls].push_back({i, (int)e});
     }
+    G->nitems = (int)items[cls].size() - G->item0;
+    std::vector<double> eo;
     if (int st = box_even_odd_table(*any, eo)) return st;
-    if (int st = G.boxGeo.upload(geo, s)) return st;
-    if (int st = G.boxEo.upload(eo, s)) return st;
-    if (int st = G.boxZ.upload(any->gllz, s)) return st;
-    if (int st = G.boxW.upload(any->gllw, s)) return st;
-    if (int st = G.boxItems.upload(items, s)) return st;
+    tab.insert(tab.end(), any->gllz.begin(), any->gllz.end());
+    tab.insert(tab.end(), any->gllw.begin(), any->gllw.end());
+    tab.insert(tab.end(), eo.begin(), eo.end());
   }
-  if (int st = o_probs.upload(probs, s)) return st;
+  if (int st = o_boxGeo.upload(geo, s)) return st;
+  if (int st = o_boxTab.upload(tab, s)) return st;
+  for (int cls = 0; cls < 2; ++cls) {
+    if (int st = boxItems[cls].upload(items[cls], s)) return st;
+    if (int st = gatherItems[cls].upload(gitems[cls], s)) return st;
+  }
 
   // ---- concatenated gather maps, super-blocks and chunks
   std::vector<dlong> rowStarts(1, 0), colIds;
@@ -175,11 +191,23 @@ int bp_batch_t::Setup(platform_t& p, const std::vector<MeshOpts>& opts, dfloat l
     pApRange[i].y = (int)supers.size();
     rrRange[i].x = (int)chunks.size();
     const dlong n = o.Ngather;
-    if (n == 0) chunks.push_back({i, off[i], off[i], 1});  // still initialises the state
+    if (n == 0) chunks.push_back({i, off[i], off[i], 0});  // still initialises the state
     for (dlong c = 0; c < n; c += kChunk)
-      chunks.push_back({i, off[i] + c, off[i] + std::min<dlong>(c + kChunk, n), c == 0 ? 1 : 0});
+      chunks.push_back({i, off[i] + c, off[i] + std::min<dlong>(c + kChunk, n), c / kChunk});
     rrRange[i].y = (int)chunks.size();
   }
+  // r.r partials of the FP64 solve: per problem room for the chunks' of the
+  // initial residual and the gather workgroups' of the later ones
+  int nrr = 0;
+  for (int i = 0; i < nprob; ++i) {
+    BoxBatchProb& pr = probs[i];
+    const int epb = box_gather_elements(meshes[i].Nq);
+    pr.rr0 = nrr;
+    pr.ninit = rrRange[i].y - rrRange[i].x;
+    pr.nrr = (meshes[i].Nelements + epb - 1) / epb;
+    nrr += std::max(pr.ninit, pr.nrr);
+  }
+  if (int st = o_probs.upload(probs, s)) return st;
   nsupers = (int)supers.size();
   nchunks = (int)chunks.size();
   if (int st = o_rowStarts.upload(rowStarts, s)) return st;
@@ -193,8 +221,9 @@ int bp_batch_t::Setup(platform_t& p, const std::vector<MeshOpts>& opts, dfloat l
   if (int st = o_p.alloc(std::max<dlong>(Ntot, 1))) return st;
   if (int st = o_Ap.alloc(std::max<dlong>(Ntot, 1))) return st;
   if (int st = o_AqL.alloc(std::max<dlong>(NLocalTot, 1))) return st;
-  if (int st = o_part_rr.alloc(std::max(nchunks, 1))) return st;
-  if (int st = o_part_pAp.alloc(std::max(nsupers, 1))) return st;
+  if (int st = o_x.alloc(std::max<dlong>(Ntot, 1))) return st;
+  if (int st = o_part_rr.alloc(std::max({nchunks, nrr, 1}))) return st;
+  if (int st = o_part_pAp.alloc(std::max({nsupers, npAp, 1}))) return st;
   if (int st = o_count.alloc(1)) return st;
   BPX_HIP(hipMemsetAsync(o_state.ptr(), 0, sizeof(BatchState) * nprob, s));
   BPX_HIP(hipMemsetAsync(o_p.ptr(), 0, sizeof(double) * std::max<dlong>(Ntot, 1), s));
@@ -202,91 +231,81 @@ int bp_batch_t::Setup(platform_t& p, const std::vector<MeshOpts>& opts, dfloat l
   return Tune();
 }
 
-int bp_batch_t::AxGroup(const Group& G, int variant, const double* q, double* AqL) const {
-  return launch_bp5_batch(stream, G.N, variant, (int)G.Nel, G.elementList.ptr(), G.G2L.ptr(), G.wJ.ptr(),
-                          G.ggeo.ptr(), G.D.ptr(), lambda, q, AqL + G.loff, G.elemPid.ptr(), o_state.ptr());
-}
-
-// the box kernels' Ax of one degree's problems that their states do not skip
-BoxAxArgs<double> bp_batch_t::BoxArgs(const Group& G, const double* q) {
+// the Ax of the problems that their states do not skip
+BoxAxArgs<double> bp_batch_t::BoxArgs(int cls, const double* q, int item0, int nitems) {
   BoxAxArgs<double> a;
-  a.g.N = G.N;
-  a.geo = G.boxGeo.ptr();
-  a.z = G.boxZ.ptr();
-  a.w = G.boxW.ptr();
-  a.eo = G.boxEo.ptr();
+  a.geo = o_boxGeo.ptr();
+  a.tab = o_boxTab.ptr();
   a.lambda = lambda;
   a.q = q;
   a.AqL = o_AqL.ptr();
-  a.nitems = (int)G.boxItems.length();
-  a.items = G.boxItems.ptr();
+  a.nitems = nitems < 0 ? (int)boxItems[cls].length() : nitems;
+  a.items = boxItems[cls].ptr() + item0;
   a.probs = o_probs.ptr();
   a.bst = o_state.ptr();
   return a;
 }
 
-// Times every workgroup shape of each degree group's Ax on the group's own
-// elements (all variants give identical results) and keeps the fastest.
+// Times each degree's Ax (the box kernel has one workgroup shape)
 int bp_batch_t::Tune() {
   hipEvent_t t0, t1;
   BPX_HIP(hipEventCreate(&t0));
-  BPX_HIP(hipEventCreate(&t1));
+  if (hipEventCreate(&t1) != hipSuccess) {
+    (void)hipEventDestroy(t0);
+    return set_error(BPX_ERR_HIP, "batch tune: event create failed");
+  }
   int st = BPX_OK;
   for (auto& G : groups) {
-    float best = 1e30f;
-    G.variant = 0;
-    for (int v = 0; v < 3 && st == BPX_OK; ++v) {
-      G.us[v] = -1;
-      if (bp5_batch_epb(G.Nq, v) == 0) continue;
-      if ((st = AxGroup(G, v, o_p.ptr(), o_AqL.ptr()))) break;  // warm-up
-      float ms = 1e30f;
-      for (int rep = 0; rep < 3 && st == BPX_OK; ++rep) {
-        float t = 0;
-        if (hipEventRecord(t0, stream) != hipSuccess || (st = AxGroup(G, v, o_p.ptr(), o_AqL.ptr())) ||
-            hipEventRecord(t1, stream) != hipSuccess || hipEventSynchronize(t1) != hipSuccess ||
-            hipEventElapsedTime(&t, t0, t1) != hipSuccess) {
-          if (!st) st = set_error(BPX_ERR_HIP, "batch tune: event timing failed");
-          break;
-        }
-        ms = std::min(ms, t);
-      }
-      G.us[v] = ms * 1e3;
-      if (ms < best) {
-        best = ms;
-        G.variant = v;
-      }
+    const int cls = box_batch_class(G.N);
+    const BoxAxArgs<double> a = BoxArgs(cls, o_p.ptr(), G.item0, G.nitems);
+    if ((st = launch_box_batch_ax(stream, cls, a))) break;  // warm-up
+    float ms = 0;
+    if (hipEventRecord(t0, stream) != hipSuccess || (st = launch_box_batch_ax(stream, cls, a)) ||
+        hipEventRecord(t1, stream) != hipSuccess || hipEventSynchronize(t1) != hipSuccess ||
+        hipEventElapsedTime(&ms, t0, t1) != hipSuccess) {
+      if (!st) st = set_error(BPX_ERR_HIP, "batch tune: event timing failed");
+      break;
     }
-    if (st) break;
+    G.us = ms * 1e3;
   }
   (void)hipEventDestroy(t0);
   (void)hipEventDestroy(t1);
   return st;
 }
 
-// One CG iteration for every problem still running (queued on `stream`).
-int bp_batch_t::Iteration(double* o_x, double tol) {
-  BatchState* stt = o_state.ptr();
-  if (int st = launch_batch_update_p(stream, nchunks, o_chunks.ptr(), o_rrRange.ptr(), o_r.ptr(), o_p.ptr(),
-                                     o_part_rr.ptr(), stt, tol))
-    return st;
-  for (const auto& G : groups)
-    if (int st = AxGroup(G, G.variant, o_p.ptr(), o_AqL.ptr())) return st;
-  if (int st = launch_batch_gather(stream, nsupers, o_supers.ptr(), o_rowStarts.ptr(), o_colIds.ptr(), o_AqL.ptr(),
-                                   o_Ap.ptr(), o_p.ptr(), o_part_pAp.ptr(), stt))
-    return st;
-  return launch_batch_update_xr(stream, nchunks, o_chunks.ptr(), o_pApRange.ptr(), o_p.ptr(), o_Ap.ptr(), o_x,
-                                o_r.ptr(), o_part_pAp.ptr(), o_part_rr.ptr(), stt);
+// One CG iteration of the problems still running
+int bp_batch_t::Iteration() {
+  for (int cls = 0; cls < 2; ++cls) {
+    BoxAxArgs<double> a = BoxArgs(cls, o_p.ptr());
+    a.fold = 1;
+    a.p = o_Ap.ptr();  // the second direction (Ap itself is never stored)
+    a.r = o_r.ptr();
+    a.x = o_x.ptr();
+    a.part = o_part_pAp.ptr();
+    a.part_rr = o_part_rr.ptr();
+    if (int st = launch_box_batch_ax(stream, cls, a)) return st;
+    BoxBatchUpdate u;
+    u.nitems = (int)gatherItems[cls].length();
+    u.items = gatherItems[cls].ptr();
+    u.probs = o_probs.ptr();
+    u.st = o_state.ptr();
+    u.AqL = o_AqL.ptr();
+    u.r = o_r.ptr();
+    u.part_pAp = o_part_pAp.ptr();
+    u.part_rr = o_part_rr.ptr();
+    if (int st = launch_box_batch_update_r(stream, cls, u)) return st;
+  }
+  return BPX_OK;
 }
 
-int bp_batch_t::Capture(double* o_x, double tol) {
-  if (graphExec && graphX == o_x && graphTol == tol) return BPX_OK;
-  if (graphExec) {
-    (void)hipGraphExecDestroy(graphExec);
-    graphExec = nullptr;
-  }
+// kGraphIters iterations and the count of finished problems. The solution
+// and the tolerance are the batch's own memory, so one graph serves every
+// call.
+int bp_batch_t::Capture() {
+  if (graphExec) return BPX_OK;
   BPX_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
   int st = BPX_OK;
-  for (int k = 0; k < kGraphIters && st == BPX_OK; ++k) st = Iteration(o_x, tol);
+  for (int k = 0; k < kGraphIters && st == BPX_OK; ++k) st = Iteration();
   if (st == BPX_OK) st = launch_batch_count_done(stream, nprob, o_state.ptr(), o_count.ptr());
   hipGraph_t graph = nullptr;
   const hipError_t e = hipStreamEndCapture(stream, &graph);
@@ -301,8 +320,6 @@ int bp_batch_t::Capture(double* o_x, double tol) {
     graphExec = nullptr;
     return hip_error(e2, "hipGraphInstantiate");
   }
-  graphX = o_x;
-  graphTol = tol;
   return BPX_OK;
 }
 
@@ -313,21 +330,27 @@ int bp_batch_t::Solve(double* o_x, const double* o_b, double tol, int maxit, int
   // order after the caller's work on the platform stream
   BPX_HIP(hipEventRecord(ev0, platform->stream));
   BPX_HIP(hipStreamWaitEvent(stream, ev0, 0));
-  if (int st = launch_batch_init(stream, nchunks, o_chunks.ptr(), o_b, o_x, o_r.ptr(), o_part_rr.ptr(),
-                                 o_state.ptr(), maxit))
+  if (int st = launch_batch_init(stream, nchunks, o_chunks.ptr(), o_b, this->o_x.ptr(), o_r.ptr(), o_probs.ptr(),
+                                 o_part_rr.ptr(), o_state.ptr(), tol, maxit))
     return st;
-  if (int st = Capture(o_x, tol)) return st;
+  if (int st = Capture()) return st;
   // every replay runs kGraphIters iterations of the problems still going;
   // maxit/kGraphIters + 1 replays let the last one reach its cap and stop
   const long long maxReplays = (long long)maxit / kGraphIters + 2;
   replays = 0;
+  // the count of replay rep is read while replay rep + 1 runs (a replay past
+  // the end finds every problem done and does nothing)
   for (long long rep = 0; rep < maxReplays; ++rep) {
     BPX_HIP(hipGraphLaunch(graphExec, stream));
-    BPX_HIP(hipMemcpyAsync(h_count, o_count.ptr(), sizeof(int), hipMemcpyDeviceToHost, stream));
-    BPX_HIP(hipStreamSynchronize(stream));
+    BPX_HIP(hipMemcpyAsync(h_count + (rep & 1), o_count.ptr(), sizeof(int), hipMemcpyDeviceToHost, stream));
+    BPX_HIP(hipEventRecord(evCount[rep & 1], stream));
     ++replays;
-    if (*h_count >= nprob) break;
+    if (rep == 0) continue;
+    BPX_HIP(hipEventSynchronize(evCount[(rep - 1) & 1]));
+    if (h_count[(rep - 1) & 1] >= nprob) break;
   }
+  if (Ntot > 0)
+    BPX_HIP(hipMemcpyAsync(o_x, this->o_x.ptr(), (size_t)Ntot * sizeof(double), hipMemcpyDeviceToDevice, stream));
   std::vector<BatchState> hs(nprob);
   BPX_HIP(hipMemcpy(hs.data(), o_state.ptr(), sizeof(BatchState) * nprob, hipMemcpyDeviceToHost));
   int anyBreak = 0;
@@ -398,8 +421,8 @@ int bp_batch_t::Segment(double* o_x, const double* o_b, double tol, int interval
       return st;
   }
   if (int st = launch_bm_flush(stream, nchunks, o_chunks.ptr(), o_c32.ptr(), o_x, out)) return st;
-  for (const auto& G : groups)
-    if (int st = launch_box_ax<double>(stream, BoxArgs(G, o_x))) return st;  // (the outer states are o_state)
+  for (int cls = 0; cls < 2; ++cls)  // (the outer states are o_state)
+    if (int st = launch_box_batch_ax(stream, cls, BoxArgs(cls, o_x))) return st;
   if (int st = launch_batch_gather_only(stream, nsupers, o_supers.ptr(), o_rowStarts.ptr(), o_colIds.ptr(),
                                         o_AqL.ptr(), o_Ax64.ptr(), out))
     return st;

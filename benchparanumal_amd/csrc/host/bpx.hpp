@@ -636,11 +636,8 @@ class bp_batch_t {
     deviceBuffer<dlong> elementList, G2L, elemPid;
     deviceBuffer<double> wJ, ggeo, D;
     deviceBuffer<float> wJ32, ggeo32, D32;  // rounded to FP32 for the mixed solve
-    // the FP64 operator on the box kernels: map coefficients, 1D data, workgroups
-    deviceBuffer<double> boxGeo, boxZ, boxW, boxEo;
-    deviceBuffer<BoxBatchItem> boxItems;
-    int variant = 0;             // workgroup shape chosen by the tuner
-    double us[3] = {-1, -1, -1};  // its timings (us; -1 = shape not available)
+    double us = -1;  // its FP64 Ax, timed at setup
+    int item0 = 0, nitems = 0;  // its Ax workgroups in boxItems[box_batch_class(N)]
   };
   platform_t* platform = nullptr;
   dfloat lambda = 1.0;
@@ -652,11 +649,15 @@ class bp_batch_t {
 
  private:
   int Tune();
-  int AxGroup(const Group& G, int variant, const double* q, double* AqL) const;
-  BoxAxArgs<double> BoxArgs(const Group& G, const double* q);
+  // the FP64 operator on the box kernels: per class of degrees its workgroups
+  // (item0.., nitems of them; nitems < 0: all), and for all problems the map
+  // coefficients and the degrees' 1D data
+  BoxAxArgs<double> BoxArgs(int cls, const double* q, int item0 = 0, int nitems = -1);
+  deviceBuffer<BoxBatchItem> boxItems[2], gatherItems[2];
+  deviceBuffer<double> o_boxGeo, o_boxTab;
   deviceBuffer<BoxBatchProb> o_probs;
-  int Iteration(double* o_x, double tol);
-  int Capture(double* o_x, double tol);
+  int Iteration();
+  int Capture();
   int Prepare32();
   int Segment(double* o_x, const double* o_b, double tol, int interval);
   int CaptureMixed(double* o_x, const double* o_b, double tol, int interval);
@@ -670,17 +671,15 @@ class bp_batch_t {
   deviceBuffer<double> o_Ax64, o_part_true;
   deviceBuffer<BatchState> o_inner;
   hipStream_t stream = nullptr;
-  hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  int* h_count = nullptr;
+  hipEvent_t ev0 = nullptr, ev1 = nullptr, evCount[2] = {nullptr, nullptr};
+  int* h_count = nullptr;  // pinned, two entries
   hipGraphExec_t graphExec = nullptr;
-  double* graphX = nullptr;
-  double graphTol = -1;
   deviceBuffer<dlong> o_rowStarts, o_colIds;
   deviceBuffer<BatchSuper> o_supers;
   deviceBuffer<BatchChunk> o_chunks;
   deviceBuffer<int2> o_pApRange, o_rrRange;
   deviceBuffer<BatchState> o_state;
-  deviceBuffer<double> o_r, o_p, o_Ap, o_AqL, o_part_rr, o_part_pAp;
+  deviceBuffer<double> o_x, o_r, o_p, o_Ap, o_AqL, o_part_rr, o_part_pAp;
   deviceBuffer<int> o_count;
 };
 

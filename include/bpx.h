@@ -507,10 +507,9 @@ int bpx_bp_time_operator_in_solve(bpx_bp b, double* o_x, const double* o_b, doub
  * 29-95), solved together by one CG per problem (the recurrence of
  * cg::Solve, libs/core/linearSolverCG.cpp:62-129) whose scalars stay on the
  * device; blocks of iterations are captured once in a hipGraph and
- * replayed until every problem has stopped. Problems of one degree share one
- * Ax launch; the setup times the workgroup shapes of each degree's Ax (all
- * give identical results) and keeps the fastest. Vectors are the problems'
- * global vectors concatenated in order (bpx_batch_offsets). */
+ * replayed until every problem has stopped. Problems of degrees up to 8
+ * share two launches per iteration, those above two more. Vectors are the
+ * problems' global vectors concatenated in order (bpx_batch_offsets). */
 int bpx_batch_create(bpx_platform p, int nprob, const bpx_mesh_opts* opts, double lambda,
                      bpx_batch* out);
 int bpx_batch_destroy(bpx_batch b);
@@ -518,8 +517,8 @@ int bpx_batch_destroy(bpx_batch b);
 int bpx_batch_info(bpx_batch b, int64_t* out, int capacity);
 /* off[0..nprob]: problem i owns [off[i], off[i+1]) of the vectors */
 int bpx_batch_offsets(bpx_batch b, int64_t* off);
-/* per degree group, 6 values: N, chosen shape, elements per workgroup,
- * time (us) of shapes 0, 1, 2 (-1 = not available). Returns the count. */
+/* per degree group, 6 values: N, workgroup shape (0: there is one), elements
+ * per workgroup, time (us) of its FP64 Ax, -1, -1. Returns the count. */
 int bpx_batch_tuning(bpx_batch b, double* out, int capacity);
 /* x_i = A_i^{-1} b_i to ||r_i|| <= max(tol ||b_i||, tol) or maxit
  * iterations, x from 0. iterations, rnorm: host arrays of nprob (may be
