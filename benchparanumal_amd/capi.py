@@ -361,7 +361,8 @@ class BP:
         check(lib().bpx_bp_set_cg_fold(self.h, int(mask)))
 
     def set_ax_engine(self, engine):
-        """BP5 at N = 15, FP64: 0 = auto (matrix cores), 1 = vector-ALU Ax,
+        """BP5 at N = 15, FP64, the kernels that read stored factors (ax_local
+        and solves with tol = 0): 0 = auto (matrix cores), 1 = vector-ALU Ax,
         2 = matrix-core Ax (the two agree to rounding, not bit for bit)."""
         check(lib().bpx_bp_set_ax_engine(self.h, int(engine)))
 

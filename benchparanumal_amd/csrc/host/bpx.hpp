@@ -418,8 +418,10 @@ class bp_t : public solver_t {
     double fused32_us = -1, unfused32_us = -1;
   } tuning;
   int Tune32();
-  // BP5, one field, N = 15, FP64: where the r and s contractions run
-  // (AX_ENGINE_AUTO: the matrix cores; see AxArgs::engine)
+  // BP5, one field, N = 15, FP64: where the r and s contractions of the
+  // stored-factor Ax run (AX_ENGINE_AUTO: the matrix cores; see
+  // AxArgs::engine). The box operator has them even-odd on the vector ALU,
+  // half of the multiply-adds at the same FP64 rate.
   int axEngine = AX_ENGINE_AUTO;
   // BP1-BP4 non-affine at Nq <= 8: pencil or wavefront-per-element kernels
   int cubForm = CUB_FORM_AUTO;
@@ -458,8 +460,10 @@ class bp_t : public solver_t {
   // solves, bit 1 for the FP32 iterations of the mixed solve
   int cgFold = 3;
   int OperatorDotUnfusedS(const dfloat* o_q, dfloat* o_Aq, double* part, int* npart);
-  // Ax into the local vector
+  // Ax into the local vector: as the caller's kernel choices have it, and as
+  // the operator applies it
   int AxLocal(const dfloat* o_q, dfloat* o_AqL);
+  int AxOperator(const dfloat* o_q, dfloat* o_AqL);
   // the same from the stored factors; G2L = the GlobalToLocal map to read q
   // through (default: the reference rows)
   int AxStored(const dfloat* o_q, dfloat* o_AqL, const dlong* G2L = nullptr);
@@ -495,7 +499,8 @@ class bp_t : public solver_t {
   BoxGrid box;
   // BP5 and BP6 on the box: the geometry formed in the kernel from the
   // elements' trilinear maps (or their affine factors), no index maps
-  // (box_ax.hip). BP5 at N = 15 in FP64 keeps the stored factors.
+  // (box_ax.hip). At p = 15 the stored-factor kernel reads 76 bytes per node
+  // and no cache holds them: 24^3, operator 1034 -> 534 us.
   bool boxAx = false;
   deviceBuffer<double> o_boxGeo, o_boxZ, o_boxEo, o_kappa;
   deviceBuffer<float> o_boxEo32;

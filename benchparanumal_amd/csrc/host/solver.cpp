@@ -437,7 +437,7 @@ int bp_t::Setup(platform_t& p, mesh_t& m, int bp_, dfloat lambda_) {
     if (!eo.empty())
       if (int st = o_eo.upload(eo, s)) return st;
   }
-  boxAx = haveBox && (bp == 6 || (bp == 5 && m.N < 15));
+  boxAx = haveBox && (bp == 5 || bp == 6);
   if (boxAx) {
     std::vector<double> eo;
     if (int st = box_even_odd_table(m, eo)) return st;
@@ -532,6 +532,13 @@ BoxAxArgs<T> bp_t::BoxArgs(const T* o_q, T* o_AqL) const {
 }
 
 int bp_t::AxLocal(const dfloat* o_q, dfloat* o_AqL) {
+  // BP5 at N = 15 has a choice of engine (AxArgs::engine), which the
+  // stored-factor kernels offer
+  if (bp == 5 && mesh->N == 15 && !haveKappa) return AxStored(o_q, o_AqL);
+  return AxOperator(o_q, o_AqL);
+}
+
+int bp_t::AxOperator(const dfloat* o_q, dfloat* o_AqL) {
   if (boxAx) return launch_box_ax<double>(platform->stream, BoxArgs<double>(o_q, o_AqL));
   return AxStored(o_q, o_AqL);
 }
@@ -607,7 +614,7 @@ int bp_t::Operator(const dfloat* o_q, dfloat* o_Aq) {
   // with no halo one launch covers every element
   if (int st = gHalo.ExchangeStart(o_q, 1)) return st;
   if (int st = gHalo.ExchangeFinish(o_q, 1)) return st;
-  if (int st = AxLocal(o_q, o_AqL.ptr())) return st;
+  if (int st = AxOperator(o_q, o_AqL.ptr())) return st;
   return GatherLocal<double>(o_AqL.ptr(), o_Aq);
 }
 
@@ -950,7 +957,7 @@ int bp_t::TimeKrhs(int K, int chunk, int launches, const dfloat* o_q, double* ou
   }
   if (int st = A.alloc((size_t)NLocal * K)) return st;
   // K right-hand sides at once, then one right-hand side per launch
-  auto run = [&](int form) { return form == 0 ? AxLocalKrhs(K, o_q, A.ptr(), chunk) : AxLocal(o_q, A.ptr()); };
+  auto run = [&](int form) { return form == 0 ? AxLocalKrhs(K, o_q, A.ptr(), chunk) : AxOperator(o_q, A.ptr()); };
   std::vector<hipEvent_t> ev(4 * (size_t)launches, nullptr);
   int st = BPX_OK;
   for (auto& e : ev)

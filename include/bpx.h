@@ -387,8 +387,11 @@ int bpx_bp_set_fp32_geometry(bpx_bp b, int mode);
 /* No reference counterpart: where the BP5 Ax at N = 15 in FP64 (one field)
  * runs its r and s contractions: 0 = auto (the matrix cores; default), 1 =
  * vector ALU, 2 = matrix cores (BPX_ERR_UNSUPPORTED for other problems).
- * Covers the plain and the fused (CG) form; the two engines agree to
- * rounding, not bit for bit. Other problems run on the vector ALU. */
+ * Covers the kernels that read stored factors: bpx_bp_ax_local and the
+ * solves with tol = 0, plain and fused; the two engines agree to rounding,
+ * not bit for bit. The operator and the solves to a tolerance form the
+ * factors from the elements' trilinear maps and run on the vector ALU at
+ * either setting, as other problems do. */
 int bpx_bp_set_ax_engine(bpx_bp b, int engine);
 /* No reference counterpart (launch choice): which kernel runs the BP1-BP4
  * Ax of a problem object on non-affine meshes at N <= 7: 0 = auto (the

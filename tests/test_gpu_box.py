@@ -35,9 +35,13 @@ BOXES = [(N, 3, 2, 2) for N in range(1, 16)] + [(1, 2, 2, 2), (1, 23, 9, 7), (2,
 @pytest.mark.parametrize("N,nx,ny,nz", BOXES)
 def test_box_gather_equals_map_gather(plat, N, nx, ny, nz, bp):
     """The operator's gather equals the ogs map gather of the local Ax bit
-    for bit, one and three fields (the copies are summed in the same order)."""
+    for bit, one and three fields (the copies are summed in the same order).
+    BP5 at N = 15, whose local Ax has kernels of its own: with a coefficient,
+    where both run the operator's kernel."""
     m = capi.Mesh(N=N, nx=nx, ny=ny, nz=nz, perturb=0.1, seed=3)
     b = capi.BP(plat, m, bp, lam=1.1)
+    if bp == 5 and N == 15:
+        b.set_kappa(torch.ones(b.Nnodes, dtype=torch.float64, device="cuda"))
     q = normal(N, b.Ngather)
     Aq, ref = torch.full((2, b.Ngather), float("nan"), dtype=torch.float64, device="cuda")
     b.operator(q, Aq)
@@ -148,7 +152,8 @@ def test_fixed_count_after_tolerance_solve(plat):
     np.testing.assert_array_equal(out[0][1], out[2][1])
 
 
-@pytest.mark.parametrize("N,affine", [(1, False), (2, True), (4, False), (8, False), (12, True), (14, False)])
+@pytest.mark.parametrize("N,affine", [(1, False), (2, True), (4, False), (8, False), (12, True), (14, False), (15, False),
+                                      (15, True)])
 def test_box_kappa_operator(plat, N, affine):
     """The variable coefficient read from the lattice, against the oracle."""
     m, P = pair(5, N, 3, 2, 2, affine=affine, lam=0.4)
