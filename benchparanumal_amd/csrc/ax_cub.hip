@@ -22,6 +22,7 @@
 
 #include "ax_common.hpp"
 #include "buffer_rsrc.hpp"
+#include "even_odd.hpp"
 
 #ifndef BPX_NQ
 #error "compile with -DBPX_NQ=<Nq>"
@@ -737,93 +738,6 @@ __global__ __launch_bounds__(128) void k_bp3_wave(int Nelements, const int* __re
 // form adds in their order). q is gathered through a bounds-checked buffer
 // resource: a masked node (G2L = -1) or an idle slot reads 0 without a
 // compare or select per load; BP2 gathers and stores in node order.
-template <typename T>
-__device__ inline T cfma(T a, T b, T c) {
-  if constexpr (sizeof(T) == 8)
-    return __builtin_fma(a, b, c);
-  else
-    return __builtin_fmaf(a, b, c);
-}
-
-// rows of a uniform R x C row-major matrix through scalar registers, row
-// n + 1 requested while row n is in use: body(n, row) for n = 0..R-1. The
-// opaque update of the pointer before each row keeps the compiler from
-// holding the whole matrix in scalar registers.
-template <int R, int C, typename T, typename F>
-__device__ inline void uniform_rows(const T* M, F&& body) {
-  typedef const __attribute__((address_space(4))) T* cptr;
-  cptr Mc = (cptr)M;
-  T d[2][C];
-  asm volatile("" : "+s"(Mc));
-#pragma unroll
-  for (int m = 0; m < C; ++m) d[0][m] = Mc[m];
-#pragma unroll
-  for (int n = 0; n < R; ++n) {
-    if (n + 1 < R) {
-      __builtin_amdgcn_sched_barrier(0);
-      asm volatile("" : "+s"(Mc));
-#pragma unroll
-      for (int m = 0; m < C; ++m) d[(n + 1) & 1][m] = Mc[(n + 1) * C + m];
-    }
-    body(n, d[n & 1]);
-  }
-}
-
-// Even-odd form of y = A x for a 1D operator A (N x M) with A[N-1-n][M-1-m]
-// = SIGN * A[n][m] (the interpolation matrix between symmetric point sets
-// and its transpose: SIGN = 1; the derivative on symmetric points and its
-// transpose: SIGN = -1). With xe[m] = x[m] + x[M-1-m], xo[m] = x[m] -
-// x[M-1-m] (m < M/2) and Ae = (A[n][m] + A[n][M-1-m]) / 2, Ao = (A[n][m] -
-// A[n][M-1-m]) / 2: ye[n] = Ae xe (+ A[n][M/2] x[M/2] for odd M), yo[n] =
-// Ao xo, y[n] = ye + yo and y[N-1-n] = SIGN (ye - yo), which halves the
-// multiply-adds (Kopriva's even-odd decomposition). Table row n (n <=
-// (N-1)/2): Ae[n][0..M/2-1], A[n][M/2] (odd M), Ao[n][0..M/2-1]; in the
-// middle row of an odd N only the part that does not vanish is used.
-template <int N, int M>
-struct EoShape {
-  static constexpr int hM = M / 2, oM = M & 1, LE = hM + oM, RL = LE + hM;
-  static constexpr int hN = N / 2, oN = N & 1, rows = hN + oN, size = rows * RL;
-};
-
-template <int N, int M, int SIGN, typename T, typename P>
-__device__ inline void eo_apply(const T* tab, const T (&x)[M], P&& put) {  // put(n, y[n])
-  using E = EoShape<N, M>;
-  T xe[E::hM > 0 ? E::hM : 1], xo[E::hM > 0 ? E::hM : 1];
-#pragma unroll
-  for (int m = 0; m < E::hM; ++m) {
-    xe[m] = x[m] + x[M - 1 - m];
-    xo[m] = x[m] - x[M - 1 - m];
-  }
-  uniform_rows<E::rows, E::RL>(tab, [&](int n, const T* r) {
-    const bool mid = E::oN && n == E::hN;
-    T ye = 0, yo = 0;
-    if (!mid || SIGN > 0) {
-#pragma unroll
-      for (int m = 0; m < E::hM; ++m) ye = cfma(r[m], xe[m], ye);
-      if constexpr (E::oM) ye = cfma(r[E::hM], x[E::hM], ye);
-    }
-    if (!mid || SIGN < 0) {
-#pragma unroll
-      for (int m = 0; m < E::hM; ++m) yo = cfma(r[E::LE + m], xo[m], yo);
-    }
-    if (mid) {
-      put(n, SIGN > 0 ? ye : yo);
-    } else {
-      put(n, ye + yo);
-      put(N - 1 - n, SIGN > 0 ? ye - yo : yo - ye);
-    }
-  });
-}
-
-// offsets of the four tables in the kernel's even-odd array: I (MQ x NQ),
-// I^T, D (MQ x MQ, the cubature derivative) and D^T
-template <int NQ>
-struct EoTables {
-  static constexpr int MQ = NQ + 1;
-  static constexpr int I = 0, IT = I + EoShape<MQ, NQ>::size, D = IT + EoShape<NQ, MQ>::size,
-                       DT = D + EoShape<MQ, MQ>::size, size = DT + EoShape<MQ, MQ>::size;
-};
-
 template <int MQ>
 constexpr int pencil_slots() {
   return MQ * MQ >= 256 ? 1 : 256 / (MQ * MQ);
@@ -966,7 +880,7 @@ k_cub_pencil(int Nelements, const int* __restrict__ elementList, const int* __re
       uniform_rows<MQ, NQ>(I, [&](int n, const T* r) {
         T acc = 0;
 #pragma unroll
-        for (int m = 0; m < NQ; ++m) acc = cfma(r[m], x[m], acc);
+        for (int m = 0; m < NQ; ++m) acc = fmad(r[m], x[m], acc);
         y[n] = acc;
       });
     }
@@ -979,7 +893,7 @@ k_cub_pencil(int Nelements, const int* __restrict__ elementList, const int* __re
       for (int n = 0; n < NQ; ++n) y[n] = T(0);
       uniform_rows<MQ, NQ>(I, [&](int m, const T* r) {
 #pragma unroll
-        for (int n = 0; n < NQ; ++n) y[n] = cfma(r[n], x[m], y[n]);
+        for (int n = 0; n < NQ; ++n) y[n] = fmad(r[n], x[m], y[n]);
       });
     }
   };
@@ -1148,7 +1062,7 @@ k_cub_pencil(int Nelements, const int* __restrict__ elementList, const int* __re
         uniform_rows<MQ, MQ>(Dq, [&](int n, const T* r) {
           T acc = 0;
 #pragma unroll
-          for (int m = 0; m < MQ; ++m) acc = cfma(r[m], v[m], acc);
+          for (int m = 0; m < MQ; ++m) acc = fmad(r[m], v[m], acc);
           dst[n * ls] = acc;
         });
       }
@@ -1164,7 +1078,7 @@ k_cub_pencil(int Nelements, const int* __restrict__ elementList, const int* __re
         for (int n = 0; n < MQ; ++n) o[n] = T(0);
         uniform_rows<MQ, MQ>(Dq, [&](int m, const T* r) {
 #pragma unroll
-          for (int n = 0; n < MQ; ++n) o[n] = cfma(r[n], v[m], o[n]);
+          for (int n = 0; n < MQ; ++n) o[n] = fmad(r[n], v[m], o[n]);
         });
       }
 #pragma unroll
@@ -1195,7 +1109,7 @@ k_cub_pencil(int Nelements, const int* __restrict__ elementList, const int* __re
       uniform_rows<MQ, MQ>(Dq, [&](int g, const T* r) {
         T ut = 0;
 #pragma unroll
-        for (int m = 0; m < MQ; ++m) ut = cfma(r[m], u[m], ut);
+        for (int m = 0; m < MQ; ++m) ut = fmad(r[m], u[m], ut);
         const T us = Bt[tp + g * PS];
         T gg[7];
         if (g < PF) {
@@ -1208,12 +1122,12 @@ k_cub_pencil(int Nelements, const int* __restrict__ elementList, const int* __re
           gg[6] = geo_load<SG>(W + cb);
         }
         const T G00 = gg[0], G01 = gg[1], G02 = gg[2], G11 = gg[3], G12 = gg[4], G22 = gg[5], WW = gg[6];
-        At[tp + g * PS] = cfma(G02, ut, cfma(G01, us, G00 * ur[g]));
-        Bt[tp + g * PS] = cfma(G12, ut, cfma(G11, us, G01 * ur[g]));
-        const T Gt = cfma(G22, ut, cfma(G12, us, G02 * ur[g]));
-        res[g] = cfma(lambda * WW, u[g], res[g]);
+        At[tp + g * PS] = fmad(G02, ut, fmad(G01, us, G00 * ur[g]));
+        Bt[tp + g * PS] = fmad(G12, ut, fmad(G11, us, G01 * ur[g]));
+        const T Gt = fmad(G22, ut, fmad(G12, us, G02 * ur[g]));
+        res[g] = fmad(lambda * WW, u[g], res[g]);
 #pragma unroll
-        for (int m = 0; m < MQ; ++m) res[m] = cfma(r[m], Gt, res[m]);
+        for (int m = 0; m < MQ; ++m) res[m] = fmad(r[m], Gt, res[m]);
       });
     }
     __syncthreads();

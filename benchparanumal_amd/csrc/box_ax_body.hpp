@@ -27,20 +27,10 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#include "box_common.hpp"
-#include "buffer_rsrc.hpp"
-#include "fold.hpp"
+#include "box_lanes.hpp"
 
 namespace bpx {
 namespace {
-
-// 1/x: FP32 by the hardware (1 ulp), FP64 by two Newton steps on it
-__device__ inline float reciprocal(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ inline double reciprocal(double x) {
-  double y = __builtin_amdgcn_rcp(x);
-  y = fmad(fmad(-x, y, 1.0), y, y);
-  return fmad(fmad(-x, y, 1.0), y, y);
-}
 
 // y = D x (or D^T x) from the even-odd table: row n <= (NQ-1)/2 holds
 // S[n][m] = (D[n][m] + D[n][NQ-1-m])/2 for m < NQ/2, D[n][NQ/2] for odd NQ,
@@ -154,14 +144,6 @@ __device__ inline void element_sync() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// MODE_FOLD: the direction update of a CG iteration and the x update of the
-// one before inside the Ax. Every element forms the new direction of all its
-// nodes from r and the old one (neighbours form the same bits), the owner
-// writes it, to another vector. An iteration is then this kernel and
-// k_box_update_r: at 24^3, p = 7 FP32 76 -> 54 us against four kernels with
-// k_bp5_ax, at 10^3, p = 4 affine FP64 23 -> 13 us.
-enum { MODE_PLAIN = 0, MODE_DOT = 1, MODE_FOLD = 2 };
-
 // GEO: where the factors come from
 enum { GEO_TRILINEAR = 0, GEO_AFFINE = 1, GEO_STORED = 2 };
 
@@ -249,93 +231,13 @@ __device__ inline void box_ax_body(BoxAxArgs<T> a, int per_xcd, BoxAxLds<T, NQ, 
   const int e = active ? grp * EPB + es : 0;
   const int f = blockIdx.y;
 
-  // rows of the lane's pencil: row0 at k = 0 (owned one layer down), then
-  // row1 + (k-1)*stride; masked ones read 0
   int ex, ey, ez;
   g.element(e, ex, ey, ez);
-  const int ox = ex - (ai == 0), oy = ey - (bj == 0);
-  const bool on = active && ox >= 0 && oy >= 0 && !(ai == N && ex == g.nx - 1) && !(bj == N && ey == g.ny - 1);
-  const int Nx = BoxGrid::owned<N>(ox, g.nx), Ny = BoxGrid::owned<N>(oy, g.ny);
-  const int stride = Nx * Ny;
-  const int at = ((bj == 0 ? N : bj) - 1) * Nx + (ai == 0 ? N : ai) - 1;
-  const int Nz = BoxGrid::owned<N>(ez, g.nz);
   unsigned off[NQ];
-  {
-    const unsigned row1 = (unsigned)(g.template base<N>(a.F, ox, oy, ez) + f * stride * Nz + at);
-    const unsigned row0 = (unsigned)(g.template base<N>(a.F, ox, oy, ez - 1) + (f * N + N - 1) * stride + at);
-    off[0] = on && ez > 0 ? row0 * S : kBoxMasked;
-#pragma unroll
-    for (int k = 1; k < NQ; ++k) off[k] = on && k <= Nz ? (row1 + (k - 1) * stride) * S : kBoxMasked;
-  }
+  box_pencil_offsets<T, NQ>(g, a.F, f, ex, ey, ez, ai, bj, active, off);
   T rq[NQ];
   if constexpr (MODE == MODE_FOLD) {
-    const __amdgpu_buffer_rsrc_t rr_ = box_rsrc(a.r), rp = box_rsrc(a.q), rx = box_rsrc(a.x), ro = box_rsrc(a.p);
-    const bool own = ai > 0 && bj > 0;
-    T pv[NQ], xv[NQ];
-    const bool first = it == 0, apply = (BATCH || a.pending) && !first;
-#pragma unroll
-    for (int k = 0; k < NQ; ++k) rq[k] = buffer_load<T>(rr_, off[k]);
-    if (!first) {
-#pragma unroll
-      for (int k = 0; k < NQ; ++k) pv[k] = buffer_load<T>(rp, off[k]);
-    }
-    if (apply) {
-#pragma unroll
-      for (int k = 1; k < NQ; ++k) xv[k] = buffer_load<T>(rx, own ? off[k] : kBoxMasked);
-    }
-    if (t < 64) {
-      const double v = wave_fold(a.part_rr, a.nrr);
-      if (t == 0) s_f[32] = v;
-    }
-    __syncthreads();
-    double rr = s_f[32], tol2;
-    const double tol = BATCH ? bs->tol : a.tol;
-    if (first) {
-      const double nrm = sqrt(rr);  // rdotr = norm2(r)^2 (linearSolverCG.cpp:84-85)
-      rr = nrm * nrm;
-      tol2 = fmax(tol * tol * rr, tol * tol);
-    } else {
-      tol2 = BATCH ? bs->tol2 : a.st->tol2;
-    }
-    bool stop = !(rr > tol2) || !isfinite(rr);
-    if constexpr (BATCH) {
-      stop = stop || it >= bs->maxit;
-      if (grp == 0 && t == 0) {
-        bs->rr_k = rr;
-        if (first) bs->tol2 = tol2;
-        if (stop) {
-          bs->rnorm = sqrt(rr);
-          if (!isfinite(rr)) bs->breakdown = 1;
-          bs->stop_at = it + 1;
-        }
-      }
-    } else if (blockIdx.x == 0 && blockIdx.y == 0 && t == 0) {
-      a.hist_rr[a.k] = rr;
-      if (first) {
-        a.st->tol2 = tol2;
-        a.st->breakdown = 0;
-        a.st->done = 0;
-        a.st->stop_at = 0;
-      }
-      if (stop) {
-        a.st->iter = a.k;
-        if (!isfinite(rr)) a.st->breakdown = 1;
-        a.st->stop_at = a.k + 1;
-      }
-    }
-    if (apply) {
-      const T al = (T)(BATCH ? bs->alpha : a.hist_alpha[it - 1]);
-#pragma unroll
-      for (int k = 1; k < NQ; ++k) buffer_store<T>(fmad(al, pv[k], xv[k]), rx, own ? off[k] : kBoxMasked);
-    }
-    if (stop) return;  // uniform over the problem
-    if (!first) {
-      const T beta = (T)(rr / (BATCH ? bs->rr_prev : a.hist_rr[it - 1]));
-#pragma unroll
-      for (int k = 0; k < NQ; ++k) rq[k] = fmad(beta, pv[k], rq[k]);
-    }
-#pragma unroll
-    for (int k = 1; k < NQ; ++k) buffer_store<T>(rq[k], ro, own ? off[k] : kBoxMasked);
+    if (box_direction<T, NQ, BATCH>(a, bs, it, grp, ai > 0 && bj > 0, off, rq, s_f)) return;  // uniform
   } else {
     const __amdgpu_buffer_rsrc_t rs = box_rsrc(a.q + (size_t)blockIdx.z * a.ldq);
 #pragma unroll
@@ -391,42 +293,10 @@ __device__ inline void box_ax_body(BoxAxArgs<T> a, int per_xcd, BoxAxLds<T, NQ, 
   EO::apply(tab, rq, gt);
   __builtin_amdgcn_sched_barrier(0);
   {
-    // TRILINEAR: along the pencil x_r = Ar + Br t, x_s = As + Bs t and x_t = Ct,
-    // so the adjugate's rows J grad r = x_s x x_t = Pr + Qr t and J grad s =
-    // x_t x x_r = Ps + Qs t are linear in t, and J grad t = x_r x x_s =
-    // T0 + T1 t + T2 t^2 and J = x_t . (J grad t) are quadratic
-    T Pr[3], Qr[3], Ps[3], Qs[3], T0[3], T1[3], T2[3], jt[3], ga[6], gw = 0;
+    TrilinearLine<T> map;
+    T ga[6], gw = 0;
     if constexpr (GEO == GEO_TRILINEAR) {
-      const T r = a.z[ai], sn = a.z[bj];
-      const cptr ce = (cptr)a.geo + (size_t)24 * e;
-      T Ar[3], Br[3], As[3], Bs[3], Ct[3];
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const T c_r = ce[8 * d + 0], c_s = ce[8 * d + 1], c_t = ce[8 * d + 2], c_rs = ce[8 * d + 3];
-        const T c_rt = ce[8 * d + 4], c_st = ce[8 * d + 5], c_rst = ce[8 * d + 6];
-        Ar[d] = fmad(c_rs, sn, c_r);
-        Br[d] = fmad(c_rst, sn, c_rt);
-        As[d] = fmad(c_rs, r, c_s);
-        Bs[d] = fmad(c_rst, r, c_st);
-        Ct[d] = fmad(Br[d], r, fmad(c_st, sn, c_t));
-      }
-      auto cross = [](const T* u, const T* v, int d) {
-        const int d1 = (d + 1) % 3, d2 = (d + 2) % 3;
-        return fmad(u[d1], v[d2], -(u[d2] * v[d1]));
-      };
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        Pr[d] = cross(As, Ct, d);
-        Qr[d] = cross(Bs, Ct, d);
-        Ps[d] = cross(Ct, Ar, d);
-        Qs[d] = cross(Ct, Br, d);
-        T0[d] = cross(Ar, As, d);
-        T1[d] = cross(Ar, Bs, d) + cross(Br, As, d);
-        T2[d] = cross(Br, Bs, d);
-      }
-      jt[0] = fmad(Ct[0], T0[0], fmad(Ct[1], T0[1], Ct[2] * T0[2]));
-      jt[1] = fmad(Ct[0], T1[0], fmad(Ct[1], T1[1], Ct[2] * T1[2]));
-      jt[2] = fmad(Ct[0], T2[0], fmad(Ct[1], T2[1], Ct[2] * T2[2]));
+      map.set((cptr)a.geo + (size_t)24 * e, a.z[ai], a.z[bj]);
     } else if constexpr (GEO == GEO_AFFINE) {
 #pragma unroll
       for (int c = 0; c < 6; ++c) ga[c] = a.geo[6 * (size_t)e + c];
@@ -453,33 +323,13 @@ __device__ inline void box_ax_body(BoxAxArgs<T> a, int per_xcd, BoxAxLds<T, NQ, 
       // one node at a time: without these the compiler forms every node's
       // map values before the first is used and spills
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (GEO == GEO_TRILINEAR) {
-#pragma unroll
-        for (int d = 0; d < 3; ++d) asm volatile("" : "+v"(Pr[d]), "+v"(Ps[d]), "+v"(T0[d]), "+v"(jt[d]));
-      }
+      if constexpr (GEO == GEO_TRILINEAR) map.pin();
       const T qr = s_b[k * LK + kb], qs = s_c[k * LK + kc], qt = gt[k];
       T Gr, Gs, Gt, W;
       if constexpr (GEO == GEO_TRILINEAR) {
-        const T tk = zk[k];
-        T ar[3], as[3], av[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          ar[d] = fmad(Qr[d], tk, Pr[d]);
-          as[d] = fmad(Qs[d], tk, Ps[d]);
-          av[d] = fmad(fmad(T2[d], tk, T1[d]), tk, T0[d]);
-        }
-        const T J = fmad(fmad(jt[2], tk, jt[1]), tk, jt[0]);
-        const T w = wij * wk[k];
-        T sc = w * reciprocal(J);
-        W = J * w;
-        if constexpr (KAPPA) sc *= kap[(size_t)k * kstep];
-        // G (grad q) as adj (w/J) adj^T, G itself not formed
-        T gx[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) gx[d] = sc * fmad(av[d], qt, fmad(as[d], qs, ar[d] * qr));
-        Gr = fmad(ar[2], gx[2], fmad(ar[1], gx[1], ar[0] * gx[0]));
-        Gs = fmad(as[2], gx[2], fmad(as[1], gx[1], as[0] * gx[0]));
-        Gt = fmad(av[2], gx[2], fmad(av[1], gx[1], av[0] * gx[0]));
+        T kv = T(1);
+        if constexpr (KAPPA) kv = kap[(size_t)k * kstep];
+        map.template flux<KAPPA>(zk[k], wij * wk[k], kv, qr, qs, qt, Gr, Gs, Gt, W);
       } else {
         T g[6];
         if constexpr (GEO == GEO_AFFINE) {

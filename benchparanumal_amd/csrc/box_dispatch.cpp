@@ -24,12 +24,16 @@ template <typename T>
 int launch_box_ax(hipStream_t s, const BoxAxArgs<T>& a) {
   const BoxGrid& g = a.g;
   if (!a.q || !a.AqL) return set_error(BPX_ERR_INVALID_ARGUMENT, "box Ax: null device pointer");
-  if (!a.geo || !a.eo || (a.geoKind == BOX_GEO_TRILINEAR && !a.z) || (a.geoKind != BOX_GEO_TRILINEAR && !a.wJ) ||
-      (a.geoKind != BOX_GEO_STORED && !a.w))
+  const bool gll = a.op == BOX_OP_GLL;
+  if (!a.eo || (gll ? !a.geo || (a.geoKind == BOX_GEO_TRILINEAR && !a.z) || (a.geoKind != BOX_GEO_TRILINEAR && !a.wJ) ||
+                          (a.geoKind != BOX_GEO_STORED && !a.w)
+                    : !a.geo64 || !a.z64 || !a.w64))
     return set_error(BPX_ERR_INVALID_ARGUMENT, "box Ax: null geometry/operator pointer");
+  if (!gll && (a.geoKind != BOX_GEO_TRILINEAR || a.kappa || a.K != 1))
+    return set_error(BPX_ERR_UNSUPPORTED, "box Ax: the cubature operators have constant coefficients and one right-hand side");
   if (a.fold && (!a.part || !a.r || !a.p || !a.x || !a.part_rr || !a.hist_rr || !a.hist_alpha || !a.st || a.p == a.q))
     return set_error(BPX_ERR_INVALID_ARGUMENT, "box Ax: incomplete CG arguments");
-#define BPX_CALL(NQ) case NQ: return launch_box_ax_nq<T, NQ>(s, a);
+#define BPX_CALL(NQ) case NQ: return gll ? launch_box_ax_nq<T, NQ>(s, a) : launch_box_cub_nq<T, NQ>(s, a);
   BPX_BOX_SWITCH(BPX_CALL)
 #undef BPX_CALL
 }
@@ -38,8 +42,8 @@ int box_gather_elements(int Nq) { return box_gather_epb(Nq); }
 
 int box_ax_elements(int Nq) { return box_epb(Nq); }
 
-int box_ax_partials(const BoxGrid& g, int F) {
-  const int epb = box_epb(g.N + 1);
+int box_ax_partials(const BoxGrid& g, int F, int op) {
+  const int epb = box_epb(g.N + (op == BOX_OP_GLL ? 1 : 2));
   return (g.elements() + epb - 1) / epb * F;
 }
 

@@ -346,16 +346,22 @@ struct BatchState;
 // reference rows, AqL in [element][field][node] layout, both smaller than
 // 2^31 - 8 bytes.
 enum { BOX_GEO_TRILINEAR = 0, BOX_GEO_AFFINE = 1, BOX_GEO_STORED = 2 };
+// the operator: BP5/BP6 on the GLL points (box_ax.hip), BP1/BP2 and BP3/BP4 on
+// the cubature points (box_cub.hip; trilinear maps, constant coefficient)
+enum { BOX_OP_GLL = 0, BOX_OP_MASS = 1, BOX_OP_STIFF = 2 };
 template <typename T>
 struct BoxAxArgs {
   BoxGrid g;
   int F = 1;
+  int op = BOX_OP_GLL;
   int geoKind = BOX_GEO_TRILINEAR;
   const T* geo = nullptr;    // 24 map coefficients per element, 6 factors per element, or 6 per node (FP32 only)
   const T* wJ = nullptr;     // J per element (affine), wJ per node (stored)
   const T* z = nullptr;      // GLL nodes (trilinear)
   const T* w = nullptr;      // GLL weights (trilinear, affine)
-  const T* eo = nullptr;     // even-odd table of D (EvenOdd, box_ax.hip)
+  // cubature operators instead: the map coefficients, points and weights
+  const double *geo64 = nullptr, *z64 = nullptr, *w64 = nullptr;
+  const T* eo = nullptr;     // even-odd table of D (EvenOdd, box_ax_body.hpp), or EoTables (even_odd.hpp)
   const T* kappa = nullptr;  // coefficient on the node lattice (FP64), or null
   T lambda = 0;
   const T* q = nullptr;
@@ -390,8 +396,8 @@ struct BoxAxArgs {
 };
 template <typename T>
 int launch_box_ax(hipStream_t s, const BoxAxArgs<T>& a);
-int box_ax_elements(int Nq);  // elements per workgroup
-int box_ax_partials(const BoxGrid& g, int F);
+int box_ax_elements(int Nq);  // elements per workgroup of the GLL operator
+int box_ax_partials(const BoxGrid& g, int F, int op);
 
 // The end of a CG iteration: r -= alpha gather(AqL) with alpha from the p.Ap
 // partials, and partials of r.r (*nrr of them, at most kBoxRrParts)

@@ -866,8 +866,7 @@ int bpx_bp_set_cub_form(bpx_bp b, int form) {
     return set_error(BPX_ERR_INVALID_ARGUMENT,
                      "bp: cubature kernel form must be 0 (auto), 1 (pencil), 2 (wavefront) or 3 (pencil, row-by-row "
                      "contractions)");
-  b->bp.cubForm = form;
-  return BPX_OK;
+  return b->bp.SetCubForm(form);
   BPX_GUARD_END
 }
 

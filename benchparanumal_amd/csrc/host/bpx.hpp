@@ -375,7 +375,7 @@ class bp_t : public solver_t {
   int OperatorDot(const dfloat* o_q, dfloat* o_Aq, double* part, int* npart) override;
   int GatherPartials() const {
     return std::max({ogs_gather_partials(ogs.NrowBlocksT), ogs_gather_partials(sharedOgs.NrowBlocksT),
-                     ogs_gather_partials(solveOgs.NrowBlocksT), haveBox ? box_ax_partials(box, Nfields) : 1, 1});
+                     ogs_gather_partials(solveOgs.NrowBlocksT), haveBox ? BoxPartials() : 1, 1});
   }
 
   // Solve space: the row order the CG solvers run in. For BP5 with one
@@ -502,14 +502,24 @@ class bp_t : public solver_t {
   // (box_ax.hip). At p = 15 the stored-factor kernel reads 76 bytes per node
   // and no cache holds them: 24^3, operator 1034 -> 534 us.
   bool boxAx = false;
-  deviceBuffer<double> o_boxGeo, o_boxZ, o_boxEo, o_kappa;
+  // BP1-BP4 on the box, trilinear elements (box_cub.hip), unless a kernel
+  // form is set: those read the stored factors
+  bool boxCub = false;
+  bool OnBox() const { return boxAx || (boxCub && cubForm == CUB_FORM_AUTO); }
+  int BoxOp() const { return bp >= 5 ? BOX_OP_GLL : bp >= 3 ? BOX_OP_STIFF : BOX_OP_MASS; }
+  int BoxPartials() const { return box_ax_partials(box, Nfields, BoxOp()); }
+  // the maps' coefficients (non-affine), then from boxZ, boxW and boxEo on the
+  // points, the weights and the GLL table of D
+  deviceBuffer<double> o_boxTab, o_kappa;
+  size_t boxZ = 0, boxW = 0, boxEo = 0;
   deviceBuffer<float> o_boxEo32;
   // the box Ax's arguments in precision T; q and AqL as given
   template <typename T>
   BoxAxArgs<T> BoxArgs(const T* o_q, T* o_AqL) const;
-  // whether precision T's operator runs on box_ax.hip
+  // whether precision T's operator runs on box_ax.hip or box_cub.hip
   template <typename T>
   bool BoxAx() const {
+    if (bp <= 4) return OnBox() && (sizeof(T) == 8 || fp32Geometry == 0);
     return sizeof(T) == 8 ? boxAx : haveBox && bp == 5;
   }
   // The CG operator in two kernels per iteration, the Ax with the direction
@@ -518,6 +528,7 @@ class bp_t : public solver_t {
   // affine elements, tuning.fused64 are timed).
   bool boxFused64 = true;
   bool BoxFused(int precision) const {
+    if (bp <= 4) return boxFused64;
     if (precision == 32) return tuning.fused32;
     return bp == 5 && mesh->opts.affine ? tuning.fused64 != 0 : boxFused64;
   }
@@ -579,12 +590,13 @@ class bp_t : public solver_t {
   // FP32 copies (created on first use)
   int Prepare32();
   bool have32 = false;
-  int tri32 = 0;  // the FP32 BP5 operator forms its geometric factors from the trilinear maps
+  int tri32 = 0;  // the FP32 operator forms its geometric factors from the trilinear maps
   // FP32 BP5 geometry (non-affine): 0 = from the elements' trilinear maps,
   // 1 = stored factors rounded to FP32. Changing it rebuilds the FP32
   // operator on next use.
   int fp32Geometry = 0;
   int SetFp32Geometry(int mode);
+  int SetCubForm(int form);
   deviceBuffer<float> o_wJ32, o_ggeo32, o_gllw32, o_D32, o_I32, o_MM32, o_invV32, o_AqL32;
   deviceBuffer<float> o_eo32;
   // nodal coordinates for the forcing (created on first use)

@@ -15,7 +15,7 @@ namespace bpx {
 // A[N-1-n][M-1-m] = sign * A[n][m]: row n (n <= (N-1)/2) holds
 // (A[n][m] + A[n][M-1-m]) / 2 for m < M/2, A[n][M/2] for odd M, then
 // (A[n][m] - A[n][M-1-m]) / 2 for m < M/2 (the layout of eo_apply in
-// ax_cub.hip). False if A is not (anti)symmetric to rounding.
+// even_odd.hpp). False if A is not (anti)symmetric to rounding.
 static bool even_odd_rows(const double* A, int N, int M, int sign, std::vector<double>& out) {
   double amax = 0;
   for (int i = 0; i < N * M; ++i) amax = std::max(amax, std::fabs(A[i]));
@@ -31,13 +31,13 @@ static bool even_odd_rows(const double* A, int N, int M, int sign, std::vector<d
   return true;
 }
 
-// the pencil kernel's tables (BP1-BP4, non-affine hex, N <= 7): I (cubNq x
-// Nq), I^T, D and D^T of the cubature grid, one after another; empty where
-// they do not apply
+// the tables of EoTables (even_odd.hpp; BP1-BP4, non-affine hex): I (cubNq x
+// Nq), I^T, D and D^T of the cubature grid, one after another, then D itself
+// by rows; empty where they do not apply
 static std::vector<double> cub_even_odd_tables(const mesh_t& m) {
   std::vector<double> t;
   const int nq = m.Nq, mq = m.cubNq;
-  if (m.elementType != ELEM_HEX || m.opts.affine || nq > 8 || mq != nq + 1 ||
+  if (m.elementType != ELEM_HEX || m.opts.affine || mq != nq + 1 ||
       m.cubInterp.size() != (size_t)mq * nq || m.cubD.size() != (size_t)mq * mq)
     return t;
   std::vector<double> IT((size_t)nq * mq), DT((size_t)mq * mq);
@@ -48,9 +48,10 @@ static std::vector<double> cub_even_odd_tables(const mesh_t& m) {
   if (!even_odd_rows(m.cubInterp.data(), mq, nq, 1, t) || !even_odd_rows(IT.data(), nq, mq, 1, t) ||
       !even_odd_rows(m.cubD.data(), mq, mq, -1, t) || !even_odd_rows(DT.data(), mq, mq, -1, t))
     t.clear();
+  else
+    t.insert(t.end(), m.cubD.begin(), m.cubD.end());
   return t;
 }
-
 
 // ------------------------------------------------------------- errors ---
 static thread_local std::string g_last_error;
@@ -438,16 +439,21 @@ int bp_t::Setup(platform_t& p, mesh_t& m, int bp_, dfloat lambda_) {
       if (int st = o_eo.upload(eo, s)) return st;
   }
   boxAx = haveBox && (bp == 5 || bp == 6);
-  if (boxAx) {
-    std::vector<double> eo;
-    if (int st = box_even_odd_table(m, eo)) return st;
-    if (int st = o_boxEo.upload(eo, s)) return st;
-    if (int st = o_boxZ.upload(m.gllz, s)) return st;
-    if (!affine) {
-      std::vector<double> c;
-      m.TrilinearCoefficients(c);
-      if (int st = o_boxGeo.upload(c, s)) return st;
+  boxCub = haveBox && bp <= 4 && o_eo.length() > 0;
+  if (boxAx || boxCub) {  // one upload: the maps, then the 1D data
+    std::vector<double> t, eo;
+    if (!affine) m.TrilinearCoefficients(t);
+    auto append = [&t](const std::vector<double>& v) {
+      t.insert(t.end(), v.begin(), v.end());
+      return t.size() - v.size();
+    };
+    boxZ = append(boxCub ? m.cubr : m.gllz);
+    boxW = append(boxCub ? m.cubw : m.gllw);
+    if (boxAx) {
+      if (int st = box_even_odd_table(m, eo)) return st;
+      boxEo = append(eo);
     }
+    if (int st = o_boxTab.upload(t, s)) return st;
   }
   if (int st = m.onDevice ? PrepareFusedDevice() : PrepareFused()) return st;
   if (boxAx && bp == 5 && affine) fused = true;
@@ -508,13 +514,22 @@ BoxAxArgs<T> bp_t::BoxArgs(const T* o_q, T* o_AqL) const {
   const int affine = mesh->opts.affine;
   a.g = box;
   a.F = Nfields;
-  if constexpr (std::is_same<T, double>::value) {
+  a.op = BoxOp();
+  if (bp <= 4) {
+    a.geo64 = o_boxTab.ptr();
+    a.z64 = o_boxTab.ptr() + boxZ;
+    a.w64 = o_boxTab.ptr() + boxW;
+    if constexpr (std::is_same<T, double>::value)
+      a.eo = o_eo.ptr();
+    else
+      a.eo = o_eo32.ptr();
+  } else if constexpr (std::is_same<T, double>::value) {
     a.geoKind = affine ? BOX_GEO_AFFINE : BOX_GEO_TRILINEAR;
-    a.geo = affine ? o_ggeo.ptr() : o_boxGeo.ptr();
+    a.geo = affine ? o_ggeo.ptr() : o_boxTab.ptr();
     a.wJ = o_wJ.ptr();
-    a.z = o_boxZ.ptr();
-    a.w = o_gllw.ptr();
-    a.eo = o_boxEo.ptr();
+    a.z = o_boxTab.ptr() + boxZ;
+    a.w = o_boxTab.ptr() + boxW;
+    a.eo = o_boxTab.ptr() + boxEo;
     a.kappa = haveKappa ? o_kappa.ptr() : nullptr;
   } else {
     a.geoKind = affine ? BOX_GEO_AFFINE : tri32 ? BOX_GEO_TRILINEAR : BOX_GEO_STORED;
@@ -539,7 +554,7 @@ int bp_t::AxLocal(const dfloat* o_q, dfloat* o_AqL) {
 }
 
 int bp_t::AxOperator(const dfloat* o_q, dfloat* o_AqL) {
-  if (boxAx) return launch_box_ax<double>(platform->stream, BoxArgs<double>(o_q, o_AqL));
+  if (OnBox()) return launch_box_ax<double>(platform->stream, BoxArgs<double>(o_q, o_AqL));
   return AxStored(o_q, o_AqL);
 }
 
@@ -631,10 +646,10 @@ int bp_t::GatherLocal(const T* o_AqL, T* o_Aq, int K) const {
 // the solve space when the rows are renumbered (the Aq rows are the same
 // sums either way, bit for bit).
 int bp_t::OperatorDot(const dfloat* o_q, dfloat* o_Aq, double* part, int* npart) {
-  if (boxAx) {
+  if (OnBox()) {
     BoxAxArgs<double> a = BoxArgs<double>(o_q, o_AqL.ptr());
     a.part = part;
-    *npart = box_ax_partials(box, Nfields);
+    *npart = BoxPartials();
     if (int st = launch_box_ax<double>(platform->stream, a)) return st;
     return GatherLocal<double>(o_AqL.ptr(), o_Aq);
   }
@@ -706,7 +721,7 @@ class BoxCgSteps : public CgSteps<T> {
       if (int st = launch_cg_update_p<T>(s, N, k, r, p[0], x, w.part_rr, this->nrr, w.state, w.hist_rr, w.hist_alpha,
                                          tol, pending))
         return st;
-    const int npAp = box_ax_partials(b.box, b.Nfields);
+    const int npAp = b.BoxPartials();
     auto apply = [&]() -> int {
       BoxAxArgs<T> a = b.BoxArgs<T>(fold ? p[(k + 1) & 1] : p[0], AqL);
       a.part = w.part_pAp;
@@ -769,7 +784,7 @@ template std::unique_ptr<CgSteps<float>> bp_t::BoxSteps<float>(float*, float*, f
 // operators 2e-12 to 1e-7 apart over 12 meshes), so a faster operator would
 // give another history, where a converged solution is the same.
 int bp_t::SolveCG(cg& solver, dfloat* o_x, dfloat* o_r, dfloat tol, int maxit, int verbose, int* iterations) {
-  if (boxAx && ogs.Ngather > 0 && (tol > 0 || haveKappa || mesh->opts.affine)) {
+  if (OnBox() && ogs.Ngather > 0 && (tol > 0 || haveKappa || mesh->opts.affine)) {
     if (solver.status()) return solver.status();
     if (maxit < 0) return set_error(BPX_ERR_INVALID_ARGUMENT, "cg: MAXIT < 0");
     cg_t<double>& c = solver.impl;
@@ -785,7 +800,7 @@ int bp_t::SolveCG(cg& solver, dfloat* o_x, dfloat* o_r, dfloat tol, int maxit, i
     return solver.Solve(*this, o_x, o_r, tol, maxit, verbose, iterations, steps.get());
   }
   if (!permuted) {
-    if (!boxAx) return solver.Solve(*this, o_x, o_r, tol, maxit, verbose, iterations);
+    if (!OnBox()) return solver.Solve(*this, o_x, o_r, tol, maxit, verbose, iterations);
     bp_solve_view_t view(*this);
     return solver.Solve(view, o_x, o_r, tol, maxit, verbose, iterations);
   }
@@ -1014,7 +1029,7 @@ int bp_t::OperatorDot32(const float* o_q, float* o_Aq, double* part, int* npart)
   if (BoxAx<float>()) {
     BoxAxArgs<float> a = BoxArgs<float>(o_q, o_AqL32.ptr());
     a.part = part;
-    *npart = box_ax_partials(box, Nfields);
+    *npart = BoxPartials();
     if (int st = launch_box_ax<float>(platform->stream, a)) return st;
     return GatherLocal<float>(o_AqL32.ptr(), o_Aq);
   }
@@ -1208,7 +1223,7 @@ int bp_t::Tune() {
 
 // The same choice for the FP32 operator, timed when it is first built
 int bp_t::Tune32() {
-  if (!BoxAx<float>()) return BPX_OK;
+  if (bp != 5 || !BoxAx<float>()) return BPX_OK;
   return TuneBox<float>(tuning.fused32, tuning.fused32_us, tuning.unfused32_us);
 }
 
@@ -1235,7 +1250,7 @@ int bp_t::TimeOperator(int precision, int launches, double* out) {
   auto run = [&]() -> int {
     int np = 0;
     if (precision == 64)
-      return boxAx ? OperatorDot(v64.ptr(), v64.ptr() + n, part.ptr(), &np)
+      return OnBox() ? OperatorDot(v64.ptr(), v64.ptr() + n, part.ptr(), &np)
                    : OperatorDotS(v64.ptr(), v64.ptr() + n, part.ptr(), &np);
     return OperatorDot32(v32.ptr(), v32.ptr() + n, part.ptr(), &np);
   };
@@ -1298,7 +1313,9 @@ int bp_t::Prepare32() {
     std::vector<double> eo;
     if ((st = box_even_odd_table(m, eo)) || (st = cvt(o_boxEo32, eo))) return st;
   }
-  if (bp == 5 && !affine && fp32Geometry == 0) {
+  if (bp <= 4 && BoxAx<float>()) {  // cubature factors from the FP64 operator's maps
+    tri32 = 1;
+  } else if (bp == 5 && !affine && fp32Geometry == 0) {
     // the FP32 operator forms its geometric factors from the elements'
     // trilinear maps: 96 B per element instead of 28 B per node
     std::vector<double> tri;
@@ -1327,6 +1344,17 @@ int bp_t::Prepare32() {
   have32 = true;
   if ((st = Tune32())) return st;
   return platform->finish();
+}
+
+int bp_t::SetCubForm(int form) {
+  if (form == cubForm) return BPX_OK;
+  if (boxCub && have32) {  // the FP32 arrays are those of one kind of kernel
+    if (int st = platform->finish()) return st;
+    have32 = false;
+    tri32 = 0;
+  }
+  cubForm = form;
+  return BPX_OK;
 }
 
 int bp_t::SetFp32Geometry(int mode) {

@@ -165,3 +165,89 @@ def test_box_kappa_operator(plat, N, affine):
     A = torch.full((b.Ngather,), float("nan"), dtype=torch.float64, device="cuda")
     b.operator(torch.from_numpy(q).cuda(), A)
     assert rel_err(host(A), P.operator(q)) <= 1e-12
+
+
+# --------------------------------------------------------- box_cub.hip ----
+def cub_pair(bp, N, nx, ny, nz, lam=1.3):
+    kw = dict(N=N, nx=nx, ny=ny, nz=nz, perturb=0.1, seed=7)
+    return capi.Mesh(cubature=True, **kw), oracle_lib.Problem(bp=bp, lam=lam, **kw)
+
+
+@pytest.mark.parametrize("bp,N", [(bp, N) for bp in (1, 2, 3, 4) for N in range(1, 16)])
+def test_box_cub_operator_matches_oracle(plat, bp, N):
+    """BP1-BP4 at every degree, the last workgroup partly empty: against the
+    oracle to the FP64 bar, against the stored-factor kernel (whose cubggeo
+    come from the cubature D, hence the bar again), q.Aq of the CG form, and
+    the local Ax through the map gather to the bit."""
+    m, P = cub_pair(bp, N, 3, 2, 3 if N < 10 else 1)
+    b = capi.BP(plat, m, bp, lam=1.3)
+    q = np.random.default_rng(N).standard_normal(b.Ngather)
+    qd = torch.from_numpy(q).cuda()
+    A, A2, A3 = torch.full((3, b.Ngather), float("nan"), dtype=torch.float64, device="cuda")
+    b.operator(qd, A)
+    assert rel_err(host(A), P.operator(q)) <= 1e-12
+    qAq = b.operator_dot(qd, A2)
+    np.testing.assert_array_equal(host(A2), host(A))
+    assert abs(qAq - float(np.dot(q, host(A)))) <= 1e-13 * np.abs(q * host(A)).sum()
+    AL = torch.full((b.NLocal,), float("nan"), dtype=torch.float64, device="cuda")
+    b.ax_local(qd, AL)
+    capi.Ogs(mesh=m, nfields=b.Nfields).gather(plat, AL, A3)
+    np.testing.assert_array_equal(host(A3), host(A))
+    b.set_cub_form(1)
+    b.operator(qd, A3)
+    assert rel_err(host(A3), host(A)) <= 1e-12
+
+
+@pytest.mark.parametrize("bp", [1, 3])
+@pytest.mark.parametrize("N", range(1, 16))
+def test_box_cub_operator_f32(plat, bp, N):
+    """FP32, factors formed and (geometry 1, or a kernel form) stored."""
+    m, P = cub_pair(bp, N, 3, 2, 2)
+    b = capi.BP(plat, m, bp, lam=1.3)
+    q = np.random.default_rng(N).standard_normal(b.Ngather)
+    ref = P.operator(q)
+    for geometry, form, formed in ((0, 0, 1), (1, 0, 0), (0, 1, 0), (0, 0, 1)):
+        b.set_fp32_geometry(geometry)
+        b.set_cub_form(form)
+        A = torch.full((b.Ngather,), float("nan"), dtype=torch.float32, device="cuda")
+        b.operator_f32(torch.from_numpy(q).cuda().float(), A)
+        assert rel_err(host(A).astype(np.float64), ref) <= 2e-5
+        assert b.tuning()["fp32_trilinear"] == formed
+
+
+@pytest.mark.parametrize("bp,N,nx,ny,nz", [(1, 6, 3, 3, 2), (2, 3, 3, 2, 2), (3, 1, 4, 4, 3), (3, 7, 3, 3, 2),
+                                           (3, 9, 2, 3, 2), (3, 12, 2, 2, 2), (4, 4, 2, 2, 3), (3, 2, 1, 1, 1)])
+def test_box_cub_cg(plat, bp, N, nx, ny, nz):
+    """CG to a tolerance with the direction update inside the Ax and in its own
+    kernel (the same bits), and the mixed-precision solve, as test_box_cg_forms;
+    a fixed number of iterations keeps the stored factors' history."""
+    m, P = cub_pair(bp, N, nx, ny, nz, lam=1.0)
+    b = capi.BP(plat, m, bp, lam=1.0)
+    rhs = capi.random_normal(5, b.Ngather)
+    x_ref, _, _, _ = P.cg(rhs, 5000, tol=1e-12)
+    sols = []
+    for fold in (3, 0):
+        b.set_cg_fold(fold)
+        x = torch.zeros(b.Ngather, dtype=torch.float64, device="cuda")
+        its, hist = b.solve(x, torch.from_numpy(rhs).cuda(), tol=1e-10, maxit=5000)
+        assert np.linalg.norm(host(x) - x_ref) <= 1e-8 * np.linalg.norm(x_ref)
+        sols.append((its, hist, host(x)))
+    assert sols[0][0] == sols[1][0]
+    np.testing.assert_array_equal(sols[0][1], sols[1][1])
+    np.testing.assert_array_equal(sols[0][2], sols[1][2])
+    if bp in (1, 3):
+        # (interval 64: where an interval ends just as the FP32 recurrence has
+        # run out of unknowns, 16 and 32 for 18 and 45 of them, a solve of
+        # either operator can stall at the FP32 level)
+        x = torch.zeros(b.Ngather, dtype=torch.float64, device="cuda")
+        st = b.solve_mixed(x, torch.from_numpy(rhs).cuda(), tol=1e-10, interval=64)
+        assert st["rel_res"] < 1e-10
+        assert np.linalg.norm(host(x) - x_ref) <= 1e-8 * np.linalg.norm(x_ref)
+    out = []
+    for form in (0, 1):  # up to N = 7 form 1 is the stored-factor default
+        b.set_cub_form(form)
+        x = torch.zeros(b.Ngather, dtype=torch.float64, device="cuda")
+        _, hist = b.solve(x, torch.from_numpy(rhs).cuda(), tol=0.0, maxit=10)
+        out.append((hist, host(x)))
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    np.testing.assert_array_equal(out[0][1], out[1][1])
