@@ -148,6 +148,10 @@ class mesh_t {
   // (24 values): the nodal coordinates are this map at the GLL nodes, by
   // construction (Setup and SetupDevice)
   void TrilinearCoefficients(std::vector<double>& c) const;
+  // whether every local node lies on its element's trilinear map of the 8
+  // vertices at the GLL point (to 1e-12 of the box size): then the
+  // geometric factors are the map's exact derivatives
+  bool NodesAreTrilinear() const;
   // mesh_t::PlotFields (libs/mesh/meshPlotFields3D.cpp:31-121): VTU file of
   // the local nodes with Nfields values each (QL: host, [e][f][n]); each
   // element is drawn as N^3 sub-cubes of 6 tetrahedra
