@@ -1011,15 +1011,26 @@ int bp_t::TimeKrhs(int K, int chunk, int launches, const dfloat* o_q, double* ou
   return BPX_OK;
 }
 
+// On the box the right-hand sides go through Ax and gather a few at a time,
+// as many as keep their local values below kKrhsBytes: those are then still
+// in the 256 MB Infinity Cache when the gather reads them, and the workspace
+// is no larger. Measured at 20^3, p = 7, K = 16: 485 us in one go, 444 with 136 MB, 461 with 104, 478 with 168.
 int bp_t::OperatorKrhs(int K, const dfloat* o_q, dfloat* o_Aq, int chunk) {
   if (K < 1) return set_error(BPX_ERR_INVALID_ARGUMENT, "bp: K < 1");
-  const size_t need = (size_t)NLocal * K;
+  constexpr size_t kKrhsBytes = (size_t)136 << 20;
+  const bool some = chunk == 0 && boxAx && bp == 5 && !haveKappa && ogs.Ngather > 0 && K <= 65535;
+  const int kc = some ? (int)std::min<size_t>(K, std::max<size_t>(1, kKrhsBytes / ((size_t)NLocal * sizeof(double)))) : K;
+  const size_t need = (size_t)NLocal * kc;
   if (o_AqLk.length() < need) {
     if (int st = platform->finish()) return st;  // the old buffer may still be in use
     if (int st = o_AqLk.alloc(need)) return st;
   }
-  if (int st = AxLocalKrhs(K, o_q, o_AqLk.ptr(), chunk)) return st;
-  return GatherLocal<double>(o_AqLk.ptr(), o_Aq, K);
+  for (int k = 0; k < K; k += kc) {
+    const int n = std::min(kc, K - k);
+    if (int st = AxLocalKrhs(n, o_q + (size_t)k * ogs.Ngather, o_AqLk.ptr(), chunk)) return st;
+    if (int st = GatherLocal<double>(o_AqLk.ptr(), o_Aq + (size_t)k * ogs.Ngather, n)) return st;
+  }
+  return BPX_OK;
 }
 
 int bp_t::OperatorDot32(const float* o_q, float* o_Aq, double* part, int* npart) {
