@@ -563,9 +563,9 @@ def main():
     ap.add_argument("--interval", type=int, default=64,
                     help="FP32 iterations between FP64 defect corrections")
     ap.add_argument("--ax-launches", type=int, default=50)
-    ap.add_argument("--cg-fold", type=int, default=1, choices=(0, 1, 2, 3),
-                    help="where the fused CG operator also does the interior rows' direction update: "
-                         "bit 0 = FP64 solves (default 1), bit 1 = FP32 iterations (same bits)")
+    ap.add_argument("--cg-fold", type=int, default=3, choices=(0, 1, 2, 3),
+                    help="where the CG operator's Ax also does the direction update: "
+                         "bit 0 = FP64 solves, bit 1 = FP32 iterations (default 3, both; same bits)")
     ap.add_argument("--setup", choices=("device", "host"), default="device",
                     help="where the mesh, ogs maps and solve-space maps are built (same arrays either way)")
     ap.add_argument("--no-setup-compare", action="store_true",

@@ -354,10 +354,10 @@ class BP:
         return _read_array(lib().bpx_bp_array, self.h, name)
 
     def set_cg_fold(self, mask):
-        """Where the fused CG operator also does the interior rows' direction
-        update: mask bit 0 = FP64 solves (the default, mask 1), bit 1 = the
-        FP32 iterations of the mixed solve; elsewhere one update kernel covers
-        all rows. Same bits either way."""
+        """Where the CG operator's Ax also does the direction update (with the
+        stored factors: of the interior rows): mask bit 0 = FP64 solves, bit 1
+        = the FP32 iterations of the mixed solve (default 3, both); elsewhere
+        one update kernel covers all rows. Same bits either way."""
         check(lib().bpx_bp_set_cg_fold(self.h, int(mask)))
 
     def set_ax_engine(self, engine):
@@ -367,7 +367,8 @@ class BP:
         check(lib().bpx_bp_set_ax_engine(self.h, int(engine)))
 
     def set_cub_form(self, form):
-        """BP1-BP4 non-affine at N <= 7: 0 = auto (pencil kernel), 1 =
+        """BP1-BP4 non-affine: 0 = auto (factors formed from the elements'
+        trilinear maps); the kernels on stored factors, at N <= 7: 1 =
         pencil (even-odd contractions), 2 = one element per wavefront, 3 =
         pencil with row-by-row contractions (the forms agree to rounding)."""
         check(lib().bpx_bp_set_cub_form(self.h, int(form)))

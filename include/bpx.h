@@ -377,7 +377,7 @@ int bpx_bp_array(bpx_bp b, const char* name, void* dst, int64_t* count, int* dty
  * 0/1, FP64 operator fused 0/1, FP32 operator fused 0/1; -1 keeps a
  * choice. */
 int bpx_bp_set_tuning(bpx_bp b, int gatherMode, int fused, int fused32);
-/* No reference counterpart: the geometry of the FP32 BP5 operator (the
+/* No reference counterpart: the geometry of the FP32 BP5, BP1 and BP3 operator (the
  * inner operator of bpx_bp_solve_mixed). mode 0 (default): formed in the
  * kernel from each element's trilinear map of its 8 vertices (what the box
  * meshes of bpx_mesh_create are); mode 1: the FP64 geometric factors
@@ -394,8 +394,10 @@ int bpx_bp_set_fp32_geometry(bpx_bp b, int mode);
  * either setting, as other problems do. */
 int bpx_bp_set_ax_engine(bpx_bp b, int engine);
 /* No reference counterpart (launch choice): which kernel runs the BP1-BP4
- * Ax of a problem object on non-affine meshes at N <= 7: 0 = auto (the
- * pencil kernel; default), 1 = pencil (several fields or elements per
+ * Ax of a problem object on non-affine meshes: 0 = auto (default: the
+ * factors formed in the kernel from the elements' trilinear maps, except in
+ * solves with tol = 0, which run form 1), or a kernel on the stored factors,
+ * with a choice at N <= 7: 1 = pencil (several fields or elements per
  * workgroup, every contraction along a line one lane holds, in even-odd
  * form), 2 = one element per wavefront, 3 = pencil with row-by-row
  * contractions (the form the kernel-level entry points run). The forms
