@@ -24,6 +24,8 @@ constexpr int kGraphIters = 8;      // CG iterations per captured graph
 }  // namespace
 
 bp_batch_t::~bp_batch_t() {
+  // (a call that failed half way may have left work queued)
+  if (stream) (void)hipStreamSynchronize(stream);
   if (graphExec) (void)hipGraphExecDestroy(graphExec);
   if (graphMixed) (void)hipGraphExecDestroy(graphMixed);
   if (h_count) (void)hipHostFree(h_count);
@@ -339,7 +341,8 @@ int bp_batch_t::Solve(double* o_x, const double* o_b, double tol, int maxit, int
   const long long maxReplays = (long long)maxit / kGraphIters + 2;
   replays = 0;
   // the count of replay rep is read while replay rep + 1 runs (a replay past
-  // the end finds every problem done and does nothing)
+  // the end finds every problem done and does nothing); both entries of
+  // h_count are the stream's until the wait below
   for (long long rep = 0; rep < maxReplays; ++rep) {
     BPX_HIP(hipGraphLaunch(graphExec, stream));
     BPX_HIP(hipMemcpyAsync(h_count + (rep & 1), o_count.ptr(), sizeof(int), hipMemcpyDeviceToHost, stream));
@@ -352,7 +355,10 @@ int bp_batch_t::Solve(double* o_x, const double* o_b, double tol, int maxit, int
   if (Ntot > 0)
     BPX_HIP(hipMemcpyAsync(o_x, this->o_x.ptr(), (size_t)Ntot * sizeof(double), hipMemcpyDeviceToDevice, stream));
   std::vector<BatchState> hs(nprob);
-  BPX_HIP(hipMemcpy(hs.data(), o_state.ptr(), sizeof(BatchState) * nprob, hipMemcpyDeviceToHost));
+  BPX_HIP(hipMemcpyAsync(hs.data(), o_state.ptr(), sizeof(BatchState) * nprob, hipMemcpyDeviceToHost, stream));
+  // x and the states are complete on return: the stream is the batch's own,
+  // which neither the caller nor the null stream waits for
+  BPX_HIP(hipStreamSynchronize(stream));
   int anyBreak = 0;
   for (int i = 0; i < nprob; ++i) {
     if (iterations) iterations[i] = hs[i].iter;

@@ -110,6 +110,34 @@ def test_batch_single_problem_and_maxit(plat):
     assert abs(rn[0] - hist[-1]) <= 1e-9 * hist[0]
 
 
+def test_batch_solution_is_complete_on_return(solved):
+    """The call returns host values, so its x is complete when it returns: a
+    platform on a stream of its own, x read at once through another stream,
+    which waits for neither, and again once the device is idle. A batch whose
+    problems are released right after a solve goes the same way."""
+    probs, _, _, ref, its, _ = solved
+    own = capi.Platform(0, torch_stream=False)
+    B = capi.Batch(own, probs, lam=1.0)
+    rhs = torch.from_numpy(capi.random_normal(77, B.Ntot)).cuda()
+    x = torch.full((B.Ntot,), float("nan"), dtype=torch.float64, device="cuda")
+    first = torch.empty(B.Ntot, dtype=torch.float64).pin_memory()
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    for tol in (1e-3, 1e-8):
+        x.fill_(float("nan"))
+        torch.cuda.synchronize()
+        got, _ = B.solve(x, rhs, tol=tol, maxit=5000)
+        with torch.cuda.stream(side):
+            first.copy_(x, non_blocking=True)
+        side.synchronize()
+        seen = first.numpy().copy()
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(seen, x.cpu().numpy())
+    np.testing.assert_array_equal(got, its)
+    np.testing.assert_array_equal(seen, ref)
+    del B
+
+
 @pytest.fixture(scope="module")
 def solved_mixed(plat, solved):
     probs, B, rhs, _, _, _ = solved
