@@ -114,15 +114,29 @@ __global__ __launch_bounds__(GT) void k_box_batch_update_r(BoxBatchUpdate u) {
 template <int LO, int HI, int MODE>
 int launch_ax(hipStream_t s, const BoxAxArgs<double>& a) {
   constexpr size_t lds = lds_bytes<LO, HI>();
-  if constexpr (lds > 65536)
-    BPX_HIP(hipFuncSetAttribute((const void*)k_box_batch_ax<LO, HI, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)lds));
   hipLaunchKernelGGL((k_box_batch_ax<LO, HI, MODE>), dim3((unsigned)a.nitems), dim3(256), lds, s, a);
   BPX_HIP(hipGetLastError());
   return BPX_OK;
 }
 
+// more than 64 KB of LDS has to be granted to a kernel
+template <int LO, int HI, int MODE>
+int grant_lds() {
+  constexpr size_t lds = lds_bytes<LO, HI>();
+  if constexpr (lds > 65536)
+    BPX_HIP(hipFuncSetAttribute((const void*)k_box_batch_ax<LO, HI, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)lds));
+  return BPX_OK;
+}
+
 }  // namespace
+
+int prepare_box_batch() {
+  if (int st = grant_lds<2, kLow, MODE_PLAIN>()) return st;
+  if (int st = grant_lds<2, kLow, MODE_FOLD>()) return st;
+  if (int st = grant_lds<kLow + 1, 16, MODE_PLAIN>()) return st;
+  return grant_lds<kLow + 1, 16, MODE_FOLD>();
+}
 
 int box_batch_class(int N) { return N + 1 <= kLow ? 0 : 1; }
 

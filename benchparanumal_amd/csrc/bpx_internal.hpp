@@ -418,7 +418,9 @@ int launch_box_update_r(hipStream_t s, const BoxGrid& g, int F, const BoxUpdateR
 
 // both kernels for the problems of a batch (FP64, trilinear; box_batch.hip):
 // cls = box_batch_class of their degrees, whose items are launched together;
-// items hold box_ax_elements and box_gather_elements elements
+// items hold box_ax_elements and box_gather_elements elements.
+// prepare_box_batch: before the first launch, outside of a stream capture
+int prepare_box_batch();
 int box_batch_class(int N);
 int launch_box_batch_ax(hipStream_t s, int cls, const BoxAxArgs<double>& a);
 struct BoxBatchUpdate {

@@ -46,6 +46,7 @@ int bp_batch_t::Setup(platform_t& p, const std::vector<MeshOpts>& opts, dfloat l
   BPX_HIP(hipEventCreateWithFlags(&ev1, hipEventDisableTiming));
   for (auto& e : evCount) BPX_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   BPX_HIP(hipHostMalloc((void**)&h_count, 2 * sizeof(int), hipHostMallocDefault));
+  if (int st = prepare_box_batch()) return st;
 
   // ---- per-problem host setup (bp5_t: mesh, masked ogs, GlobalToLocal)
   std::vector<mesh_t> meshes(nprob);

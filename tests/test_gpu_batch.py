@@ -203,3 +203,69 @@ def test_batch_mixed_deterministic_and_limits(plat, solved_mixed):
     assert (its3[capped] == 40).all() and (ups3[capped] == 3).all()
     with pytest.raises(capi.BpxError):
         B.solve_mixed(x3, rhs, tol=0.0, interval=16, maxit=40)
+
+
+# Degrees outside the 64 problems' 3..8, alone and together: both kernel
+# classes (degrees up to 8 and above, which holds more than 64 KB of LDS), the
+# degrees whose last elements own no layer or no row at all, uneven boxes, one
+# element along a direction, a problem without unknowns
+DEGREES = [
+    [(1, 5, 4, 3)], [(2, 4, 3, 3)], [(9, 2, 3, 2)], [(12, 2, 2, 1)], [(15, 2, 1, 2)],
+    [(10, 1, 2, 2), (11, 2, 1, 1), (13, 1, 1, 2), (14, 2, 2, 1)],
+    [(1, 6, 5, 4), (2, 1, 3, 2), (5, 3, 2, 2), (8, 2, 2, 3), (9, 2, 2, 2), (12, 1, 2, 2), (15, 2, 1, 1), (1, 1, 3, 2)],
+]
+
+
+@pytest.mark.parametrize("boxes", DEGREES, ids=lambda b: "-".join(str(p[0]) for p in b))
+def test_batch_of_any_degree(plat, boxes):
+    """solve, the mixed solve's residual and the iteration caps against the oracle's CG, whose
+    iterates a problem follows up to rounding (the 64 problems' bars)."""
+    probs = [{"N": N, "nx": nx, "ny": ny, "nz": nz, "perturb": 0.1, "seed": 40 + i}
+             for i, (N, nx, ny, nz) in enumerate(boxes)]
+    B = capi.Batch(plat, probs, lam=1.0)
+    rhs_h = capi.random_normal(3, B.Ntot)
+    rhs = torch.from_numpy(rhs_h).cuda()
+    x = torch.full_like(rhs, float("nan"))
+    its, rn = B.solve(x, rhs, tol=1e-8, maxit=5000)
+    xm = torch.full_like(rhs, float("nan"))
+    # (the FP32 recurrence can stall at the FP32 level once it has run out of
+    # unknowns, as it did before the box kernels: 24 of them at N = 1, interval
+    # 32. So what is checked of the mixed solve is its FP64 residual, the
+    # kernels of every degree's box operator, not that it converges.)
+    _, _, rel = B.solve_mixed(xm, rhs, tol=1e-10, interval=64, maxit=640)
+    x5 = torch.full_like(rhs, float("nan"))
+    its5, _ = B.solve(x5, rhs, tol=0.0, maxit=5)
+    x0 = torch.full_like(rhs, float("nan"))
+    its0, rn0 = B.solve(x0, rhs, tol=1e-8, maxit=0)
+    x, xm, x5, x0 = (v.cpu().numpy() for v in (x, xm, x5, x0))
+    np.testing.assert_array_equal(x0, np.zeros(B.Ntot))
+    for i, pr in enumerate(probs):
+        a, b = int(B.offsets[i]), int(B.offsets[i + 1])
+        if a == b:
+            assert its[i] == its0[i] == its5[i] == 0 and rn[i] == 0.0
+            continue
+        P = oracle_lib.Problem(bp=5, N=pr["N"], nx=pr["nx"], ny=pr["ny"], nz=pr["nz"], lam=1.0, perturb=0.1,
+                               seed=pr["seed"])
+        bi = rhs_h[a:b].copy()
+        nb = np.linalg.norm(bi)
+        xr, it_ref, _, _ = P.cg(bi, 5000, tol=1e-8)
+        assert abs(int(its[i]) - it_ref) <= 1, (i, int(its[i]), it_ref)
+        if int(its[i]) == it_ref:
+            assert np.linalg.norm(x[a:b] - xr) <= 1e-8 * np.linalg.norm(xr), i
+        assert np.linalg.norm(bi - P.operator(x[a:b].copy())) <= 1.01e-8 * max(nb, 1.0), i
+        # residuals of 1e-10 and more, by operators 1e-12 apart (1e-2 of them)
+        assert abs(np.linalg.norm(bi - P.operator(xm[a:b].copy())) / nb - rel[i]) <= 1e-2 * rel[i] + 1e-12, i
+        assert its0[i] == 0 and abs(rn0[i] - nb) <= 1e-14 * nb
+        x5r, it5, _, _ = P.cg(bi, 5, tol=0.0)
+        assert int(its5[i]) == it5
+        assert np.linalg.norm(x5[a:b] - x5r) <= 1e-10 * np.linalg.norm(x5r), i
+
+
+@pytest.mark.parametrize("N,elements", [(1, 64), (2, 28), (3, 16), (7, 4), (8, 3), (9, 2), (10, 2), (11, 1), (15, 1)])
+def test_batch_tuning_reports_the_launch(plat, N, elements):
+    """Per degree: the elements that a workgroup of about 256 lanes holds (one
+    lane per pencil) and a measured time of the FP64 Ax."""
+    B = capi.Batch(plat, [{"N": N, "nx": 2, "ny": 2, "nz": 2, "perturb": 0.1, "seed": 1}], lam=1.0)
+    (t,) = B.tuning()
+    assert t["N"] == N and t["elements_per_workgroup"] == elements
+    assert 0.0 < t["us"][0] < 1e5
