@@ -14,7 +14,7 @@ template <typename T>
 int launch_box_gather(hipStream_t s, const BoxGrid& g, int F, int K, const T* AqL, long long ldL, T* out,
                       long long ldo) {
   if (!AqL || !out) return set_error(BPX_ERR_INVALID_ARGUMENT, "box gather: null device pointer");
-  if (K < 1 || K > 65535) return set_error(BPX_ERR_INVALID_ARGUMENT, "box gather: K outside 1..65535");
+  if (K < 1 || K > kBoxMaxRhs) return set_error(BPX_ERR_INVALID_ARGUMENT, "box gather: K outside 1..65535");
 #define BPX_CALL(NQ) case NQ: return launch_box_gather_nq<T, NQ>(s, g, F, K, AqL, ldL, out, ldo);
   BPX_BOX_SWITCH(BPX_CALL)
 #undef BPX_CALL
@@ -24,6 +24,7 @@ template <typename T>
 int launch_box_ax(hipStream_t s, const BoxAxArgs<T>& a) {
   const BoxGrid& g = a.g;
   if (!a.q || !a.AqL) return set_error(BPX_ERR_INVALID_ARGUMENT, "box Ax: null device pointer");
+  if (a.K < 1 || a.K > kBoxMaxRhs) return set_error(BPX_ERR_INVALID_ARGUMENT, "box Ax: K outside 1..65535");
   const bool gll = a.op == BOX_OP_GLL;
   if (!a.eo || (gll ? !a.geo || (a.geoKind == BOX_GEO_TRILINEAR && !a.z) || (a.geoKind != BOX_GEO_TRILINEAR && !a.wJ) ||
                           (a.geoKind != BOX_GEO_STORED && !a.w)

@@ -319,6 +319,9 @@ template <typename T>
 int launch_ogs_gather_dot(hipStream_t s, int Nblocks, const int* blockStarts, const int* rowStarts,
                           const int* colIds, const T* q, T* gq, const T* p, double* part, int mode = 0);
 
+// right-hand sides of one box launch (the grid's third direction)
+constexpr int kBoxMaxRhs = 65535;
+
 // The same gather on a structured hex box, no maps (box_gather.hip): F
 // fields in [element][field][node] layout, K vectors of AqL ldL apart and of
 // out ldo apart. A vector of AqL must be smaller than 2^31 - 8 bytes.

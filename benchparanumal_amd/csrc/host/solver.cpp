@@ -635,8 +635,14 @@ int bp_t::Operator(const dfloat* o_q, dfloat* o_Aq) {
 
 template <typename T>
 int bp_t::GatherLocal(const T* o_AqL, T* o_Aq, int K) const {
-  if (haveBox && ogs.Ngather > 0)
-    return launch_box_gather<T>(platform->stream, box, Nfields, K, o_AqL, NLocal, o_Aq, ogs.Ngather);
+  if (haveBox && ogs.Ngather > 0) {
+    for (int k = 0; k < K; k += kBoxMaxRhs)
+      if (int st = launch_box_gather<T>(platform->stream, box, Nfields, std::min(kBoxMaxRhs, K - k),
+                                        o_AqL + (size_t)k * NLocal, NLocal, o_Aq + (size_t)k * ogs.Ngather,
+                                        ogs.Ngather))
+        return st;
+    return BPX_OK;
+  }
   for (int r = 0; r < K; ++r)  // one gather per vector, same maps
     if (int st = ogs.Gather<T>(*platform, o_Aq + (size_t)r * ogs.Ngather, o_AqL + (size_t)r * NLocal, 1)) return st;
   return BPX_OK;
@@ -932,12 +938,15 @@ int bp_t::AxLocalKrhs(int K, const dfloat* o_q, dfloat* o_AqL, int chunk) {
     return set_error(BPX_ERR_UNSUPPORTED, "bp: k right-hand sides are implemented for BP5 on hexahedra");
   if (haveKappa) return set_error(BPX_ERR_UNSUPPORTED, "bp: k right-hand sides use the constant coefficient");
   if (chunk == 0 && boxAx) {
-    if (K < 1 || K > 65535) return set_error(BPX_ERR_INVALID_ARGUMENT, "bp: K outside 1..65535");
-    BoxAxArgs<double> b = BoxArgs<double>(o_q, o_AqL);
-    b.K = K;
-    b.ldq = ogs.Ngather;
-    b.ldAq = NLocal;
-    return launch_box_ax<double>(platform->stream, b);
+    if (K < 1) return set_error(BPX_ERR_INVALID_ARGUMENT, "bp: K < 1");
+    for (int k = 0; k < K; k += kBoxMaxRhs) {
+      BoxAxArgs<double> b = BoxArgs<double>(o_q + (size_t)k * ogs.Ngather, o_AqL + (size_t)k * NLocal);
+      b.K = std::min(kBoxMaxRhs, K - k);
+      b.ldq = ogs.Ngather;
+      b.ldAq = NLocal;
+      if (int st = launch_box_ax<double>(platform->stream, b)) return st;
+    }
+    return BPX_OK;
   }
   AxArgs<double> a;
   a.N = mesh->N;
@@ -1018,7 +1027,11 @@ int bp_t::TimeKrhs(int K, int chunk, int launches, const dfloat* o_q, double* ou
 int bp_t::OperatorKrhs(int K, const dfloat* o_q, dfloat* o_Aq, int chunk) {
   if (K < 1) return set_error(BPX_ERR_INVALID_ARGUMENT, "bp: K < 1");
   constexpr size_t kKrhsBytes = (size_t)136 << 20;
-  const bool some = chunk == 0 && boxAx && bp == 5 && !haveKappa && ogs.Ngather > 0 && K <= 65535;
+  // (vectors that overlap other than one for one: every Ax before the first
+  // gather, which would overwrite what a later run reads)
+  const size_t n = (size_t)K * ogs.Ngather;
+  const bool apart = o_q == o_Aq || o_q + n <= o_Aq || o_Aq + n <= o_q;
+  const bool some = chunk == 0 && boxAx && bp == 5 && !haveKappa && ogs.Ngather > 0 && apart;
   const int kc = some ? (int)std::min<size_t>(K, std::max<size_t>(1, kKrhsBytes / ((size_t)NLocal * sizeof(double)))) : K;
   const size_t need = (size_t)NLocal * kc;
   if (o_AqLk.length() < need) {

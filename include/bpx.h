@@ -445,7 +445,9 @@ int bpx_bp_ax_local(bpx_bp b, const double* o_q, double* o_AqL);
 int bpx_bp_operator_f32(bpx_bp b, const float* o_q, float* o_Aq);
 /* No reference counterpart: bpN_t::Operator (BP/BP5/src/bp5Operator.cpp:29-85)
  * on K right-hand sides (BP5 only), stored one after another: o_q and o_Aq
- * hold K vectors of Ngather. k-RHS Ax, then one gather per right-hand side. */
+ * hold K vectors of Ngather, which may overlap in any way. k-RHS Ax, then the
+ * gather, a few right-hand sides at a time where the vectors are apart or the
+ * same. */
 int bpx_bp_operator_krhs(bpx_bp b, int K, int chunk, const double* o_q, double* o_Aq);
 /* No reference counterpart (the reference's BP5 coefficient is constant,
  * okl/bp5AxHex3D.okl:415-569): variable coefficient -div(kappa grad u) +

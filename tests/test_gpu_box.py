@@ -65,6 +65,27 @@ def test_box_gather_of_several_vectors(plat, N, K):
         np.testing.assert_array_equal(host(Aq[r * b.Ngather:(r + 1) * b.Ngather]), host(one))
 
 
+def test_krhs_beyond_a_launch(plat):
+    """More right-hand sides than a launch holds (65535), in more than one run
+    through the workspace: the same bits as a few at a time, also where the
+    results lie one vector behind the right-hand sides, in the same buffer."""
+    m = capi.Mesh(N=1, nx=3, ny=3, nz=3, perturb=0.1, seed=3)
+    b = capi.BP(plat, m, 5, lam=1.1)
+    K, n = 90000, b.Ngather
+    q = normal(4, K * n)
+    ref = torch.empty_like(q)
+    for k in range(0, K, 1000):
+        b.operator_krhs(q[k * n:(k + 1000) * n], ref[k * n:(k + 1000) * n], 1000)
+    Aq = torch.full_like(q, float("nan"))
+    b.operator_krhs(q, Aq, K)
+    np.testing.assert_array_equal(host(Aq), host(ref))
+    both = torch.cat((q, torch.full((n,), float("nan"), dtype=torch.float64, device="cuda")))
+    b.operator_krhs(both[:K * n], both[n:], K)
+    np.testing.assert_array_equal(host(both[n:]), host(ref))
+    b.operator_krhs(q, q, K)
+    np.testing.assert_array_equal(host(q), host(ref))
+
+
 # ---------------------------------------------------------- box_ax.hip ----
 def pair(bp, N, nx, ny, nz, affine=False, lam=1.3):
     kw = dict(N=N, nx=nx, ny=ny, nz=nz, affine=affine, perturb=0.0 if affine else 0.1, seed=7)
