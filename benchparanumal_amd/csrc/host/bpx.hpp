@@ -553,7 +553,7 @@ class bp_t : public solver_t {
   struct MixedWork {
     dlong N = -1;
     int maxit = 0;
-    deviceBuffer<double> Ax64, part_true, part_rr, part_pAp, hist_rr, hist_alpha, norm;
+    deviceBuffer<double> Ax64, b, part_true, part_rr, part_pAp, hist_rr, hist_alpha, norm;
     deviceBuffer<float> r32, p32, Ap32, c32;
     deviceBuffer<CgState> state;
   } mixed;

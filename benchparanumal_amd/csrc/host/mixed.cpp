@@ -41,6 +41,12 @@ int bp_t::SolveMixed(dfloat* o_x, const dfloat* o_b, double tol, int interval, i
     w.N = N;
     w.maxit = maxit;
   }
+  if (o_x < o_b + N && o_b < o_x + N) {  // x may be b: the corrections need b as it was
+    if (w.b.length() < (size_t)N)
+      if (int st = w.b.alloc(N)) return st;
+    BPX_HIP(hipMemcpyAsync(w.b.ptr(), o_b, (size_t)N * sizeof(double), hipMemcpyDeviceToDevice, s));
+    o_b = w.b.ptr();
+  }
   linAlg_t la(*platform);
   double nb = 0;
   if (int st = la.norm2(ogs.Ngather, o_b, &nb)) return st;

@@ -496,7 +496,7 @@ int bpx_bp_solve(bpx_bp b, double* o_x, double* o_r, double tol, int maxit, int 
  * dot accumulation) with an FP64 defect correction every `interval`
  * iterations (x += c; r = b - A x in FP64; the FP32 recurrence continues
  * from float(r)) until ||b - A x|| / ||b|| < tol. o_x: initial guess and
- * solution (device, FP64). stats (host, may be NULL): [defect corrections,
+ * solution (device, FP64; may be o_b). stats (host, may be NULL): [defect corrections,
  * FP32 iterations, final FP64 relative residual]. */
 int bpx_bp_solve_mixed(bpx_bp b, double* o_x, const double* o_b, double tol, int interval,
                        int maxit, double* stats);

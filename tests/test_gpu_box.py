@@ -173,6 +173,20 @@ def test_fixed_count_after_tolerance_solve(plat):
     np.testing.assert_array_equal(out[0][1], out[2][1])
 
 
+@pytest.mark.parametrize("bp,N", [(5, 4), (5, 15), (3, 3)])
+def test_mixed_solve_in_place(plat, bp, N):
+    """x and b in one buffer: the initial guess is b, and b the right-hand side
+    throughout, as with b in a buffer of its own."""
+    m = capi.Mesh(N=N, nx=2, ny=2, nz=2, perturb=0.1, seed=7, cubature=bp <= 4)
+    b = capi.BP(plat, m, bp, lam=1.0)
+    rhs = normal(6, b.Ngather)
+    x, both = rhs.clone(), rhs.clone()
+    st = b.solve_mixed(x, rhs, tol=1e-11, interval=16)
+    st2 = b.solve_mixed(both, both, tol=1e-11, interval=16)
+    assert st == st2 and st["rel_res"] < 1e-11
+    np.testing.assert_array_equal(host(both), host(x))
+
+
 @pytest.mark.parametrize("N,affine", [(1, False), (2, True), (4, False), (8, False), (12, True), (14, False), (15, False),
                                       (15, True)])
 def test_box_kappa_operator(plat, N, affine):
