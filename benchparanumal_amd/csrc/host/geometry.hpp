@@ -49,4 +49,24 @@ BPX_HD inline double vertex_weight(int v, double r, double s, double t) {
   return 0.125 * (1 + vertex_r(v) * r) * (1 + vertex_s(v) * s) * (1 + vertex_t(v) * t);
 }
 
+// The coefficients of r, s, t, rs, rt, st and rst of the trilinear map whose
+// values at the 8 vertices are V, and one pad. Differences along the edges
+// come first: they are exact, or rounded relative to themselves, where sums
+// of coordinates would be rounded relative to the distance from the origin
+// (which left the operator of N = 1 on 15 elements a side twice as far from
+// exact arithmetic as its stored factors are).
+BPX_HD inline void trilinear_coefficients(const double* V, double* c) {
+  const double r0 = V[1] - V[0], r1 = V[2] - V[3], r2 = V[5] - V[4], r3 = V[6] - V[7];  // edges along r
+  const double s0 = V[3] - V[0], s1 = V[2] - V[1], s2 = V[7] - V[4], s3 = V[6] - V[5];
+  const double t0 = V[4] - V[0], t1 = V[5] - V[1], t2 = V[6] - V[2], t3 = V[7] - V[3];
+  c[0] = 0.125 * ((r0 + r1) + (r2 + r3));
+  c[1] = 0.125 * ((s0 + s1) + (s2 + s3));
+  c[2] = 0.125 * ((t0 + t1) + (t2 + t3));
+  c[3] = 0.125 * ((r1 - r0) + (r3 - r2));  // rs
+  c[4] = 0.125 * ((r2 - r0) + (r3 - r1));  // rt
+  c[5] = 0.125 * ((s2 - s0) + (s3 - s1));  // st
+  c[6] = 0.125 * ((r3 - r2) - (r1 - r0));  // rst
+  c[7] = 0.0;
+}
+
 }  // namespace bpx

@@ -32,23 +32,9 @@ void mesh_t::TrilinearCoefficients(std::vector<double>& c) const {
   // (serial up to 2^16 elements: waking the threads costs more, 4 ms here)
 #pragma omp parallel for if (Nelements > (1 << 16))
   for (dlong e = 0; e < Nelements; ++e)
-    for (int d = 0; d < 3; ++d) {
-      const double* V = (d == 0 ? EX.data() : d == 1 ? EY.data() : EZ.data()) + (size_t)e * 8;
-      double* ce = &c[(size_t)e * 24 + 8 * d];
-      double S[4], D[4];  // over the two t faces: vertices in the order (-,-), (+,-), (+,+), (-,+) in (r, s)
-      for (int v = 0; v < 4; ++v) {
-        S[v] = 0.125 * (V[v] + V[v + 4]);
-        D[v] = 0.125 * (V[v + 4] - V[v]);
-      }
-      ce[0] = (S[1] - S[0]) + (S[2] - S[3]);  // r
-      ce[1] = (S[3] - S[0]) + (S[2] - S[1]);  // s
-      ce[2] = (D[0] + D[1]) + (D[2] + D[3]);  // t
-      ce[3] = (S[2] - S[1]) - (S[3] - S[0]);  // rs
-      ce[4] = (D[1] - D[0]) + (D[2] - D[3]);  // rt
-      ce[5] = (D[3] - D[0]) + (D[2] - D[1]);  // st
-      ce[6] = (D[2] - D[1]) - (D[3] - D[0]);  // rst
-      ce[7] = 0.0;
-    }
+    for (int d = 0; d < 3; ++d)
+      trilinear_coefficients((d == 0 ? EX.data() : d == 1 ? EY.data() : EZ.data()) + (size_t)e * 8,
+                             &c[(size_t)e * 24 + 8 * d]);
 }
 
 bool mesh_t::NodesAreTrilinear() const {

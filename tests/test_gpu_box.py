@@ -115,6 +115,24 @@ def test_box_operator_matches_oracle(plat, bp, N, affine):
     assert abs(qAq - float(np.dot(q, host(A)))) <= 1e-13 * np.abs(q * host(A)).sum()
 
 
+@pytest.mark.parametrize("on_device", [False, True])
+@pytest.mark.parametrize("bp", [1, 3, 5, 6])
+def test_box_operator_away_from_the_origin(plat, bp, on_device):
+    """Elements 500 times smaller than their distance from the origin. At N = 1
+    the oracle's factors are exact differences of the vertices, so its rounding
+    is that of 8 nodes' sums, and so must the kernel's be: about 20 roundings
+    of 1.1e-16 where coefficients from rounded coordinate sums are off by
+    500 * 1.1e-16 = 6e-14 each."""
+    kw = dict(N=1, nx=16, ny=12, nz=10, lo=(64.0, -64.0, 64.0), perturb=0.1, seed=7)
+    m = capi.Mesh(cubature=bp <= 4, platform=plat if on_device else None, **kw)
+    P = oracle_lib.Problem(bp=bp, lam=1.3, **kw)
+    b = capi.BP(plat, m, bp, lam=1.3)
+    q = np.random.default_rng(1).standard_normal(b.Ngather)
+    A = torch.full((b.Ngather,), float("nan"), dtype=torch.float64, device="cuda")
+    b.operator(torch.from_numpy(q).cuda(), A)
+    assert rel_err(host(A), P.operator(q)) <= 5e-15
+
+
 @pytest.mark.parametrize("geometry", [0, 1])
 @pytest.mark.parametrize("N,affine", [(N, False) for N in range(1, 16)] + [(2, True), (7, True), (11, True)])
 def test_box_operator_f32(plat, N, affine, geometry):
