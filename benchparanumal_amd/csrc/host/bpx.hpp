@@ -169,6 +169,7 @@ class mesh_t {
   bool onDevice = false;
   platform_t* devPlatform = nullptr;
   deviceBuffer<double> o_x, o_y, o_z, o_wJ, o_ggeo, o_cubwJ, o_cubggeo;
+  deviceBuffer<double> o_tri;  // TrilinearCoefficients (non-affine)
   deviceBuffer<hlong> o_globalIds;
 
   // quad, triangle and tetrahedral boxes (host/mesh_other.cpp)

@@ -440,12 +440,14 @@ int bp_t::Setup(platform_t& p, mesh_t& m, int bp_, dfloat lambda_) {
   }
   boxAx = haveBox && (bp == 5 || bp == 6);
   boxCub = haveBox && bp <= 4 && o_eo.length() > 0;
-  if (boxAx || boxCub) {  // one upload: the maps, then the 1D data
+  if (boxAx || boxCub) {
+    // the maps (a device mesh has them; on 375,000 elements of N = 1 forming
+    // and sending them from here took 34 of the setup's 39 ms), then the 1D data
+    const size_t nmap = affine ? 0 : (size_t)24 * m.Nelements;
     std::vector<double> t, eo;
-    if (!affine) m.TrilinearCoefficients(t);
-    auto append = [&t](const std::vector<double>& v) {
+    auto append = [&t, nmap](const std::vector<double>& v) {
       t.insert(t.end(), v.begin(), v.end());
-      return t.size() - v.size();
+      return nmap + t.size() - v.size();
     };
     boxZ = append(boxCub ? m.cubr : m.gllz);
     boxW = append(boxCub ? m.cubw : m.gllw);
@@ -453,7 +455,15 @@ int bp_t::Setup(platform_t& p, mesh_t& m, int bp_, dfloat lambda_) {
       if (int st = box_even_odd_table(m, eo)) return st;
       boxEo = append(eo);
     }
-    if (int st = o_boxTab.upload(t, s)) return st;
+    if (int st = o_boxTab.alloc(nmap + t.size())) return st;
+    BPX_HIP(hipMemcpy(o_boxTab.ptr() + nmap, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
+    if (nmap > 0 && m.onDevice) {
+      BPX_HIP(hipMemcpyAsync(o_boxTab.ptr(), m.o_tri.ptr(), nmap * sizeof(double), hipMemcpyDeviceToDevice, s));
+    } else if (nmap > 0) {
+      std::vector<double> tri;
+      m.TrilinearCoefficients(tri);
+      BPX_HIP(hipMemcpy(o_boxTab.ptr(), tri.data(), nmap * sizeof(double), hipMemcpyHostToDevice));
+    }
   }
   if (int st = m.onDevice ? PrepareFusedDevice() : PrepareFused()) return st;
   if (boxAx && bp == 5 && affine) fused = true;

@@ -156,6 +156,16 @@ __global__ void k_geo_affine(dlong Nel, const double* __restrict__ EX, const dou
   for (int c = 0; c < 6; ++c) ggeo[(size_t)e * 6 + c] = g[c];
 }
 
+// the trilinear maps' coefficients (mesh_t::TrilinearCoefficients)
+__global__ void k_trilinear(dlong Nel, const double* __restrict__ EX, const double* __restrict__ EY,
+                            const double* __restrict__ EZ, double* __restrict__ c) {
+  const dlong e = (dlong)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (e >= Nel) return;
+  trilinear_coefficients(EX + (size_t)e * 8, c + (size_t)e * 24);
+  trilinear_coefficients(EY + (size_t)e * 8, c + (size_t)e * 24 + 8);
+  trilinear_coefficients(EZ + (size_t)e * 8, c + (size_t)e * 24 + 16);
+}
+
 // Cubature factors, in four passes over a chunk of elements (e0 ..
 // e0 + Nc - 1) with three scratch arrays, as the host does per element:
 // the 9 derivatives at the GLL nodes (a0: [el][f][Np]), interpolated to the
@@ -430,6 +440,10 @@ int mesh_t::SetupDevice(platform_t& p, const MeshOpts& o) {
     if (int st = o_ggeo.alloc(NL * 6)) return st;
     hipLaunchKernelGGL(k_geo_nodes, dim3(blocks_for(NL)), dim3(kT), 0, s, Nelements, Nq, dD.ptr(), dw.ptr(),
                        o_x.ptr(), o_y.ptr(), o_z.ptr(), o_wJ.ptr(), o_ggeo.ptr(), bad.ptr());
+    BPX_HIP(hipGetLastError());
+    if (int st = o_tri.alloc((size_t)Nelements * 24)) return st;
+    hipLaunchKernelGGL(k_trilinear, dim3(blocks_for(Nelements)), dim3(kT), 0, s, Nelements, dEX.ptr(), dEY.ptr(),
+                       dEZ.ptr(), o_tri.ptr());
   }
   BPX_HIP(hipGetLastError());
   int hbad = 0;
