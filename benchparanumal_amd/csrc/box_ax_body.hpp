@@ -37,7 +37,9 @@ namespace {
 // A[n][m] = (D[n][m] - D[n][NQ-1-m])/2 for m < NQ/2. Rows come through
 // scalar loads. Up to Nq = 8 the table (64 scalar registers in FP64) may
 // stay in registers; beyond, each row is requested where it is used.
-template <typename T, int NQ>
+//
+// BY_ROWS: D itself, which follows the table, in sums of Nq terms in order.
+template <typename T, int NQ, bool BY_ROWS>
 struct EvenOdd {
   static constexpr int H = NQ / 2, ODD = NQ & 1, ROWS = H + ODD;
   typedef const __attribute__((address_space(4))) T* cptr;
@@ -73,6 +75,16 @@ struct EvenOdd {
   }
 
   __device__ static inline void apply(cptr tab, const T (&x)[NQ], T (&y)[NQ]) {
+    if constexpr (BY_ROWS) {
+#pragma unroll
+      for (int n = 0; n < NQ; ++n) {
+        T a = 0;
+#pragma unroll
+        for (int m = 0; m < NQ; ++m) a = fmad(tab[(ROWS + n) * NQ + m], x[m], a);
+        y[n] = a;
+      }
+      return;
+    }
     T xe[H], xo[H];
 #pragma unroll
     for (int m = 0; m < H; ++m) {
@@ -98,6 +110,15 @@ struct EvenOdd {
   }
 
   __device__ static inline void apply_transposed(cptr tab, const T (&x)[NQ], T (&y)[NQ]) {
+    if constexpr (BY_ROWS) {
+#pragma unroll
+      for (int n = 0; n < NQ; ++n) y[n] = T(0);
+#pragma unroll
+      for (int m = 0; m < NQ; ++m)
+#pragma unroll
+        for (int n = 0; n < NQ; ++n) y[n] = fmad(tab[(ROWS + m) * NQ + n], x[m], y[n]);
+      return;
+    }
     T ye[H], yo[H], ym = 0;
 #pragma unroll
     for (int n = 0; n < H; ++n) ye[n] = yo[n] = T(0);
@@ -147,6 +168,17 @@ __device__ inline void element_sync() {
 // GEO: where the factors come from
 enum { GEO_TRILINEAR = 0, GEO_AFFINE = 1, GEO_STORED = 2 };
 
+// D by rows where the even-odd parts cost bits: up to Nq = 6 they take a
+// tenth off the operations, but rounded to FP32 they leave the operator up to
+// 20% (Nq = 6, affine) farther from exact arithmetic than rows do, from Nq = 7
+// on 5 to 25% closer. In FP64, where the formed factors are far closer than
+// the stored ones, only affine elements (whose factors are the stored ones)
+// show it, 6% at Nq = 6.
+template <typename T, int NQ, int GEO>
+constexpr bool box_by_rows() {
+  return sizeof(T) == 4 ? NQ <= 6 : GEO == GEO_AFFINE && NQ == 6;
+}
+
 // LDS of one workgroup: the two pencil buffers and the sums
 template <typename T, int NQ, int MODE>
 struct BoxAxLds {
@@ -161,7 +193,7 @@ template <typename T, int NQ, int GEO, bool KAPPA, int MODE, bool BATCH>
 __device__ inline void box_ax_body(BoxAxArgs<T> a, int per_xcd, BoxAxLds<T, NQ, MODE>& lds) {
   constexpr int N = NQ - 1, NQ2 = NQ * NQ, NP = NQ2 * NQ, EPB = box_epb(NQ);
   constexpr int LK = NQ2 + 8, LE = NQ * LK, S = (int)sizeof(T);
-  using EO = EvenOdd<T, NQ>;
+  using EO = EvenOdd<T, NQ, box_by_rows<T, NQ, GEO>()>;
   typedef typename EO::cptr cptr;
   T* const s_b = lds.b;
   T* const s_c = lds.c;
@@ -194,8 +226,8 @@ __device__ inline void box_ax_body(BoxAxArgs<T> a, int per_xcd, BoxAxLds<T, NQ, 
     grp = item->e0 / EPB;
     row0v = pr->off;
     a.z = a.tab + pr->tab;
-    a.w = a.z + NQ;
-    a.eo = a.w + NQ;
+    a.w64 = a.z + NQ;
+    a.eo = a.w64 + NQ;
     a.geo += 24 * pr->el0;
     a.AqL += pr->loc;
     if constexpr (MODE == MODE_FOLD) {
@@ -302,13 +334,18 @@ __device__ inline void box_ax_body(BoxAxArgs<T> a, int per_xcd, BoxAxLds<T, NQ, 
       for (int c = 0; c < 6; ++c) ga[c] = a.geo[6 * (size_t)e + c];
       gw = a.wJ[e];
     }
-    const T wij = GEO == GEO_STORED ? T(0) : a.w[ai] * a.w[bj];
-    T zk[NQ], wk[NQ];  // uniform: scalar loads
+    // a node's weight is formed in FP64 and, in FP32, rounded once: rounded
+    // 1D weights shift all nodes of a kind at once (N = 2, 1/3 and 4/3: half of
+    // the FP32 operator's error; N = 7, affine: a third), for 0.5% of its time
+    typedef const __attribute__((address_space(4))) double* wptr;
+    const double wij = GEO == GEO_STORED ? 0.0 : a.w64[ai] * a.w64[bj];
+    T zk[NQ];  // uniform: scalar loads
+    double wk[NQ];
     if constexpr (GEO != GEO_STORED) {
 #pragma unroll
       for (int k = 0; k < NQ; ++k) {
         if constexpr (GEO == GEO_TRILINEAR) zk[k] = ((cptr)a.z)[k];
-        wk[k] = ((cptr)a.w)[k];
+        wk[k] = ((wptr)a.w64)[k];
       }
     }
     const T* kap = nullptr;
@@ -329,11 +366,11 @@ __device__ inline void box_ax_body(BoxAxArgs<T> a, int per_xcd, BoxAxLds<T, NQ, 
       if constexpr (GEO == GEO_TRILINEAR) {
         T kv = T(1);
         if constexpr (KAPPA) kv = kap[(size_t)k * kstep];
-        map.template flux<KAPPA>(zk[k], wij * wk[k], kv, qr, qs, qt, Gr, Gs, Gt, W);
+        map.template flux<KAPPA>(zk[k], (T)(wij * wk[k]), kv, qr, qs, qt, Gr, Gs, Gt, W);
       } else {
         T g[6];
         if constexpr (GEO == GEO_AFFINE) {
-          const T w = wij * wk[k];
+          const T w = (T)(wij * wk[k]);
           T wg = w;
           if constexpr (KAPPA) wg *= kap[(size_t)k * kstep];
 #pragma unroll

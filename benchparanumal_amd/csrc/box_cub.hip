@@ -129,16 +129,18 @@ __global__ __launch_bounds__((NQ + 1) * (NQ + 1) * box_epb(NQ + 1))
   const int so = ls * TILE + lh * PS + lw;       // s-line, step PR
   const int to = ls * TILE + lh * PR + lw;       // t-line, step PS
   const T* const eo = a.eo;
+  const double* const eo64 = a.eo64;
 
   auto interp = [&](const T(&x)[NQ], T(&y)[MQ]) { eo_apply<MQ, NQ, 1>(eo + ET::I, x, [&](int n, T v) { y[n] = v; }); };
   auto project = [&](const T(&x)[MQ], T(&y)[NQ]) { eo_apply<NQ, MQ, 1>(eo + ET::IT, x, [&](int n, T v) { y[n] = v; }); };
   auto diff = [&](const T(&x)[MQ], T(&y)[MQ]) { eo_apply<MQ, MQ, -1>(eo + ET::D, x, [&](int n, T v) { y[n] = v; }); };
   auto diff_t = [&](const T(&x)[MQ], T(&y)[MQ]) { eo_apply<MQ, MQ, -1>(eo + ET::DT, x, [&](int n, T v) { y[n] = v; }); };
 
-  // Along t, FP32 up to Nq = 8 (where the stored-factor kernel has it so): D
-  // by rows. Its even-odd parts round differently, which at p = 5 makes the
-  // operator's error 9% larger (2.22e-7 against 2.04e-7; this way 2.00e-7).
-  constexpr bool ROWS = sizeof(T) == 4 && NQ <= 8;
+  // Along t, FP32 up to Nq = 6: D by rows. Its even-odd parts round
+  // differently, which at p = 5 makes the operator's error 9% larger (2.22e-7
+  // against 2.04e-7; this way 2.00e-7); at p = 6 and 7 they are as close and
+  // faster (24^3, p = 7: mixed solve 88 -> 85.5 ms).
+  constexpr bool ROWS = sizeof(T) == 4 && NQ <= 6;
   auto diff_line = [&](const T(&x)[MQ], T(&y)[MQ]) {
     if constexpr (ROWS) {
       uniform_rows<MQ, MQ>(eo + ET::ROWS, [&](int n, const T* r) {
@@ -162,6 +164,23 @@ __global__ __launch_bounds__((NQ + 1) * (NQ + 1) * box_epb(NQ + 1))
       diff_t(x, v);
 #pragma unroll
       for (int m = 0; m < MQ; ++m) y[m] += v[m];
+    }
+  };
+
+  // FP32 up to Nq = 8: the last projection in FP64 (which issues at the same
+  // rate), its result rounded once. It pays for the factors, whose 7 values a
+  // point are formed in FP32 instead of rounded from FP64 ones: without it the
+  // operator's error is up to 3.5% larger than with stored factors (p = 7),
+  // with it smaller at every degree.
+  constexpr bool END64 = sizeof(T) == 4 && NQ <= 8;
+  auto project_last = [&](const T(&x)[MQ], T(&y)[NQ]) {
+    if constexpr (END64) {
+      double xd[MQ];
+#pragma unroll
+      for (int m = 0; m < MQ; ++m) xd[m] = x[m];
+      eo_apply<NQ, MQ, 1>(eo64 + ET::IT, xd, [&](int n, double v) { y[n] = (T)v; });
+    } else {
+      project(x, y);
     }
   };
 
@@ -323,7 +342,7 @@ __global__ __launch_bounds__((NQ + 1) * (NQ + 1) * box_epb(NQ + 1))
     T v[MQ], y[NQ];
 #pragma unroll
     for (int m = 0; m < MQ; ++m) v[m] = Ak[m * PS];
-    project(v, y);
+    project_last(v, y);
     if constexpr (MODE != MODE_PLAIN && sizeof(T) == 4) {  // q.Aq from the rounded results, as the rows see them
       if (active)
 #pragma unroll

@@ -26,9 +26,9 @@ int launch_box_ax(hipStream_t s, const BoxAxArgs<T>& a) {
   if (!a.q || !a.AqL) return set_error(BPX_ERR_INVALID_ARGUMENT, "box Ax: null device pointer");
   if (a.K < 1 || a.K > kBoxMaxRhs) return set_error(BPX_ERR_INVALID_ARGUMENT, "box Ax: K outside 1..65535");
   const bool gll = a.op == BOX_OP_GLL;
-  if (!a.eo || (gll ? !a.geo || (a.geoKind == BOX_GEO_TRILINEAR && !a.z) || (a.geoKind != BOX_GEO_TRILINEAR && !a.wJ) ||
-                          (a.geoKind != BOX_GEO_STORED && !a.w)
-                    : !a.geo64 || !a.z64 || !a.w64))
+  const bool geo = gll ? a.geo && (a.geoKind == BOX_GEO_TRILINEAR ? a.z : a.wJ) && (a.geoKind == BOX_GEO_STORED || a.w64)
+                       : a.geo64 && a.z64 && a.w64 && (sizeof(T) == 8 || a.eo64);
+  if (!a.eo || !geo)
     return set_error(BPX_ERR_INVALID_ARGUMENT, "box Ax: null geometry/operator pointer");
   if (!gll && (a.geoKind != BOX_GEO_TRILINEAR || a.kappa || a.K != 1))
     return set_error(BPX_ERR_UNSUPPORTED, "box Ax: the cubature operators have constant coefficients and one right-hand side");

@@ -361,9 +361,10 @@ struct BoxAxArgs {
   const T* geo = nullptr;    // 24 map coefficients per element, 6 factors per element, or 6 per node (FP32 only)
   const T* wJ = nullptr;     // J per element (affine), wJ per node (stored)
   const T* z = nullptr;      // GLL nodes (trilinear)
-  const T* w = nullptr;      // GLL weights (trilinear, affine)
-  // cubature operators instead: the map coefficients, points and weights
-  const double *geo64 = nullptr, *z64 = nullptr, *w64 = nullptr;
+  const double* w64 = nullptr;  // GLL weights (trilinear, affine)
+  // cubature operators instead of geo and z: the map coefficients, the points
+  // (w64: their weights) and, for FP32, the FP64 EoTables
+  const double *geo64 = nullptr, *z64 = nullptr, *eo64 = nullptr;
   const T* eo = nullptr;     // even-odd table of D (EvenOdd, box_ax_body.hpp), or EoTables (even_odd.hpp)
   const T* kappa = nullptr;  // coefficient on the node lattice (FP64), or null
   T lambda = 0;

@@ -602,7 +602,7 @@ class bp_t : public solver_t {
   int fp32Geometry = 0;
   int SetFp32Geometry(int mode);
   int SetCubForm(int form);
-  deviceBuffer<float> o_wJ32, o_ggeo32, o_gllw32, o_D32, o_I32, o_MM32, o_invV32, o_AqL32;
+  deviceBuffer<float> o_wJ32, o_ggeo32, o_D32, o_I32, o_MM32, o_invV32, o_AqL32;
   deviceBuffer<float> o_eo32;
   // nodal coordinates for the forcing (created on first use)
   deviceBuffer<double> o_x, o_y, o_z, o_gllwRhs;

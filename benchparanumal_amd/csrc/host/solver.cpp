@@ -73,6 +73,7 @@ int hip_error(hipError_t e, const char* what) {
 int box_even_odd_table(const mesh_t& m, std::vector<double>& t) {
   if (!even_odd_rows(m.D.data(), m.Nq, m.Nq, -1, t))
     return set_error(BPX_ERR_INVALID_ARGUMENT, "bp: the derivative matrix is not antisymmetric");
+  t.insert(t.end(), m.D.begin(), m.D.end());
   return BPX_OK;
 }
 
@@ -529,6 +530,7 @@ BoxAxArgs<T> bp_t::BoxArgs(const T* o_q, T* o_AqL) const {
     a.geo64 = o_boxTab.ptr();
     a.z64 = o_boxTab.ptr() + boxZ;
     a.w64 = o_boxTab.ptr() + boxW;
+    a.eo64 = o_eo.ptr();
     if constexpr (std::is_same<T, double>::value)
       a.eo = o_eo.ptr();
     else
@@ -538,14 +540,14 @@ BoxAxArgs<T> bp_t::BoxArgs(const T* o_q, T* o_AqL) const {
     a.geo = affine ? o_ggeo.ptr() : o_boxTab.ptr();
     a.wJ = o_wJ.ptr();
     a.z = o_boxTab.ptr() + boxZ;
-    a.w = o_boxTab.ptr() + boxW;
+    a.w64 = o_boxTab.ptr() + boxW;
     a.eo = o_boxTab.ptr() + boxEo;
     a.kappa = haveKappa ? o_kappa.ptr() : nullptr;
   } else {
     a.geoKind = affine ? BOX_GEO_AFFINE : tri32 ? BOX_GEO_TRILINEAR : BOX_GEO_STORED;
     a.geo = o_ggeo32.ptr();
     a.wJ = a.z = o_wJ32.ptr();  // the GLL nodes with the trilinear maps
-    a.w = o_gllw32.ptr();
+    a.w64 = o_boxTab.ptr() + boxW;
     a.eo = o_boxEo32.ptr();
   }
   a.lambda = (T)lambda;
@@ -1067,7 +1069,7 @@ int bp_t::OperatorDot32(const float* o_q, float* o_Aq, double* part, int* npart)
     if (int st = launch_box_ax<float>(platform->stream, a)) return st;
     return GatherLocal<float>(o_AqL32.ptr(), o_Aq);
   }
-  if (int st = ax<float>(o_q, o_AqL32.ptr(), o_wJ32.ptr(), o_ggeo32.ptr(), o_gllw32.ptr(), o_D32.ptr(),
+  if (int st = ax<float>(o_q, o_AqL32.ptr(), o_wJ32.ptr(), o_ggeo32.ptr(), nullptr, o_D32.ptr(),
                          o_I32.ptr(), o_MM32.ptr(), o_invV32.ptr()))
     return st;
   *npart = ogs_gather_partials(ogs.NrowBlocksT);
@@ -1352,14 +1354,15 @@ int bp_t::Prepare32() {
   } else if (bp == 5 && !affine && fp32Geometry == 0) {
     // the FP32 operator forms its geometric factors from the elements'
     // trilinear maps: 96 B per element instead of 28 B per node
-    std::vector<double> tri;
-    m.TrilinearCoefficients(tri);
-    if ((st = cvt(o_wJ32, m.gllz)) || (st = cvt(o_ggeo32, tri)) || (st = cvt(o_gllw32, m.gllw))) return st;
+    const size_t nmap = (size_t)24 * m.Nelements;
+    if ((st = cvt(o_wJ32, m.gllz)) || (st = o_ggeo32.alloc(nmap)) ||
+        (st = launch_to_f32(s, nmap, o_boxTab.ptr(), o_ggeo32.ptr())))
+      return st;
     tri32 = 1;
   } else if ((st = mesh->EnsureHost())) {
     return st;
   } else if (bp == 5) {
-    if ((st = cvt(o_wJ32, m.wJ)) || (st = cvt(o_ggeo32, m.ggeo)) || (st = cvt(o_gllw32, m.gllw))) return st;
+    if ((st = cvt(o_wJ32, m.wJ)) || (st = cvt(o_ggeo32, m.ggeo))) return st;
   } else if (bp == 1 || bp == 2) {
     if ((st = cvt(o_wJ32, affine ? m.wJ : m.cubwJ)) || (st = cvt(o_I32, m.cubInterp)) || (st = cvt(o_MM32, m.MM)))
       return st;
@@ -1407,7 +1410,7 @@ int bp_t::Operator32(const float* o_q, float* o_Aq) {
   if (int st = Prepare32()) return st;
   const int st = BoxAx<float>()
                      ? launch_box_ax<float>(platform->stream, BoxArgs<float>(o_q, o_AqL32.ptr()))
-                     : ax<float>(o_q, o_AqL32.ptr(), o_wJ32.ptr(), o_ggeo32.ptr(), o_gllw32.ptr(), o_D32.ptr(),
+                     : ax<float>(o_q, o_AqL32.ptr(), o_wJ32.ptr(), o_ggeo32.ptr(), nullptr, o_D32.ptr(),
                                  o_I32.ptr(), o_MM32.ptr(), o_invV32.ptr());
   if (st) return st;
   return GatherLocal<float>(o_AqL32.ptr(), o_Aq);

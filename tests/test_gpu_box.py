@@ -220,6 +220,52 @@ def test_box_kappa_operator(plat, N, affine):
     assert rel_err(host(A), P.operator(q)) <= 1e-12
 
 
+def f32_error(plat, bp, N, affine, geometry):
+    """Relative error (2-norm) of the FP32 operator on FP32 values over 8 boxes,
+    against the FP64 operator, whose own is a millionth of it."""
+    n = max(2, round(20.0 / (N + 1)))
+    e2 = r2 = 0.0
+    for seed in range(1, 9):
+        m = capi.Mesh(N=N, nx=n + 1, ny=n, nz=n, affine=affine, cubature=bp <= 4, perturb=0.0 if affine else 0.1,
+                      seed=seed, dim=(2.0, 2.0 + 0.1 * seed, 2.0 + 0.03 * seed))
+        b = capi.BP(plat, m, bp, lam=1.3)
+        b.set_fp32_geometry(geometry)
+        q = normal(seed, b.Ngather).float()
+        A = torch.full_like(q, float("nan"))
+        ref = torch.zeros(b.Ngather, dtype=torch.float64, device="cuda")
+        b.operator_f32(q, A)
+        b.operator(q.double(), ref)
+        e2 += float(((A.double() - ref) ** 2).sum())
+        r2 += float((ref * ref).sum())
+    return (e2 / r2) ** 0.5
+
+
+# 1e-9 times: f32_error of the kernels that read every node's factors or, for
+# trilinear ones, summed D in order with rounded weights (N = 1..15)
+F32_BEFORE = {
+    "trilinear": (59.7, 123.7, 91.5, 104.1, 108.1, 111.5, 142.2, 132.3, 143.3, 171.3, 149.5, 160.6, 160.2, 164.1, 179.4),
+    "stored": (54.4, 53.8, 59.5, 73.6, 78.7, 82.3, 94.5, 96.5, 100.1, 114.8, 110.3, 117.8, 120.4, 135.0, 131.9),
+    "affine": (58.9, 116.9, 68.0, 84.2, 80.4, 87.6, 112.5, 104.6, 109.4, 146.7, 120.4, 130.8, 130.6, 133.8, 151.0),
+}
+
+
+@pytest.mark.parametrize("N", range(1, 16))
+@pytest.mark.parametrize("factors", ["trilinear", "stored", "affine"])
+def test_box_operator_f32_error(plat, factors, N):
+    """FP32 BP5 is no farther from exact arithmetic than the kernels before it,
+    within the 3% by which one set of boxes differs from another."""
+    err = f32_error(plat, 5, N, factors == "affine", int(factors == "stored"))
+    assert err <= 1.03e-9 * F32_BEFORE[factors][N - 1]
+
+
+@pytest.mark.parametrize("bp", [1, 3])
+@pytest.mark.parametrize("N", range(1, 16))
+def test_box_cub_operator_f32_error(plat, bp, N):
+    """FP32 BP1 and BP3 with formed factors are no farther from exact
+    arithmetic than with the stored ones rounded to FP32."""
+    assert f32_error(plat, bp, N, False, 0) <= f32_error(plat, bp, N, False, 1)
+
+
 # --------------------------------------------------------- box_cub.hip ----
 def cub_pair(bp, N, nx, ny, nz, lam=1.3):
     kw = dict(N=N, nx=nx, ny=ny, nz=nz, perturb=0.1, seed=7)
