@@ -510,6 +510,7 @@ class bp_t : public solver_t {
   // BP1-BP4 on the box, trilinear elements (box_cub.hip), unless a kernel
   // form is set: those read the stored factors
   bool boxCub = false;
+  bool StoredPays() const;  // where the stored factors are the faster ones
   bool OnBox() const { return boxAx || (boxCub && cubForm == CUB_FORM_AUTO); }
   int BoxOp() const { return bp >= 5 ? BOX_OP_GLL : bp >= 3 ? BOX_OP_STIFF : BOX_OP_MASS; }
   int BoxPartials() const { return box_ax_partials(box, Nfields, BoxOp()); }
@@ -524,9 +525,20 @@ class bp_t : public solver_t {
   // whether precision T's operator runs on box_ax.hip or box_cub.hip
   template <typename T>
   bool BoxAx() const {
-    if (bp <= 4) return OnBox() && (sizeof(T) == 8 || fp32Geometry == 0);
+    if (bp <= 4) return OnBox() && (sizeof(T) == 8 || (fp32Geometry == 0 && !StoredPays32()));
     return sizeof(T) == 8 ? boxAx : haveBox && bp == 5;
   }
+  // the same for FP32: BP1 (whose one factor per point is half as large),
+  // operator, stored -> formed: N = 1, 2e5 nodes 7.5 -> 7.8 us, 1e6 11.6 ->
+  // 16.1; N = 2, 2e5 8.0 -> 6.7, 1e6 10.9 -> 11.8, 7e6 45.5 -> 48.9
+  bool StoredPays32() const { return bp == 1 && mesh->N <= 2 && NLocal > (mesh->N << 17); }
+  // Folded, the direction update reads r and the old direction once per
+  // element that holds a node: 8 times a row at N = 1 and 3.4 times at N = 2,
+  // which costs more than the kernel it saves once they leave the L2s. 64
+  // iterations, folded / not: N = 2, BP6, 2e5 nodes a field (5 MB of local
+  // values) 1.22 / 1.38 ms, 1e6 (24 MB) 3.58 / 3.30, 7e6 30.0 / 22.6; N = 1,
+  // BP3, 2e5 (1.6 MB) 1.18 / 1.32, 1e6 (8 MB) 3.36 / 3.02.
+  bool FoldPays(size_t bytes) const { return mesh->N > 2 || (size_t)NLocal * bytes <= ((size_t)6 << 20); }
   // The CG operator in two kernels per iteration, the Ax with the direction
   // update and the gather with the residual update, on the reference rows
   // unless pinned off: boxFused64 (FP64), tuning.fused32 (FP32 and, for

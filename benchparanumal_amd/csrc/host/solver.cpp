@@ -439,8 +439,8 @@ int bp_t::Setup(platform_t& p, mesh_t& m, int bp_, dfloat lambda_) {
     if (!eo.empty())
       if (int st = o_eo.upload(eo, s)) return st;
   }
-  boxAx = haveBox && (bp == 5 || bp == 6);
-  boxCub = haveBox && bp <= 4 && o_eo.length() > 0;
+  boxAx = haveBox && (bp == 5 || bp == 6) && !StoredPays();
+  boxCub = haveBox && bp <= 4 && o_eo.length() > 0 && !StoredPays();
   if (boxAx || boxCub) {
     // the maps (a device mesh has them; on 375,000 elements of N = 1 forming
     // and sending them from here took 34 of the setup's 39 ms), then the 1D data
@@ -470,6 +470,23 @@ int bp_t::Setup(platform_t& p, mesh_t& m, int bp_, dfloat lambda_) {
   if (boxAx && bp == 5 && affine) fused = true;
   if (int st = Tune()) return st;
   return p.finish();
+}
+
+// At the lowest degrees few points share an element's map, and forming their
+// factors, for each field again, costs more than reading them once vectors and
+// factors leave the caches. Measured per operator, stored -> formed:
+//  - N = 1: BP1 1e6 nodes 16.2 -> 18.2 us, 3e6 34.7 -> 43.4; BP2 2e5 nodes a
+//    field 11.8 -> 13.9, 3e6 102 -> 128; BP4 2e5 19.4 -> 22.3, 1e6 63 -> 88;
+//    BP6 1e6 28.7 -> 39.1. Up to 5e4 nodes a field, in all degrees from 3 on
+//    and at N = 1 for BP3 (1e6 36.6 -> 32.2) and BP5 (17.7 -> 14.9) formed
+//    factors are faster.
+//  - N = 2, BP4: 1e6 nodes a field 52.5 -> 58.6 us, where the stored factors
+//    stay in the 256 MB Infinity Cache; 2e5 17.6 -> 16.7, 3e6 179 -> 164.
+bool bp_t::StoredPays() const {
+  const int N = mesh->N;
+  if (N == 1) return bp != 3 && bp != 5 && NLocal > (1 << 18);
+  const size_t factors = (size_t)mesh->Nelements * mesh->cubNp * 7 * sizeof(double);
+  return N == 2 && bp == 4 && NLocal > (1 << 20) && factors <= ((size_t)256 << 20);
 }
 
 template <typename T>
@@ -730,7 +747,7 @@ class BoxCgSteps : public CgSteps<T> {
     const int precision = 8 * (int)sizeof(T);
     this->rows = b.ogs.Ngather;
     fused = b.BoxFused(precision);
-    fold = fused && (b.cgFold & (precision == 64 ? 1 : 2));
+    fold = fused && (b.cgFold & (precision == 64 ? 1 : 2)) && b.FoldPays(sizeof(T));
   }
   int iterate(int k, double tol, bool pending) override {
     hipStream_t s = b.platform->stream;

@@ -350,3 +350,46 @@ def test_box_cub_cg(plat, bp, N, nx, ny, nz):
         out.append((hist, host(x)))
     np.testing.assert_array_equal(out[0][0], out[1][0])
     np.testing.assert_array_equal(out[0][1], out[1][1])
+
+
+# ------------------------------------------- the lowest degrees, large ----
+@pytest.mark.parametrize("bp,N,n", [(1, 1, 33), (2, 1, 23), (4, 1, 23), (6, 1, 23), (3, 1, 33), (4, 2, 24), (6, 2, 24),
+                                    (1, 2, 22)])
+def test_lowest_degrees_beyond_the_caches(plat, bp, N, n):
+    """Sizes just past the lines where stored factors are read (N = 1, BP4 at
+    N = 2, FP32 BP1) and where the direction update leaves the Ax: the operator
+    and q.Aq against the oracle, a solve to a tolerance with and without the
+    fold (the same bits) and, of the mixed solve, the true residual."""
+    kw = dict(N=N, nx=n, ny=n, nz=n + 1, perturb=0.1, seed=7)
+    m = capi.Mesh(cubature=bp <= 4, platform=plat, **kw)
+    P = oracle_lib.Problem(bp=bp, lam=1.0, **kw)
+    b = capi.BP(plat, m, bp, lam=1.0)
+    q = np.random.default_rng(N).standard_normal(b.Ngather)
+    qd = torch.from_numpy(q).cuda()
+    A, A2 = torch.full((2, b.Ngather), float("nan"), dtype=torch.float64, device="cuda")
+    b.operator(qd, A)
+    ref = P.operator(q)
+    assert rel_err(host(A), ref) <= 1e-12
+    qAq = b.operator_dot(qd, A2)
+    np.testing.assert_array_equal(host(A2), host(A))
+    assert abs(qAq - float(np.dot(q, host(A)))) <= 1e-13 * np.abs(q * host(A)).sum()
+    sols = []
+    for fold in (3, 0):
+        b.set_cg_fold(fold)
+        x = torch.zeros_like(qd)
+        its, hist = b.solve(x, qd.clone(), tol=1e-8, maxit=5000)
+        assert np.linalg.norm(q - P.operator(host(x))) <= 1.01e-8 * np.linalg.norm(q)
+        sols.append((its, hist, host(x)))
+    assert sols[0][0] == sols[1][0]
+    np.testing.assert_array_equal(sols[0][1], sols[1][1])
+    np.testing.assert_array_equal(sols[0][2], sols[1][2])
+    if bp in (1, 3):
+        A3 = torch.full((b.Ngather,), float("nan"), dtype=torch.float32, device="cuda")
+        b.operator_f32(qd.float(), A3)
+        assert rel_err(host(A3).astype(np.float64), ref) <= 2e-6
+        x = torch.zeros_like(qd)
+        # (interval 16: fewer iterations than the mass operator's FP32 recurrence
+        # takes to run out, beyond which a correction comes too late, with any
+        # of the kernels)
+        assert b.solve_mixed(x, qd, tol=1e-10, interval=16)["rel_res"] < 1e-10
+        assert np.linalg.norm(q - P.operator(host(x))) <= 1.01e-10 * np.linalg.norm(q)
