@@ -203,11 +203,7 @@ int bp5_workgroups(int N, int Nelements);
 template <typename T> int launch_bp1_ax(hipStream_t s, const AxArgs<T>& a);
 template <typename T> int launch_bp3_ax(hipStream_t s, const AxArgs<T>& a);
 
-// variable-coefficient BP5: kappa-scaled geometry (affine meshes expanded
-// to per-node factors) and the adjoint gradient per local node
-int launch_kappa_geometry(hipStream_t s, long long NLocal, int Nq, int affine, const int* lattice,
-                          const double* kappa, const double* ggeo, const double* wJ, const double* gllw,
-                          double* ggeoK, double* wJK);
+// variable-coefficient BP5: the adjoint gradient per local node
 int launch_bp5_kappa_grad(hipStream_t s, int N, int Nelements, int affine, const int* G2L, const double* ggeo,
                           const double* gllw, const double* D, const double* u, const double* lam, double* gL);
 

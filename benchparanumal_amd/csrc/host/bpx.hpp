@@ -589,14 +589,14 @@ class bp_t : public solver_t {
   std::shared_ptr<void> blas;
   deviceBuffer<double> o_AqL;
   deviceBuffer<double> o_AqLk;  // K local vectors for OperatorKrhs, grown on demand
-  // variable coefficient: lattice point of each local node, the lattice
-  // sum maps, kappa-scaled factors (per node) and, for affine meshes, wJ per node
+  // variable coefficient: lattice point of each local node, the lattice sum
+  // maps, the gradient per local node (the coefficient itself: o_kappa)
   bool haveKappa = false;
   deviceBuffer<dlong> o_lattice;
   ogs::ogs_t latticeOgs;
-  deviceBuffer<double> o_ggeoK, o_wJK, o_gradL;
+  deviceBuffer<double> o_gradL;
   // fused operator (solve space): the surface-node values of each element
-  // (FP64; FP32 in o_slots32), the shared rows' maps over them (rows
+  // (FP64), the shared rows' maps over them (rows
   // 0..Nshared-1 of the solve space), the first interior row, the Ax
   // kernel's p.Ap partials
   deviceBuffer<double> o_slots;

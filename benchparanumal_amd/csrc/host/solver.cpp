@@ -496,7 +496,7 @@ int bp_t::ax(const T* q, T* AqL, const T* wJ, const T* ggeo, const T* gllw, cons
   a.N = mesh->N;
   a.Nelements = mesh->Nelements;
   a.Nfields = Nfields;
-  a.affine = haveKappa ? 0 : mesh->opts.affine;  // kappa-scaled factors are per node
+  a.affine = mesh->opts.affine;
   a.elementList = o_elementList.ptr();
   a.GlobalToLocal = G2L ? G2L : o_GlobalToLocal.ptr();
   a.wJ = wJ;
@@ -511,7 +511,7 @@ int bp_t::ax(const T* q, T* AqL, const T* wJ, const T* ggeo, const T* gllw, cons
   a.Aq = AqL;
   if constexpr (std::is_same<T, double>::value) a.engine = axEngine;
   a.cubForm = cubForm;
-  if (bp <= 4 && !haveKappa) {
+  if (bp <= 4) {
     if constexpr (std::is_same<T, double>::value)
       a.eo = o_eo.length() ? o_eo.ptr() : nullptr;
     else
@@ -588,9 +588,7 @@ int bp_t::AxOperator(const dfloat* o_q, dfloat* o_AqL) {
 }
 
 int bp_t::AxStored(const dfloat* o_q, dfloat* o_AqL, const dlong* G2L) {
-  if (haveKappa)
-    return ax<double>(o_q, o_AqL, mesh->opts.affine ? o_wJK.ptr() : o_wJ.ptr(), o_ggeoK.ptr(), o_gllw.ptr(),
-                      o_D.ptr(), nullptr, nullptr, nullptr, G2L);
+  if (haveKappa) return set_error(BPX_ERR_UNSUPPORTED, "bp: the stored factors have no variable coefficient");
   return ax<double>(o_q, o_AqL, o_wJ.ptr(), o_ggeo.ptr(), o_gllw.ptr(), o_D.ptr(), o_I.ptr(), o_MM.ptr(),
                     o_invV.ptr(), G2L);
 }
@@ -619,23 +617,11 @@ int bp_t::SetKappa(const dfloat* o_kappa) {
     if (int st = o_lattice.upload(lat, s)) return st;
     if (int st = latticeOgs.SetupRows(NLocal, (dlong)Nnodes, lat.data())) return st;
     if (int st = latticeOgs.Upload(*platform)) return st;
-    if (boxAx) {
-      if (int st = this->o_kappa.alloc((size_t)Nnodes)) return st;
-    } else {
-      if (int st = o_ggeoK.alloc((size_t)NLocal * 6)) return st;
-      if (m.opts.affine)
-        if (int st = o_wJK.alloc(NLocal)) return st;
-    }
+    if (int st = this->o_kappa.alloc((size_t)Nnodes)) return st;
     if (int st = o_gradL.alloc(NLocal)) return st;
   }
-  if (boxAx) {  // the kernel scales by the lattice values themselves
-    BPX_HIP(hipMemcpyAsync(this->o_kappa.ptr(), o_kappa, (size_t)Nnodes * sizeof(double), hipMemcpyDeviceToDevice, s));
-    haveKappa = true;
-    return BPX_OK;
-  }
-  if (int st = launch_kappa_geometry(s, NLocal, m.Nq, m.opts.affine, o_lattice.ptr(), o_kappa, o_ggeo.ptr(),
-                                     o_wJ.ptr(), o_gllw.ptr(), o_ggeoK.ptr(), o_wJK.ptr()))
-    return st;
+  // the kernel scales by the lattice values themselves
+  BPX_HIP(hipMemcpyAsync(this->o_kappa.ptr(), o_kappa, (size_t)Nnodes * sizeof(double), hipMemcpyDeviceToDevice, s));
   haveKappa = true;
   return BPX_OK;
 }
@@ -810,14 +796,20 @@ std::unique_ptr<CgSteps<T>> bp_t::BoxSteps(T* p0, T* p1, T* x, T* r, T* AqL, con
 template std::unique_ptr<CgSteps<float>> bp_t::BoxSteps<float>(float*, float*, float*, float*, float*,
                                                                const CgWork<float>&);
 
-// Solves to a tolerance, with a variable coefficient or on affine elements
-// run on the box operator. A fixed number of iterations (tol = 0) on the
-// perturbed box keeps the reference's stored factors and the summation order
-// that its history is compared in: once CG has resolved the isolated top of
-// the spectrum, a difference of 1e-16 in the operator grows 1000-fold every
-// 30 iterations (24^3, p = 7, 100 iterations: residuals of two equally exact
-// operators 2e-12 to 1e-7 apart over 12 meshes), so a faster operator would
-// give another history, where a converged solution is the same.
+// Which operator a solve applies. To a tolerance: the box operator, as
+// Operator does. A fixed number of iterations (tol = 0) on perturbed elements:
+// the stored factors in the summation order that they have had, for the
+// residual history is what such a run is compared by, and another operator
+// gives another one, however exact. Distance of x and r from long double (BP5,
+// 24^3, p = 7, three meshes; stored / box operator):
+//   after 40 iterations x 2.5e-14 / 8e-16, r 2e-12 / 1e-14; after 100 x
+//   2e-14 / 9e-16, r 2e-12 and 8e-12 / 2e-13 and 3e-14 on two of them. On the
+//   third (isolated extreme eigenvalues: CG magnifies any difference some
+//   300-fold every 20 iterations) r 2e-10 / 2e-10 after 80 and 9e-8 / 8e-8 after 100.
+// So the box operator is the more exact one, but the two histories part by up
+// to 1e-7. On affine elements both read the same 6 factors and differ by
+// rounding (10^3, p = 4, 100 iterations: r 2.2e-13 and 4e-14 / 1.1e-13 and
+// 7e-14), and with a coefficient only the box operator exists.
 int bp_t::SolveCG(cg& solver, dfloat* o_x, dfloat* o_r, dfloat tol, int maxit, int verbose, int* iterations) {
   if (OnBox() && ogs.Ngather > 0 && (tol > 0 || haveKappa || mesh->opts.affine)) {
     if (solver.status()) return solver.status();
@@ -931,6 +923,7 @@ dlong bp_t::FoldRows() const {
 }
 
 int bp_t::OperatorDotFused(const double* o_q, double* o_Aq, double* part, int* npart, const CgFold<double>* fold) {
+  if (haveKappa) return set_error(BPX_ERR_UNSUPPORTED, "bp: the stored factors have no variable coefficient");
   hipStream_t s = platform->stream;
   AxArgs<double> a;
   if (fold) a.fold = *fold;
@@ -942,9 +935,9 @@ int bp_t::OperatorDotFused(const double* o_q, double* o_Aq, double* part, int* n
   a.lambda = lambda;
   a.q = o_q;
   a.ldq = fusedS0;  // the first interior row
-  a.affine = haveKappa ? 0 : mesh->opts.affine;
-  a.wJ = (haveKappa && mesh->opts.affine) ? o_wJK.ptr() : o_wJ.ptr();
-  a.ggeo = haveKappa ? o_ggeoK.ptr() : o_ggeo.ptr();
+  a.affine = mesh->opts.affine;
+  a.wJ = o_wJ.ptr();
+  a.ggeo = o_ggeo.ptr();
   a.gllw = o_gllw.ptr();
   a.D = o_D.ptr();
   a.engine = axEngine;
