@@ -320,7 +320,7 @@ constexpr int kBoxMaxRhs = 65535;
 
 // The same gather on a structured hex box, no maps (box_gather.hip): F
 // fields in [element][field][node] layout, K vectors of AqL ldL apart and of
-// out ldo apart. A vector of AqL must be smaller than 2^31 - 8 bytes.
+// out ldo apart. A vector of AqL holds at most kBoxRange bytes.
 template <typename T>
 int launch_box_gather(hipStream_t s, const BoxGrid& g, int F, int K, const T* AqL, long long ldL, T* out,
                       long long ldo);
@@ -342,8 +342,8 @@ struct BoxBatchItem {
 struct BatchState;
 
 // BP5 / BP6 Ax on a structured hex box (box_ax.hip): F fields, q on the
-// reference rows, AqL in [element][field][node] layout, both smaller than
-// 2^31 - 8 bytes.
+// reference rows, AqL in [element][field][node] layout, both of at most
+// kBoxRange bytes.
 enum { BOX_GEO_TRILINEAR = 0, BOX_GEO_AFFINE = 1, BOX_GEO_STORED = 2 };
 // the operator: BP5/BP6 on the GLL points (box_ax.hip), BP1/BP2 and BP3/BP4 on
 // the cubature points (box_cub.hip; trilinear maps, constant coefficient)

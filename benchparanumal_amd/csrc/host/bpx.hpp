@@ -499,7 +499,7 @@ class bp_t : public solver_t {
   int KappaGradient(const dfloat* o_u, const dfloat* o_lam, dfloat* o_grad);
   hlong LatticeNodes() const;
   // the hex box's rows in closed form (box.hpp): local values are gathered
-  // without maps while a local vector's byte offsets fit in 31 bits
+  // without maps while a local vector is no larger than kBoxRange bytes
   bool haveBox = false;
   BoxGrid box;
   // BP5 and BP6 on the box: the geometry formed in the kernel from the

@@ -393,3 +393,44 @@ def test_lowest_degrees_beyond_the_caches(plat, bp, N, n):
         # of the kernels)
         assert b.solve_mixed(x, qd, tol=1e-10, interval=16)["rel_res"] < 1e-10
         assert np.linalg.norm(q - P.operator(host(x))) <= 1.01e-10 * np.linalg.norm(q)
+
+
+# -------------------------------------------- vectors above 2 GB ----
+@pytest.mark.parametrize("bp", [2, 4, 6])
+def test_vectors_above_2_gb(plat, bp):
+    """Three fields of 90 million unknowns: the global vector 2.2 GB and the
+    local one 2.7 GB, past 31-bit byte offsets. Each field is the one-field
+    operator of the same mesh, whose vectors are below 1 GB, bit for bit; an
+    element's rows of a field follow those of the field before. Three CG
+    iterations with the same right-hand side in every field are the one-field
+    problem's (r.r and p.Ap three times as large)."""
+    n, N = 30, 15
+    m = capi.Mesh(N=N, nx=n, ny=n, nz=n, perturb=0.1, seed=3, cubature=bp <= 4, platform=plat)
+    one, three = capi.BP(plat, m, bp - 1, lam=1.1), capi.BP(plat, m, bp, lam=1.1)
+    assert three.NLocal * 8 > 1 << 31 and three.Ngather * 8 > 1 << 31 and one.NLocal * 8 < 1 << 30
+    e = torch.arange(n ** 3, device="cuda")
+    size = torch.ones_like(e)
+    for at in (e % n, e // n % n, e // n ** 2):
+        size *= torch.where(at == n - 1, N - 1, N)  # rows of an element
+    base = torch.cumsum(size, 0) - size
+    row = torch.arange(one.Ngather, device="cuda")
+    row += torch.repeat_interleave(2 * base, size)  # of field 0
+    size = torch.repeat_interleave(size, size)
+    q = torch.randn(one.Ngather, dtype=torch.float64, device="cuda", generator=torch.Generator("cuda").manual_seed(5))
+    scale = (1.0, -2.0, 0.25)  # powers of two: exact in every operation
+    q3 = torch.empty(three.Ngather, dtype=torch.float64, device="cuda")
+    for f in range(3):
+        q3[row + f * size] = scale[f] * q
+    A = torch.full_like(q, float("nan"))
+    A3 = torch.full_like(q3, float("nan"))
+    one.operator(q, A)
+    three.operator(q3, A3)
+    for f in range(3):
+        assert torch.equal(A3[row + f * size], scale[f] * A)
+        q3[row + f * size] = q
+    x, x3 = torch.zeros_like(q), torch.zeros_like(q3)
+    _, hist = one.solve(x, q.clone(), tol=1e-300, maxit=3)
+    _, hist3 = three.solve(x3, q3, tol=1e-300, maxit=3)
+    np.testing.assert_allclose(hist3, np.sqrt(3.0) * hist, rtol=1e-10)
+    for f in range(3):
+        assert float((x3[row + f * size] - x).norm()) <= 1e-10 * float(x.norm())
