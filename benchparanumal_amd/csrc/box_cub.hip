@@ -27,7 +27,7 @@
 //   i-lines (g,b):  A + D^T Gr, back along i, in place           -> A
 //   j-lines (g,i):  back along j, in place                       -> A
 //   k-lines (j,i):  back along k                                 -> Aq
-// 20 LDS accesses per point (mass: 8); odd line strides keep
+// 23 LDS accesses per point (mass: 8); odd line strides keep
 // all but the k, j and s lines free of bank conflicts.
 //
 // Measured at 24^3, p = 7: BP4 operator 319 -> 243 us, BP3 mixed solve 150 ->

@@ -1,4 +1,4 @@
-// Pieces that the structured-box operators (box_ax_body.hpp, box_cub_body.hpp)
+// Pieces that the structured-box operators (box_ax_body.hpp, box_cub.hip)
 // share: the rows of a lane's pencil, the start of a CG iteration, and the
 // factors of a trilinear element along a line of nodes.
 #pragma once

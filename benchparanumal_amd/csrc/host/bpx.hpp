@@ -641,8 +641,9 @@ class bp_solve_view_t : public solver_t {
   bp_t& bp;
 };
 
-// the box kernels' table of D (EvenOdd in box_ax.hip): one row of Nq values
-// per n <= (Nq-1)/2; an error if D is not antisymmetric to rounding
+// the box kernels' table of D (EvenOdd in box_ax_body.hpp): one row of Nq
+// values per n <= (Nq-1)/2, then D by rows; an error if D is not antisymmetric
+// to rounding
 int box_even_odd_table(const mesh_t& m, std::vector<double>& t);
 
 // Ragged batch of BP5 problems (box meshes of any size and degree), one CG

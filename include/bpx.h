@@ -408,7 +408,8 @@ int bpx_bp_set_cub_form(bpx_bp b, int form);
  * default): those CG solves do the direction update (x += alpha p, p = r +
  * beta p) inside the operator's Ax (with the stored factors: the elements'
  * interior rows; the separate update kernel then covers the shared rows
- * only); elsewhere (mask 0: everywhere) one update kernel covers all rows. */
+ * only); elsewhere (mask 0: everywhere; N <= 2: for vectors beyond the L2s)
+ * one update kernel covers all rows. */
 int bpx_bp_set_cg_fold(bpx_bp b, int mask);
 /* No reference counterpart (measurement): the CG operator as the solvers
  * apply it (their row order, the tuned fused or unfused form) in FP64
@@ -428,10 +429,12 @@ int bpx_bp_time_operator(bpx_bp b, int precision, int launches, double* out);
  * us. Synchronises. */
 int bpx_bp_time_krhs(bpx_bp b, int K, int chunk, int launches, const double* o_q, double* out);
 /* bpN_t::Operator(o_q, o_Aq) (BP/BP5/src/bp5Operator.cpp:29-85): Ax over the
- * local elements, then the T gather. Device vectors of length Ngather. BP5
- * (N <= 14) and BP6 on hexahedra form the geometric factors in the kernel
- * from the elements' trilinear maps (the stored factors' values to their
- * rounding, and closer to the exact ones). */
+ * local elements, then the T gather. Device vectors of length Ngather. On
+ * non-affine hexahedra the geometric factors are formed in the kernel from the
+ * elements' trilinear maps (the stored factors' values to their rounding, and
+ * closer to the exact ones), except where reading the stored ones is faster
+ * (large vectors at N = 1 and, BP4, 2) and where bpx_bp_set_cub_form asks for
+ * a kernel that does. */
 int bpx_bp_operator(bpx_bp b, const double* o_q, double* o_Aq);
 /* The operator as CG applies it: cg::Solve's Operator followed by
  * innerProd(p, Ap) (libs/core/linearSolverCG.cpp:99-106); o_Aq equals
@@ -486,10 +489,10 @@ int bpx_bp_rhs_forcing(bpx_bp b, double* o_b);
  * scalars: no host wait inside an iteration. o_r holds b on entry and the
  * residual on exit; o_x the initial guess / solution. rnorm_hist (host,
  * may be NULL) gets maxit+1 residual norms (entry 0 = initial). Returns
- * BPX_OK and *iterations. BP5 and BP6 on hexahedra: solves to a tolerance
- * apply the operator of bpx_bp_operator; a fixed number of iterations (tol =
- * 0, constant coefficient, not affine) applies the reference's stored
- * factors, whose residual history it reproduces. */
+ * BPX_OK and *iterations. On hexahedra, solves to a tolerance apply the
+ * operator of bpx_bp_operator; a fixed number of iterations (tol = 0, constant
+ * coefficient, not affine) applies the stored factors, whose residual history
+ * it reproduces. */
 int bpx_bp_solve(bpx_bp b, double* o_x, double* o_r, double tol, int maxit, int verbose,
                  int* iterations, double* rnorm_hist);
 /* No reference counterpart: CG in FP32 (FP32 operator and vectors, FP64
@@ -515,7 +518,8 @@ int bpx_bp_time_operator_in_solve(bpx_bp b, double* o_x, const double* o_b, doub
  * cg::Solve, libs/core/linearSolverCG.cpp:62-129) whose scalars stay on the
  * device; blocks of iterations are captured once in a hipGraph and
  * replayed until every problem has stopped. Problems of degrees up to 8
- * share two launches per iteration, those above two more. Vectors are the
+ * share two launches per iteration, those above two more. Both solves
+ * synchronise: x, iterations and residuals are complete on return. Vectors are the
  * problems' global vectors concatenated in order (bpx_batch_offsets). */
 int bpx_batch_create(bpx_platform p, int nprob, const bpx_mesh_opts* opts, double lambda,
                      bpx_batch* out);
