@@ -11,12 +11,12 @@ right-hand side at the 167^3 = 4,657,463 masked DOFs):
 value = Ndofs * N_it(FP64 CG to 1e-10) / T_step, the FP64-equivalent CG
 rate in GDOF*it/s; the plain FP64 CG (same tolerance) is timed beside it.
 The roofline object covers the dominant kernel of the timed solve, the Ax
-of the FP32 CG operator (the fused form when the setup's timing picked it),
-timed inside one more solve identical to the timed ones, with HIP events
-around each of its applications on the stream it is launched on (the same
-kernel launched back to back is reported beside it); its algorithmic bytes
-are the reference model (BK/BK5/src/bk5Run.cpp:116-122) with 4-byte values. The FP64 BK5 Ax (the reference's Ax benchmark) is
-reported beside it with the FP64 model. The CPU baseline is the
+of the FP32 CG iteration with the direction and x updates in front, timed
+inside one more solve identical to the timed ones, with HIP events stamped by
+each of its dispatches. The FP64 BK5 Ax (the reference's Ax benchmark) is
+reported beside it, with the bytes that it moves at least and with those of
+the reference's model (BK/BK5/src/bk5Run.cpp:116-122), whose kernel reads
+stored factors and maps. The CPU baseline is the
 oracle (C++/OpenMP restatement of the reference kernels) running a bounded
 number of FP64 CG iterations of the same problem on the host cores.
 """
@@ -52,11 +52,9 @@ def physical_cores():
         return os.cpu_count() or 1
 
 
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_bp5_ax_fp64_p7_24cube_hbm_traffic.txt")
-TRAFFIC_FILE_F32 = os.path.join(ROOT, "profiles", "k_bp5_ax_fp32_cg_operator_p7_24cube_hbm_traffic.txt")
-
-
-LIMITER_FILE_F32 = os.path.join(ROOT, "profiles", "k_bp5_ax_fp32_cg_operator_p7_24cube_sq_counters.txt")
+# counters of the two kernels that the timings below are of
+COUNTER_FILE = os.path.join(ROOT, "profiles", "k_box_ax_fp64_p7_24cube_counters.txt")
+COUNTER_FILE_F32 = os.path.join(ROOT, "profiles", "k_box_ax_fp32_fold_p7_24cube_counters.txt")
 
 
 def kernel_limiter(path):
@@ -79,7 +77,7 @@ def kernel_limiter(path):
     return out or None
 
 
-def measured_traffic(path=TRAFFIC_FILE):
+def measured_traffic(path=COUNTER_FILE):
     """HBM bytes per Ax launch from the committed counter summary (FETCH_SIZE and
     WRITE_SIZE scaled by a plain copy of known size), or None."""
     try:
@@ -91,18 +89,16 @@ def measured_traffic(path=TRAFFIC_FILE):
     return None
 
 
-def bk5_bytes(Ndofs, Nel, Np, value_bytes=8):
-    # BK/BK5/src/bk5Run.cpp:116-122 (non-affine hex, 4-byte dlong); value_bytes
-    # = 4 for the FP32 operator (values float, indices unchanged)
-    w = value_bytes
-    return Ndofs * w + Nel * (Np * 7 * w + 4 + Np * 4 + Np * w)
+def bk5_bytes(Ndofs, Nel, Np):
+    # BK/BK5/src/bk5Run.cpp:116-122 (non-affine hex, 4-byte dlong)
+    return Ndofs * 8 + Nel * (Np * 7 * 8 + 4 + Np * 4 + Np * 8)
 
 
-def bk5_tri_bytes(Ndofs, Nel, Np):
-    # the FP32 operator, which forms its geometric factors from each element's
-    # trilinear map: bk5_bytes with 4-byte values and the 7 factors per node
-    # replaced by the map's 24 coefficients per element
-    return Ndofs * 4 + Nel * (24 * 4 + 4 + Np * 4 + Np * 4)
+def box_bytes(Ndofs, Nel, Np, nfields=1, value_bytes=8, vectors=1):
+    """What an Ax on the structured box moves at least (no factors, no index
+    maps): `vectors` passes over the rows, the 24 coefficients of each
+    element's map, and the local values written."""
+    return value_bytes * (vectors * Ndofs + Nel * Np * nfields) + Nel * 24 * 8
 
 
 def bp5_ax_flops(Nq, Nel, affine=False, nfields=1):
@@ -127,9 +123,10 @@ def cg_solve_model(Ndofs, NLocal, ax_bytes, ax_flops, iterations):
     return nbytes, nflops
 
 
-def krhs_bytes(K, Ndofs, Nel, Np):
-    # k right-hand sides: vectors K times, geometry and GlobalToLocal once
-    return K * (Ndofs * 8 + Nel * Np * 8) + Nel * (Np * 7 * 8 + 4 + Np * 4)
+def krhs_bytes(K, Ndofs, Nel, Np, stored):
+    # k right-hand sides: vectors K times, the maps or (kernels on stored
+    # factors) the factors and GlobalToLocal once
+    return K * (Ndofs * 8 + Nel * Np * 8) + Nel * ((Np * 7 * 8 + 4 + Np * 4) if stored else 24 * 8)
 
 
 def event_time(fn, reps, warm=2):
@@ -151,7 +148,7 @@ def event_time(fn, reps, warm=2):
 
 def bench_krhs(capi, plat):
     """k-RHS BP5 Ax at 20^3, p=7 on the problem's arrays: each form (chunk 0 =
-    the default, the pencil form here; -1 the sheet workgroup form; 1, 2, 4
+    the default, the box kernel; on stored factors -1 the sheet workgroup form; 1, 2, 4
     the sweep form) against the single-vector Ax, both timed by HIP events
     their own dispatches stamp (kernel time, 10 launches after 2 warm-ups),
     on random right-hand sides."""
@@ -178,7 +175,7 @@ def bench_krhs(capi, plat):
         chunk = min(per_chunk, key=per_chunk.get)
         t = per_chunk[chunk] * 1e-6
         t1 = float(np.median(singles)) * 1e-6
-        nb = krhs_bytes(K, Ndofs, Nel, Np)
+        nb = krhs_bytes(K, Ndofs, Nel, Np, chunk != 0)
         rows.append({"K": K, "chunk": chunk, "us": t * 1e6, "gdof_per_s": K * Ndofs / t / 1e9,
                      "gbs": nb / t / 1e9, "algorithmic_bytes": nb, "speedup_vs_K_single": K * t1 / t,
                      "us_by_chunk": per_chunk})
@@ -288,9 +285,10 @@ def bench_p15(capi, plat):
 
 def bench_other_bps(capi, plat):
     """BP1, BP2, BP4 and BP6 Ax at 24^3, p = 7 (the perturbed box; three
-    fields for BP2/4/6), against each one's own byte model: BP1/BP2
-    BP/BP1/src/bp1Run.cpp:107-120 (cubature weights), BP4
-    BP/BP4/src/bp4Run.cpp:106-119 (cubature factors), BP6
+    fields for BP2/4/6), against what the box kernels move at least
+    (box_bytes), and the bytes of the reference's kernels, which read stored
+    factors and maps: BP1/BP2 BP/BP1/src/bp1Run.cpp:107-120 (cubature weights),
+    BP4 BP/BP4/src/bp4Run.cpp:106-119 (cubature factors), BP6
     BP/BP6/src/bp6Run.cpp:106-134 (node factors). Each is timed over 20
     launches after 200 untimed ones (8-48 ms): launches in the first ~20 ms
     after a problem's setup run up to 15% slower (BP4 268 against 235 us)."""
@@ -305,9 +303,10 @@ def bench_other_bps(capi, plat):
         AqL = torch.empty(bp.NLocal, dtype=torch.float64, device="cuda")
         t = event_time(lambda: bp.ax_local(q, AqL), 20, warm=200)
         geo = m.cubNp * 8 if bpn <= 2 else (m.cubNp if bpn == 4 else Np) * 7 * 8
-        nb = Nd * 8 + Nel * (geo + 4 + Np * nf * (4 + 8))
+        nb = box_bytes(Nd, Nel, Np, nf)
         rows.append({"bp": bpn, "fields": nf, "Ndofs": Nd, "us": t * 1e6, "gdof_per_s": Nd / t / 1e9,
-                     "algorithmic_bytes": nb, "gbs": nb / t / 1e9, "frac": nb / t / 1e9 / HBM_PEAK_GBS})
+                     "algorithmic_bytes": nb, "gbs": nb / t / 1e9, "frac": nb / t / 1e9 / HBM_PEAK_GBS,
+                     "reference_model_bytes": Nd * 8 + Nel * (geo + 4 + Np * nf * (4 + 8))})
         del bp, m, q, AqL
         torch.cuda.empty_cache()
     return {"workload": "BP1/BP2/BP4/BP6 Ax, 24^3 hex p=7 perturbed, FP64", "rows": rows}
@@ -358,7 +357,8 @@ def bench_bp3(capi, plat, args):
     q = torch.from_numpy(capi.random_normal(2, Nd)).cuda()
     AqL = torch.empty(bp.NLocal, dtype=torch.float64, device="cuda")
     t_ax = event_time(lambda: bp.ax_local(q, AqL), 20, warm=200)
-    nb = Nd * 8 + Nel * (cubNp * 7 * 8 + 4 + Np * 12)  # BP/BP3/src/bp3Run.cpp:114-118
+    nb = box_bytes(Nd, Nel, Np)
+    nref = Nd * 8 + Nel * (cubNp * 7 * 8 + 4 + Np * 12)  # BP/BP3/src/bp3Run.cpp:114-118
     b = torch.from_numpy(capi.random_normal(7, Nd)).cuda()
     x = torch.zeros_like(b)
     r = torch.empty_like(b)
@@ -386,7 +386,7 @@ def bench_bp3(capi, plat, args):
     tm = time.perf_counter() - t0
     return {"workload": f"BP3 hex p=7 24^3 perturbed, lambda=1, N(0,1) rhs, tol {args.tol:g}", "Ndofs": Nd,
             "ax_us": t_ax * 1e6, "ax_gbs": nb / t_ax / 1e9, "ax_algorithmic_bytes": nb,
-            "fp64_iterations": its, "fp64_ms": t64 * 1e3, "mixed_fp32_iterations": st["iterations"],
+            "ax_reference_model_bytes": nref, "fp64_iterations": its, "fp64_ms": t64 * 1e3, "mixed_fp32_iterations": st["iterations"],
             "mixed_corrections": st["updates"], "mixed_ms": tm * 1e3, "speedup_vs_fp64": t64 / tm,
             "fp64_equivalent_gdof_it_per_s": Nd * its / tm / 1e9}
 
@@ -507,30 +507,27 @@ def cpu_baselines(args, b_host, Ndofs):
 
 
 def roofline_object(ins, op32, nbytes32, achieved32, copy_gbs, Nel, args):
-    """The roofline of the dominant kernel of the timed solve, the FP32 CG
-    operator's Ax. Its bound is VALU issue (it forms the geometric factors
-    from the trilinear maps instead of streaming them): the committed SQ
-    counter summary gives its VALU instructions per launch, each wave64 FP32
-    instruction takes 4 cycles of one of the 1,024 SIMDs, and the launch's
-    own duration, timed in this run inside one more mixed solve, gives the
-    issue rate it reaches. The HBM figure (the reference byte model with
-    4-byte values and the map coefficients in place of the stored factors)
-    is reported beside it."""
+    """The roofline of the dominant kernel of the timed solve, the Ax of the
+    FP32 CG iteration with the direction and x updates in front. Its bound is
+    VALU issue (it forms the geometric factors): the committed counter summary
+    gives its VALU instructions per launch, each wave64 FP32 or FP64 instruction
+    takes 4 cycles of one of the 1,024 SIMDs, and the launch's own duration,
+    timed in this run inside one more mixed solve, gives the issue rate it
+    reaches. The HBM figure (box_bytes: r, p and x read, p and x written, the
+    maps, the local values) is reported beside it."""
     t = ins["ax_us"] * 1e-6
     hbm = {"achieved": achieved32, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved32 / HBM_PEAK_GBS,
-           "algorithmic_bytes": nbytes32, "traffic": measured_traffic(TRAFFIC_FILE_F32),
-           "traffic_source": "committed counter summary " + os.path.relpath(TRAFFIC_FILE_F32, ROOT) +
+           "algorithmic_bytes": nbytes32, "traffic": measured_traffic(COUNTER_FILE_F32),
+           "traffic_source": "committed counter summary " + os.path.relpath(COUNTER_FILE_F32, ROOT) +
                              " (rocprofv3 FETCH_SIZE + WRITE_SIZE, scaled by a 512 MiB copy); not measured in "
                              "this run"}
-    out = {"kernel": ("k_bp5_ax FP32 CG operator, " +
-                      ("fused (interior rows + surface run)" if ins["fused"] else "plain") +
-                      ", geometric factors from the trilinear map, non-affine, Nq=8"),
+    out = {"kernel": "k_box_ax<float, 8, trilinear factors, direction and x update folded in>",
            "us_per_launch": ins["ax_us"], "launches_timed": ins["launches"],
            "timed_in": "one more mixed solve identical to the timed ones (dispatch-stamped HIP events)",
-           "gather_us_per_launch": ins["gather_us"], "us_per_launch_back_to_back": op32["ax_us"],
+           "rest_of_iteration_us": ins["gather_us"], "us_without_updates_back_to_back": op32["ax_us"],
            "device_copy_gbs": copy_gbs,
            "model_gflops": bp5_ax_flops(args.N + 1, Nel) / t / 1e9}
-    lim = kernel_limiter(LIMITER_FILE_F32)
+    lim = kernel_limiter(COUNTER_FILE_F32)
     if lim and "valu_instructions_per_launch" in lim:
         instr = lim["valu_instructions_per_launch"]
         lanes_per_clk = 64 / lim["valu_cycles_per_instruction"]
@@ -548,6 +545,62 @@ def roofline_object(ins, op32, nbytes32, achieved32, copy_gbs, Nel, args):
     return out
 
 
+def box_kernels(capi, plat):
+    """A few launches of every structured-box kernel at the sizes that the
+    documents quote, after one device copy of 512 MiB (counter calibration)."""
+    import numpy as np
+    import torch
+
+    src = torch.ones(64 * 1024 * 1024, dtype=torch.float64, device="cuda")
+    dst = torch.empty_like(src)
+    dst.copy_(src)
+    del src, dst
+
+    def problem(bp, N, nx, ny=None, nz=None, affine=False):
+        m = capi.Mesh(N=N, nx=nx, ny=ny, nz=nz, affine=affine, cubature=bp <= 4, perturb=0.0 if affine else 0.1,
+                      seed=1, platform=plat)
+        b = capi.BP(plat, m, bp, lam=1.0)
+        v = torch.from_numpy(capi.random_normal(2, b.Ngather)).cuda()
+        return m, b, v
+
+    def iterations(b, v, its, tol=1e-300):
+        x = torch.zeros_like(v)
+        b.solve(x, v.clone(), tol=tol, maxit=its, history=False)
+
+    for bp, N, n in ((5, 7, (24,)), (5, 15, (24,)), (1, 6, (23, 21, 19)), (4, 7, (24,)), (6, 7, (24,))):
+        m, b, v = problem(bp, N, *n)
+        Av = torch.empty_like(v)
+        for _ in range(4):
+            b.operator(v, Av)
+        if bp == 5:  # the FP32 solve, the FP64 solve to a tolerance
+            for k in ((5, 3) if N == 7 else ()):
+                mk, bk, vk = (m, b, v) if k == 5 else problem(3, 7, 24)
+                bk.solve_mixed(torch.zeros_like(vk), vk, tol=1e-12, interval=24, maxit=24)
+            iterations(b, v, 8)
+        torch.cuda.synchronize()
+        del m, b, v, Av
+        torch.cuda.empty_cache()
+    m, b, v = problem(5, 4, 10, affine=True)
+    iterations(b, v, 24, tol=0.0)
+    m, b, v = problem(5, 7, 16)  # variable coefficient
+    b.set_kappa(torch.ones(b.Nnodes, dtype=torch.float64, device="cuda"))
+    iterations(b, v, 24)
+    m, b, _ = problem(5, 7, 20)
+    q = torch.from_numpy(capi.random_normal(4, b.Ngather * 16)).cuda()
+    for _ in range(3):
+        b.operator_krhs(q, torch.empty_like(q), 16)
+    rng = np.random.default_rng(2024)
+    probs = []
+    for i in range(64):
+        nx, ny, nz = (int(v) for v in rng.integers(2, 9, size=3))
+        probs.append({"N": int(rng.integers(3, 9)), "nx": nx, "ny": ny, "nz": nz, "perturb": 0.1, "seed": 100 + i})
+    B = capi.Batch(plat, probs, lam=1.0)
+    rhs = torch.from_numpy(capi.random_normal(77, B.Ntot)).cuda()
+    B.solve(torch.zeros_like(rhs), rhs, tol=1e-8, maxit=24)
+    torch.cuda.synchronize()
+    log("box kernels done")
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -557,9 +610,9 @@ def main():
     ap.add_argument("--nx", type=int, default=24)
     ap.add_argument("--tol", type=float, default=1e-10)
     # the solve stops at a correction, so it overshoots by about interval/2
-    # FP32 iterations (~108 us each at 24^3, p=7) against N/interval
-    # corrections (~215 us each): the sum is least near interval ~ 70 for
-    # N ~ 1270; measured 140.2/138.0/136.7/133.7/138.4 ms at 24/32/48/64/96
+    # FP32 iterations (~50 us each at 24^3, p=7), and a correction costs ~100:
+    # measured 72.7/71.5/70.7/69.0/71.5/67.5 ms at 24/32/48/64/96/128, the
+    # iteration count deciding between the longer ones (1280 at 64 and 128)
     ap.add_argument("--interval", type=int, default=64,
                     help="FP32 iterations between FP64 defect corrections")
     ap.add_argument("--ax-launches", type=int, default=50)
@@ -589,6 +642,9 @@ def main():
     ap.add_argument("--cub-only", action="store_true",
                     help="only 10 launches each of the FP64 BP1-BP4 Ax (default kernel form) on the 24^3 p=7 "
                          "perturbed box and one 512 MiB device copy (for counter runs)")
+    ap.add_argument("--box-kernels", action="store_true",
+                    help="only a few launches of every structured-box kernel and one 512 MiB device copy (for "
+                         "counter and trace runs)")
     args = ap.parse_args()
 
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
@@ -603,6 +659,9 @@ def main():
 
     torch.cuda.set_device(0)
     plat = capi.Platform(0)
+    if args.box_kernels:
+        box_kernels(capi, plat)
+        return
     if args.krhs_only:
         K = 32
         mk = capi.Mesh(N=7, nx=20, perturb=0.1, seed=1)
@@ -756,7 +815,7 @@ def main():
     relmix_s = float(torch.linalg.norm(b - Ax) / torch.linalg.norm(b))
     x.zero_()
     ins_s = bp.time_operator_in_solve(x, b, tol=args.tol, interval=args.interval)
-    stored32 = bk5_bytes(Ndofs, Nel, Np, 4)
+    stored32 = box_bytes(Ndofs, Nel, Np, value_bytes=4, vectors=5) + Nel * Np * 7 * 4
     mixed_stored = {"fp32_geometry": "stored factors rounded to FP32", "fp32_iterations": st_s["iterations"],
                     "fp64_corrections": st_s["updates"], "ms_per_solve": tmix_s * 1e3, "true_rel_res": relmix_s,
                     "fp64_equivalent_gdof_it_per_s": Ndofs * its64 / tmix_s / 1e9,
@@ -774,18 +833,17 @@ def main():
     log(f"reference protocol (FP64 CG, 100 its): {refp['elapsed_s'] * 1e3:.1f} ms, {refp['gbs']:.0f} GB/s, "
         f"{refp['gflops']:.0f} GFLOP/s, {refp['gdof_it_per_s']:.2f} GDOF*it/s")
 
-    # ---- roofline: the Ax of the FP32 CG operator, the dominant kernel of the
+    # ---- roofline: the Ax of the FP32 CG iteration, the dominant kernel of the
     # timed solve, timed inside one more solve identical to the timed ones
-    # (events around each application on the library's stream); back to
-    # back for comparison (its inputs then stay partly in the 256 MB
-    # Infinity Cache)
+    # (events stamped by its dispatches); the operator without the updates,
+    # back to back, for comparison
     x.zero_()
     ins = bp.time_operator_in_solve(x, b, tol=args.tol, interval=args.interval)
     op32 = bp.time_operator(32, args.ax_launches)
-    nbytes32 = bk5_tri_bytes(Ndofs, Nel, Np)
+    nbytes32 = box_bytes(Ndofs, Nel, Np, value_bytes=4, vectors=5)
     achieved32 = nbytes32 / (ins["ax_us"] * 1e-6) / 1e9
-    log(f"FP32 CG operator in the solve ({ins['launches']} applications): Ax {ins['ax_us']:.1f} us "
-        f"({achieved32:.0f} GB/s), gather {ins['gather_us']:.1f} us, fused {ins['fused']}; back to back: "
+    log(f"FP32 CG iteration in the solve ({ins['launches']} of them): Ax with updates {ins['ax_us']:.1f} us "
+        f"({achieved32:.0f} GB/s), rest {ins['gather_us']:.1f} us; the operator back to back: "
         f"Ax {op32['ax_us']:.1f} us, gather {op32['gather_us']:.1f} us")
 
     # ---- FP64 BK5 Ax (HIP events on the launch stream = torch's current stream)
@@ -801,8 +859,9 @@ def main():
     ev1.record()
     torch.cuda.synchronize()
     t_ax = ev0.elapsed_time(ev1) / 1e3 / args.ax_launches
-    nbytes = bk5_bytes(Ndofs, Nel, Np)
-    achieved = nbytes / t_ax / 1e9
+    nbytes = bk5_bytes(Ndofs, Nel, Np)  # of the reference's kernel; what the box kernel moves:
+    nbox = box_bytes(Ndofs, Nel, Np)
+    achieved = nbox / t_ax / 1e9
     log(f"BK5 Ax: {t_ax * 1e6:.1f} us, {achieved:.0f} GB/s, {Ndofs / t_ax / 1e9:.1f} GDOF/s")
 
     # plain device copy of 512 MiB on the same stream: the attainable HBM rate
@@ -879,8 +938,9 @@ def main():
                   "speedup_vs_fp64": t64 / tmix},
         "roofline": roofline_object(ins, op32, nbytes32, achieved32, copy_gbs, Nel, args),
         "bk5_fp64": {"achieved": achieved, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
-                     "traffic": measured_traffic(), "kernel": "k_bp5_ax (FP64, non-affine, Nq=8)",
-                     "us_per_launch": t_ax * 1e6, "algorithmic_bytes": nbytes,
+                     "traffic": measured_traffic(), "kernel": "k_box_ax<double, 8, trilinear factors>",
+                     "us_per_launch": t_ax * 1e6, "algorithmic_bytes": nbox,
+                     "reference_model_bytes": nbytes, "reference_model_gbs": nbytes / t_ax / 1e9,
                      "gdof_per_s": Ndofs / t_ax / 1e9,
                      "gflops": bp5_ax_flops(args.N + 1, Nel) / t_ax / 1e9},
         "tuning": bp.tuning(),
