@@ -10,8 +10,9 @@
 // 94 MB. The factors are the exact derivatives of the map; the stored ones
 // are derivatives by D, whose rounding the operator magnifies (relative
 // error against exact arithmetic at 24^3, p = 7: 8e-14 stored, 2e-15 here).
-// Measured there, FP64: Ax 97 -> 30 us, operator 127 -> 57 us; BP6 (three
-// fields, the geometry formed for each) 255 -> 172 us.
+// Measured there, FP64: Ax 97 -> 38 us, operator 127 -> 55 us; BP6 (three
+// fields, the geometry formed for each) 255 -> 166 us. Of the 38 us the vector
+// ALU issues for 21 and LDS for 9; 103 MB move.
 //
 // Layout (the pencil form of ax_bp5.hip): a lane owns the nodes (k, b, a),
 // k = 0..Nq-1, of its element; one-dimensional contractions run along a

@@ -14,7 +14,14 @@
 namespace bpx {
 namespace {
 
-constexpr int kLow = 9;  // the largest Nq of the first kernel
+// The largest Nq of the first kernel. A batch with degrees on both sides pays
+// for two launch pairs, one with only low degrees in the second kernel for
+// that one's registers. us per iteration with 6 / 7 / 9 / 12 (24 to 64 boxes):
+// degrees 3-8 47.1 / 46.5 / 34.7 / 35.8, 1-4 17.0 / 17.0 / 17.2 / 17.3, 5-12
+// 55.6 / 55.1 / 57.3 / 55.6, 6-9 31.3 / 41.4 / 42.1 / 28.0, 8-15 42.8 / 42.1 /
+// 52.0 / 52.2, 1-15 49.3 / 49.4 / 50.4 / 52.6 (one kernel for all degrees does
+// not compile): 9 keeps the common degrees, up to 8, in one.
+constexpr int kLow = 9;
 
 template <int LO, int HI, typename F>
 __device__ inline void dispatch(int nq, F&& f) {

@@ -30,10 +30,11 @@
 // 23 LDS accesses per point (mass: 8); odd line strides keep
 // all but the k, j and s lines free of bank conflicts.
 //
-// Measured at 24^3, p = 7: BP4 operator 319 -> 243 us, BP3 mixed solve 150 ->
-// 88 ms; BP1 on 23 x 21 x 19, p = 6, operator 41 -> 24 us. FP64 stiffness is
-// then bound by the vector ALU (76% busy; 1283 instructions per wavefront, 500
-// of them the factors) with LDS 62% busy beside it.
+// Measured at 24^3, p = 7: BP4 operator 319 -> 245 us, BP3 mixed solve 150 ->
+// 86 ms; BP1 on 23 x 21 x 19, p = 6, operator 41 -> 24 us. Of the 200 us of
+// BP4's Ax the vector ALU issues for 117 (1295 instructions per wavefront, 500
+// of them the factors) and LDS for 50, a third as much again lost to bank
+// conflicts; 323 MB move.
 #include "box_lanes.hpp"
 #include "even_odd.hpp"
 

@@ -1045,7 +1045,12 @@ int bp_t::TimeKrhs(int K, int chunk, int launches, const dfloat* o_q, double* ou
 // On the box the right-hand sides go through Ax and gather a few at a time,
 // as many as keep their local values below kKrhsBytes: those are then still
 // in the 256 MB Infinity Cache when the gather reads them, and the workspace
-// is no larger. Measured at 20^3, p = 7, K = 16: 485 us in one go, 444 with 136 MB, 461 with 104, 478 with 168.
+// is no larger. Measured with 64 / 100 / 136 / 200 MB / in one go, K = 32: 20^3,
+// p = 7 969 / 921 / 893 / 1013 / 963 us, 12^3 225 / 222 / 213 / 234 / 230, 28^3
+// 2567 / 2575 / 2575 / 2828 / 2723, 32^3, p = 3 525 / 509 / 481 / 523 / 536,
+// 40^3, p = 4 2074 / 2062 / 1923 / 2133 / 2086, 18^3, p = 5 336 / 317 / 314 /
+// 320 / 335, 12^3, p = 10 703 / 634 / 615 / 713 / 692, 12^3, p = 15 2254 /
+// 2256 / 2032 / 2274 / 2133.
 int bp_t::OperatorKrhs(int K, const dfloat* o_q, dfloat* o_Aq, int chunk) {
   if (K < 1) return set_error(BPX_ERR_INVALID_ARGUMENT, "bp: K < 1");
   constexpr size_t kKrhsBytes = (size_t)136 << 20;
