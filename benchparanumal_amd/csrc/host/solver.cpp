@@ -955,11 +955,28 @@ int bp_t::OperatorDotFused(const double* o_q, double* o_Aq, double* part, int* n
   return launch_fold(s, o_partAx.ptr(), naxParts, part);
 }
 
+// Several right-hand sides at the lowest degrees: the stored factors are read
+// once for all of them, the box kernel forms them for each, which is the
+// slower way past the caches. Operator on K vectors, stored -> formed us:
+//  - N = 1: 1e6 nodes, K = 16 153 -> 152; 1.4e6, K = 6 86 -> 85, K = 16 190 ->
+//    217; 2e6, K = 4 83 -> 82, K = 6 107 -> 119; 8e6, K = 32 1832 -> 3026;
+//    16e6, K = 3 557 -> 568, K = 4 659 -> 749.
+//  - N = 2: 8e6, K = 16 1147 -> 1113, K = 32 2220 -> 2222; 16e6, K = 8 1231 ->
+//    1222, K = 16 2295 -> 2416; 30e6, K = 32 8430 -> 9980.
+//  - N = 3: 8e6, K = 16 975 -> 953, K = 32 1815 -> 1903; 16e6, K = 16 1821 ->
+//    2018; 30e6, K = 32 7200 -> 8260. N = 4: 30e6, K = 32 8610 -> 8220.
+// Affine elements, and all degrees from 4 on, are faster formed.
+bool bp_t::KrhsStoredPays(int K) const {
+  const int N = mesh->N;
+  if (mesh->opts.affine || N > 3 || K < 4) return false;
+  return N == 1 ? NLocal > (5 << 18) && (double)K * NLocal > 10e6 : NLocal > (7 << 20) && (double)K * NLocal > 190e6;
+}
+
 int bp_t::AxLocalKrhs(int K, const dfloat* o_q, dfloat* o_AqL, int chunk) {
   if (bp != 5 || mesh->elementType != ELEM_HEX)
     return set_error(BPX_ERR_UNSUPPORTED, "bp: k right-hand sides are implemented for BP5 on hexahedra");
   if (haveKappa) return set_error(BPX_ERR_UNSUPPORTED, "bp: k right-hand sides use the constant coefficient");
-  if (chunk == 0 && boxAx) {
+  if (chunk == 0 && boxAx && !KrhsStoredPays(K)) {
     if (K < 1) return set_error(BPX_ERR_INVALID_ARGUMENT, "bp: K < 1");
     for (int k = 0; k < K; k += kBoxMaxRhs) {
       BoxAxArgs<double> b = BoxArgs<double>(o_q + (size_t)k * ogs.Ngather, o_AqL + (size_t)k * NLocal);
@@ -1058,7 +1075,8 @@ int bp_t::OperatorKrhs(int K, const dfloat* o_q, dfloat* o_Aq, int chunk) {
   // gather, which would overwrite what a later run reads)
   const size_t n = (size_t)K * ogs.Ngather;
   const bool apart = o_q == o_Aq || o_q + n <= o_Aq || o_Aq + n <= o_q;
-  const bool some = chunk == 0 && boxAx && bp == 5 && !haveKappa && ogs.Ngather > 0 && apart;
+  const bool some =
+      chunk == 0 && boxAx && bp == 5 && !haveKappa && ogs.Ngather > 0 && apart && !KrhsStoredPays(K);
   const int kc = some ? (int)std::min<size_t>(K, std::max<size_t>(1, kKrhsBytes / ((size_t)NLocal * sizeof(double)))) : K;
   const size_t need = (size_t)NLocal * kc;
   if (o_AqLk.length() < need) {

@@ -395,6 +395,29 @@ def test_lowest_degrees_beyond_the_caches(plat, bp, N, n):
         assert np.linalg.norm(q - P.operator(host(x))) <= 1.01e-10 * np.linalg.norm(q)
 
 
+@pytest.mark.parametrize("N,n,K", [(1, 54, 8), (1, 55, 7), (1, 55, 8), (3, 49, 25), (3, 50, 24)])
+def test_krhs_lowest_degrees(plat, N, n, K):
+    """Several right-hand sides on both sides of the line from which the stored
+    factors are read, in place as well: each vector as the operator gives it
+    alone (to the 1e-12 of the other comparisons of the two kinds of
+    factors), and symmetric, u.Av = v.Au."""
+    b = capi.BP(plat, capi.Mesh(N=N, nx=n, ny=n, nz=n, perturb=0.1, seed=7, platform=plat), 5, lam=1.0)
+    gen = torch.Generator(device="cuda").manual_seed(N * n)
+    q = torch.randn((K, b.Ngather), generator=gen, device="cuda", dtype=torch.float64)
+    A = torch.full_like(q, float("nan"))
+    b.operator_krhs(q, A, K)
+    one = torch.full_like(q[0], float("nan"))
+    for k in range(K):
+        b.operator(q[k], one)
+        assert float((A[k] - one).norm() / one.norm()) <= 1e-12
+    u, v = q[0], q[K - 1]
+    scale = float((u * A[K - 1]).abs().sum() + (v * A[0]).abs().sum())
+    assert abs(float((u * A[K - 1]).sum() - (v * A[0]).sum())) <= 1e-12 * scale
+    p = q.clone()
+    b.operator_krhs(p, p, K)
+    assert torch.equal(p, A)
+
+
 # -------------------------------------------- vectors above 2 GB ----
 @pytest.mark.parametrize("bp", [2, 4, 6])
 def test_vectors_above_2_gb(plat, bp):
