@@ -512,7 +512,6 @@ class bp_t : public solver_t {
   bool boxCub = false;
   bool StoredPays() const;  // where the stored factors are the faster ones
   bool KrhsStoredPays(int K) const;
-  bool CgStoredPays() const;
   bool OnBox() const { return boxAx || (boxCub && cubForm == CUB_FORM_AUTO); }
   int BoxOp() const { return bp >= 5 ? BOX_OP_GLL : bp >= 3 ? BOX_OP_STIFF : BOX_OP_MASS; }
   int BoxPartials() const { return box_ax_partials(box, Nfields, BoxOp()); }

@@ -810,18 +810,8 @@ template std::unique_ptr<CgSteps<float>> bp_t::BoxSteps<float>(float*, float*, f
 // to 1e-7. On affine elements both read the same 6 factors and differ by
 // rounding (10^3, p = 4, 100 iterations: r 2.2e-13 and 4e-14 / 1.1e-13 and
 // 7e-14), and with a coefficient only the box operator exists.
-// At N = 2 the vector operators' iterations past the caches are faster on the
-// stored factors (per iteration, stored -> box: BP4, 6e6 nodes a field 469 ->
-// 454 us, 8e6 610 -> 623, 24e6 1836 -> 1955, 35e6 2617 -> 2940; BP6, 8e6 430 ->
-// 428, 12e6 649 -> 645, 20e6 1025 -> 1115, 24e6 1301 -> 1341, 30e6 1633 -> 1620,
-// 35e6 1848 -> 2040; BP2 and N = 3 2 to 25% faster on the box).
-bool bp_t::CgStoredPays() const {
-  const dlong nodes = NLocal / Nfields;
-  return mesh->N == 2 && ((bp == 4 && nodes > (7 << 20)) || (bp == 6 && nodes > (1 << 24)));
-}
-
 int bp_t::SolveCG(cg& solver, dfloat* o_x, dfloat* o_r, dfloat tol, int maxit, int verbose, int* iterations) {
-  if (OnBox() && ogs.Ngather > 0 && (haveKappa || mesh->opts.affine || (tol > 0 && !CgStoredPays()))) {
+  if (OnBox() && ogs.Ngather > 0 && (tol > 0 || haveKappa || mesh->opts.affine)) {
     if (solver.status()) return solver.status();
     if (maxit < 0) return set_error(BPX_ERR_INVALID_ARGUMENT, "cg: MAXIT < 0");
     cg_t<double>& c = solver.impl;
