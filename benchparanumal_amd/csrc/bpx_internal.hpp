@@ -449,6 +449,15 @@ int launch_copy_f64_to_f32(hipStream_t s, dlong N, double scale, const double* x
 template <typename T>
 int launch_dot_partials(hipStream_t s, dlong N, const T* x, const T* y, double* part);
 int launch_fold(hipStream_t s, const double* part, int n, double* out);
+// n partials into kRedBlocks of them (out: apart from part). Every workgroup
+// of an update kernel folds all the partials that it is given (some thousand
+// workgroups, n / 256 loads one after another), which beyond kPartsFolded
+// costs more than this launch. Per CG iteration, without / with it: 1563
+// partials 22.5 / 24.8 us, 2980 35.6 / 35.7, 3485 45.9 / 44.8, 3907 (BP5, p = 7,
+// 8e6 nodes) 100.1 / 98.7, 5832 43.2 / 39.8, 15625 (FP32 BP5, N = 1, 8e6) 93.1 /
+// 78.3, 94332 (BP4, N = 3, 2e7 nodes a field) 1409 / 1274.
+constexpr int kPartsFolded = 3584;
+int launch_fold_parts(hipStream_t s, const double* part, int n, double* out);
 // x.y into *out (device); part holds kRedBlocks doubles
 template <typename T>
 int launch_dot(hipStream_t s, dlong N, const T* x, const T* y, double* part, double* out);

@@ -380,7 +380,7 @@ class bp_t : public solver_t {
   int OperatorDot(const dfloat* o_q, dfloat* o_Aq, double* part, int* npart) override;
   int GatherPartials() const {
     return std::max({ogs_gather_partials(ogs.NrowBlocksT), ogs_gather_partials(sharedOgs.NrowBlocksT),
-                     ogs_gather_partials(solveOgs.NrowBlocksT), haveBox ? BoxPartials() : 1, 1});
+                     ogs_gather_partials(solveOgs.NrowBlocksT), haveBox ? BoxPartials() + kRedBlocks : 1});
   }
 
   // Solve space: the row order the CG solvers run in. For BP5 with one

@@ -742,7 +742,8 @@ class BoxCgSteps : public CgSteps<T> {
       if (int st = launch_cg_update_p<T>(s, N, k, r, p[0], x, w.part_rr, this->nrr, w.state, w.hist_rr, w.hist_alpha,
                                          tol, pending))
         return st;
-    const int npAp = b.BoxPartials();
+    int npAp = b.BoxPartials();
+    double* pAp = w.part_pAp;
     auto apply = [&]() -> int {
       BoxAxArgs<T> a = b.BoxArgs<T>(fold ? p[(k + 1) & 1] : p[0], AqL);
       a.part = w.part_pAp;
@@ -761,13 +762,18 @@ class BoxCgSteps : public CgSteps<T> {
         a.tol = tol;
       }
       if (int st = launch_box_ax<T>(s, a)) return st;
+      if (npAp > kPartsFolded) {  // the buffers hold kRedBlocks more (GatherPartials)
+        pAp += npAp;
+        if (int st = launch_fold_parts(s, w.part_pAp, npAp, pAp)) return st;
+        npAp = kRedBlocks;
+      }
       if (!fused) return b.GatherLocal<T>(AqL, p[1]);
       BoxUpdateR<T> u;
       u.AqL = AqL;
       u.r = r;
       u.k = k;
       u.npAp = npAp;
-      u.part_pAp = w.part_pAp;
+      u.part_pAp = pAp;
       u.part_rr = w.part_rr;
       u.st = w.state;
       u.hist_rr = w.hist_rr;
@@ -777,7 +783,7 @@ class BoxCgSteps : public CgSteps<T> {
     if (int st = sizeof(T) == 4 ? b.TimedStep32(apply) : apply()) return st;
     if (fused) return BPX_OK;
     this->nrr = kRedBlocks;
-    return launch_cg_update_r<T>(s, N, k, p[1], r, w.part_pAp, npAp, w.part_rr, w.state, w.hist_rr, w.hist_alpha);
+    return launch_cg_update_r<T>(s, N, k, p[1], r, pAp, npAp, w.part_rr, w.state, w.hist_rr, w.hist_alpha);
   }
   const T* direction(int k) const override { return fold ? p[k & 1] : p[0]; }
 

@@ -147,6 +147,17 @@ __global__ __launch_bounds__(RT) void k_fold(const double* __restrict__ part, in
   if (threadIdx.x == 0) *out = t;
 }
 
+// many partials to gridDim.x of them
+__global__ __launch_bounds__(256) void k_fold_parts(const double* __restrict__ part, int n, double* __restrict__ out) {
+  __shared__ double s_w[33];
+  const int per = (n + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int base = min((int)blockIdx.x * per, n), end = min(base + per, n);
+  double a = 0;
+  for (int i = base + (int)threadIdx.x; i < end; i += 256) a += part[i];
+  const double t = block_allsum(a, s_w);
+  if (threadIdx.x == 0) out[blockIdx.x] = t;
+}
+
 // r <- r - Ap (residual of the initial guess) with r.r partials
 template <typename T>
 __global__ __launch_bounds__(RT) void k_cg_init(dlong N, const T* __restrict__ Ap, T* __restrict__ r,
@@ -474,6 +485,12 @@ int launch_dot_partials(hipStream_t s, dlong N, const T* x, const T* y, double* 
 
 int launch_fold(hipStream_t s, const double* part, int n, double* out) {
   hipLaunchKernelGGL(k_fold, dim3(1), dim3(RT), 0, s, part, n, out);
+  BPX_HIP(hipGetLastError());
+  return BPX_OK;
+}
+
+int launch_fold_parts(hipStream_t s, const double* part, int n, double* out) {
+  hipLaunchKernelGGL(k_fold_parts, dim3(RB), dim3(256), 0, s, part, n, out);
   BPX_HIP(hipGetLastError());
   return BPX_OK;
 }

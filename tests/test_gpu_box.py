@@ -418,6 +418,39 @@ def test_krhs_lowest_degrees(plat, N, n, K):
     assert torch.equal(p, A)
 
 
+@pytest.mark.parametrize("bp,N,n", [(5, 1, 61), (5, 1, 62), (4, 2, 26), (4, 2, 27), (1, 3, 35)])
+def test_many_partials(plat, bp, N, n):
+    """On both sides of the number of p.Ap partials from which a kernel of its
+    own folds them: the residual that CG carries is b - A x, with and without
+    the direction update in the Ax (the same bits) and the update kernel
+    fused; and the mixed solve meets its tolerance."""
+    b = capi.BP(plat, capi.Mesh(N=N, nx=n, ny=n, nz=n, perturb=0.1, seed=7, cubature=bp <= 4, platform=plat), bp,
+                lam=1.0)
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    rhs = torch.randn(b.Ngather, generator=gen, device="cuda", dtype=torch.float64)
+    Ax = torch.full_like(rhs, float("nan"))
+    sols = []
+    for fold, fused in ((3, -1), (0, -1), (0, 0)):
+        b.set_cg_fold(fold)
+        b.set_tuning(fused=fused)
+        x, r = torch.zeros_like(rhs), rhs.clone()
+        its, hist = b.solve(x, r, tol=1e-300, maxit=20)
+        assert its == 20 and abs(float(hist[0]) - float(rhs.norm())) <= 1e-12 * float(hist[0])
+        b.operator(x, Ax)
+        # rounding of 20 updates: some 1e-15 of |A| |x|, below 1e3 |b| here
+        assert float((rhs - Ax - r).norm()) <= 1e-11 * float(rhs.norm())
+        sols.append((hist, host(x)))
+    np.testing.assert_array_equal(sols[0][0], sols[1][0])
+    np.testing.assert_array_equal(sols[0][1], sols[1][1])
+    np.testing.assert_allclose(sols[2][0], sols[0][0], rtol=1e-9)
+    if bp != 4:
+        # (interval 16: see test_lowest_degrees_beyond_the_caches)
+        x = torch.zeros_like(rhs)
+        assert b.solve_mixed(x, rhs, tol=1e-10, interval=16)["rel_res"] < 1e-10
+        b.operator(x, Ax)
+        assert float((rhs - Ax).norm()) <= 1.01e-10 * float(rhs.norm())
+
+
 # -------------------------------------------- vectors above 2 GB ----
 @pytest.mark.parametrize("bp", [2, 4, 6])
 def test_vectors_above_2_gb(plat, bp):
